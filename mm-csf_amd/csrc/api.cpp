@@ -772,6 +772,7 @@ int mmcsf_format_build(const mmcsf_tensor *th, int type, const mmcsf_options *op
                           "warpPerFbr (-w) or fbrPerWarp (-s) cannot be higher than threadblock size!\n"
                           "hint: increase -b!");
         hipStream_t s = static_cast<hipStream_t>(stream);
+        BuildPool pool;  // before every array of the build, which may hold its blocks
         auto fh = std::make_unique<mmcsf_format>();
         Format &f = fh->f;
         f.type = type;
@@ -845,7 +846,7 @@ int mmcsf_format_build(const mmcsf_tensor *th, int type, const mmcsf_options *op
             order_tensormode(t.ndims, t.dims, (int)opt->mode, nat, order);
             if (type == MMCSF_TYPE_COO || type == MMCSF_TYPE_COO_CPU) {
                 for (int l = 0; l < t.ndims; ++l) f.cooOrder[l] = order[l];
-                sort_coo(t, order, f.cooKeys, f.cooVals, s);
+                sort_coo(t, order, f.cooKeys, f.cooVals, s, nullptr, true);
             } else {
                 const bool bcsf = type != MMCSF_TYPE_HBCSF;  // types 8, 9, 13, 14
                 DevArray<uint32_t> pos;

