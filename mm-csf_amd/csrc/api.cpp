@@ -815,8 +815,7 @@ int mmcsf_format_build(const mmcsf_tensor *th, int type, const mmcsf_options *op
                     c.pos = std::move(p2);
                 };
                 uint64_t hot[kMaxDims] = {0, 0, 0, 0};
-                if (t.ndims == 3)
-                    for (int m = 0; m < t.ndims; ++m) hot[m] = hot_footprint(t, m, 0.9, s);
+                if (t.ndims == 3) hot_footprints(t, 0.9, hot, s);
                 for (int m = 0; m < t.ndims; ++m) {
                     if (m == order[0]) continue;
                     int o2[kMaxDims];

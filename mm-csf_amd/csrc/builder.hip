@@ -1000,25 +1000,89 @@ void build_hot_table(const Csf &c, int level, uint64_t rows, HotTable &h, hipStr
     MMCSF_HIP(hipStreamSynchronize(s));
 }
 
-// Rows of tensor mode m that hold `frac` of the nonzeros, the most used rows
-// first: the working set of gathers from that mode's factor table (small for
-// skewed modes, most of the rows for uniform ones).
-uint64_t hot_footprint(const Tensor &t, int m, double frac, hipStream_t s) {
-    const uint64_t rows = t.dims[m], n = t.nnz;
-    if (n == 0 || rows == 0) return 0;
-    TmpArray<uint32_t> cnt(rows);
-    MMCSF_HIP(hipMemsetAsync(cnt.p, 0, rows * 4, s));
-    hipLaunchKernelGGL(k_hist, dim3(nblk(n)), dim3(kBS), 0, s, t.inds[m].p, n, cnt.p);
-    MMCSF_HIP(hipGetLastError());
-    std::vector<uint32_t> h(rows);
-    MMCSF_HIP(hipMemcpyAsync(h.data(), cnt.p, rows * 4, hipMemcpyDeviceToHost, s));
+namespace {
+
+// Row counts of one mode.  What bounds a plain histogram is the hot rows: on a
+// Zipf(1.2) mode the top row takes ~18 % of the increments, and global atomics
+// on one address run one after another (20M nonzeros: 37 ms).  Every block
+// therefore counts in an LDS table of kHistSlots (row, count) pairs, hashed by
+// row and claimed first come, first served (a hot row comes within the first
+// elements), and adds each pair to the global counts once; rows that find
+// their slot taken are cold and go to the global counts directly.
+// 20M nonzeros in 500000 rows, Zipf(1.2): 37.5 ms with plain atomics, 0.34 here.
+constexpr int kHistThreads = 1024;
+constexpr uint32_t kHistBits = 13, kHistSlots = 1u << kHistBits;
+constexpr uint32_t kNoRow = 0xffffffffu;  // coordinates are below 2^31
+__global__ __launch_bounds__(kHistThreads) void k_hist_cached(const uint32_t *__restrict__ idx, uint64_t n,
+                                                              uint32_t *__restrict__ cnt) {
+    __shared__ uint32_t row[kHistSlots], num[kHistSlots];
+    for (uint32_t i = threadIdx.x; i < kHistSlots; i += kHistThreads) {
+        row[i] = kNoRow;
+        num[i] = 0;
+    }
+    __syncthreads();
+    for (uint64_t i = blockIdx.x * (uint64_t)kHistThreads + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kHistThreads) {
+        const uint32_t v = idx[i];
+        const uint32_t slot = (v * 2654435761u) >> (32 - kHistBits);
+        uint32_t owner = row[slot];
+        if (owner == kNoRow) {
+            owner = atomicCAS(&row[slot], kNoRow, v);
+            if (owner == kNoRow) owner = v;
+        }
+        if (owner == v) atomicAdd(&num[slot], 1u);
+        else atomicAdd(&cnt[v], 1u);
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < kHistSlots; i += kHistThreads)
+        if (num[i]) atomicAdd(&cnt[row[i]], num[i]);
+}
+
+// out = the number of leading entries (counts in descending order, prefix =
+// their inclusive sums) it takes to reach `want`
+__global__ void k_reach(const uint64_t *__restrict__ prefix, uint64_t rows, double want, uint32_t *out) {
+    const uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+    if (i >= rows) return;
+    const double before = i ? (double)prefix[i - 1] : 0.0;
+    if (before < want && (i + 1 == rows || (double)prefix[i] >= want)) *out = (uint32_t)(i + 1);
+}
+
+}  // namespace
+
+// Per mode m, the rows that hold `frac` of the nonzeros, most used rows first:
+// the working set of gathers from that mode's factor table (small for skewed
+// modes, most of the rows for uniform ones).  Counted, ordered and summed on
+// the GPU; the host reads the results of all modes at once.
+void hot_footprints(const Tensor &t, double frac, uint64_t *hot, hipStream_t s) {
+    const uint64_t n = t.nnz;
+    for (int m = 0; m < t.ndims; ++m) hot[m] = 0;
+    if (n == 0) return;
+    uint64_t most = 0;
+    for (int m = 0; m < t.ndims; ++m) most = std::max(most, t.dims[m]);
+    Temp tmp;
+    TmpArray<uint32_t> cnt(most), sorted(most), found(kMaxDims);
+    TmpArray<uint64_t> prefix(most);
+    hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(kBS), 0, s, found.p, (uint64_t)kMaxDims);
+    const unsigned blocks = (unsigned)std::min<uint64_t>(2ull * device_cu_count(), (n + kHistThreads - 1) / kHistThreads);
+    for (int m = 0; m < t.ndims; ++m) {
+        const uint64_t rows = t.dims[m];
+        if (rows == 0) continue;
+        hipLaunchKernelGGL(k_zero_words, dim3(nblk(rows)), dim3(kBS), 0, s, cnt.p, rows);
+        hipLaunchKernelGGL(k_hist_cached, dim3(blocks), dim3(kHistThreads), 0, s, t.inds[m].p, n, cnt.p);
+        MMCSF_HIP(hipGetLastError());
+        const unsigned bits = (unsigned)bitwidth(n);
+        size_t bytes = 0;
+        MMCSF_HIP(rocprim::radix_sort_keys_desc(nullptr, bytes, cnt.p, sorted.p, (size_t)rows, 0u, bits, s));
+        MMCSF_HIP(rocprim::radix_sort_keys_desc(tmp.get(bytes), bytes, cnt.p, sorted.p, (size_t)rows, 0u, bits, s));
+        MMCSF_HIP(rocprim::inclusive_scan(nullptr, bytes, sorted.p, prefix.p, (size_t)rows, rocprim::plus<uint64_t>(), s));
+        MMCSF_HIP(rocprim::inclusive_scan(tmp.get(bytes), bytes, sorted.p, prefix.p, (size_t)rows,
+                                          rocprim::plus<uint64_t>(), s));
+        hipLaunchKernelGGL(k_reach, dim3(nblk(rows)), dim3(kBS), 0, s, prefix.p, rows, frac * (double)n, found.p + m);
+        MMCSF_HIP(hipGetLastError());
+    }
+    uint32_t h[kMaxDims];
+    MMCSF_HIP(hipMemcpyAsync(h, found.p, sizeof(h), hipMemcpyDeviceToHost, s));
     MMCSF_HIP(hipStreamSynchronize(s));
-    std::sort(h.begin(), h.end(), [](uint32_t a, uint32_t b) { return a > b; });
-    const double want = frac * (double)n;
-    double acc = 0;
-    uint64_t k = 0;
-    while (k < rows && acc < want) acc += h[k++];
-    return k;
+    for (int m = 0; m < t.ndims; ++m) hot[m] = h[m];
 }
 
 

@@ -300,8 +300,8 @@ void build_hyb(int ndims, const uint64_t *dims, Csf &&src, Hyb &out, hipStream_t
 // the CSL part of a built 3-D HB-CSF as a walkable tree (h.cslWalk)
 void build_csl_walk(Hyb &h, hipStream_t s);
 void build_hot_table(const Csf &c, int level, uint64_t rows, HotTable &h, hipStream_t s);
-// rows of tensor mode m holding `frac` of the nonzeros, most used first
-uint64_t hot_footprint(const Tensor &t, int m, double frac, hipStream_t s);
+// hot[m] = the rows of tensor mode m holding `frac` of the nonzeros, most used first
+void hot_footprints(const Tensor &t, double frac, uint64_t *hot, hipStream_t s);
 // mixed-mode partition: level-1 entry of every nonzero of an unsplit CSF (at
 // its tensor position, resolved like the reference's search over
 // denseSlcPtr; 0xFFFFFFFF where that search reads before the first entry)
