@@ -51,3 +51,60 @@ def test_mode_tree_orders_follow_the_footprints(cuda, dims, skew, nnz):
             na, nb = sum(na), sum(nb)
             want = [m, b, a] if nb < na else [m, a, b]
         assert info["modeTreeOrder"][m] == want, (m, hot)
+
+
+# ---- builder: sorted keys unpacked, values carried, start bits by windows ---------
+
+def rel(a, b):
+    b = np.asarray(b, dtype=np.float64)
+    n = np.linalg.norm(b)
+    return float(np.linalg.norm(np.asarray(a, np.float64) - b) / (n if n > 0 else 1.0))
+
+
+def fibers_tensor(rng, fibers, per_fiber, leaf_dim):
+    """`fibers` leaf fibers of `per_fiber` nonzeros each, in random order."""
+    f = np.repeat(np.arange(fibers, dtype=np.int64), per_fiber)
+    leaf = np.concatenate([np.sort(rng.choice(leaf_dim, per_fiber, replace=False)) for _ in range(fibers)])
+    p = rng.permutation(len(f))
+    inds = [(f // 50)[p], (f % 50)[p], leaf[p].astype(np.int64)]
+    dims = [int(inds[0].max()) + 1, 50, leaf_dim]
+    return dims, inds, (rng.random(len(f)) + 0.25).astype(np.float32)
+
+
+@pytest.mark.parametrize("fibers,per_fiber", [(1, 1), (2047, 1), (2048, 3), (2049, 2), (2048, 32), (2049, 33), (4100, 40)])
+def test_fiber_start_bits(cuda, fibers, per_fiber):
+    """A block of the start-bit kernel marks 2048 fibers in a window of 65536
+    nonzeros: one fiber below, at and above the block, at and past the window."""
+    import torch
+    import mmcsf
+    import oracle as O
+    from test_gpu_builder import check_format
+    rng = np.random.default_rng(fibers)
+    dims, inds, vals = fibers_tensor(rng, fibers, per_fiber, 64)
+    t = mmcsf.Tensor.from_numpy(dims, inds, vals)
+    U = [rng.random((d, 8)).astype(np.float32) for d in dims]
+    Ud = [torch.from_numpy(u).to(cuda) for u in U]
+    for fmt_type in (8, 10):
+        fmt, _ = check_format(mmcsf, t, fmt_type, dims, inds, vals, 0, 1 << 30)
+        assert rel(mmcsf.mttkrp(fmt, 0, Ud).cpu().numpy(), O.mttkrp_coo_f64(inds, vals, 0, U)) < 1e-5
+
+
+@pytest.mark.parametrize("dims", [[1 << 21, 1 << 21, 1 << 21], [(1 << 21) + 1, 1 << 21, (1 << 22) - 1],
+                                  [1 << 16, 1 << 16, 1 << 16, 1 << 16], [1 << 20, (1 << 18) + 5, 1 << 19, 1 << 17]])
+@pytest.mark.parametrize("fmt_type", [3, 8, 10, 12])
+def test_sort_key_widths(cuda, dims, fmt_type):
+    """Coordinates of 63, 64 and more than 64 bits in all: one sort whose keys
+    are unpacked, and two of which the second holds only the upper levels."""
+    import mmcsf
+    from test_gpu_builder import check_format
+    rng = np.random.default_rng(len(dims) + fmt_type)
+    inds, vals = random_tensor(rng, dims, 3000, [1.3] + [None] * (len(dims) - 1))
+    for a, d in zip(inds, dims):
+        a[rng.integers(0, len(a), 20)] = d - 1  # the largest coordinate
+    key = np.stack(inds)
+    _, first = np.unique(key, axis=1, return_index=True)
+    first = np.sort(first)
+    inds, vals = [a[first] for a in inds], vals[first]
+    t = mmcsf.Tensor.from_numpy(dims, inds, vals)
+    for mode in ([2] if fmt_type == 12 else range(len(dims))):
+        check_format(mmcsf, t, fmt_type, dims, inds, vals, mode, 128)
