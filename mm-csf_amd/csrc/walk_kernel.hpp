@@ -168,8 +168,14 @@ constexpr uint32_t kOobOffset = 0xFFFFF000u;
 template <int N, int G, int NB, int OP>
 constexpr bool kFactorOf = OP == kMttkrp && NB <= 2 && G >= 2 && !(N == 4 && G == 8);
 
+// 64 nonzeros a chunk; a block is 4 waves, neighbours in the tree.  Larger
+// blocks would join more of a hot slice's partial rows (below), but 12
+// neighbouring waves on one CU share its slow stretches: 768-thread blocks
+// cost 5 % on 4-D trees and 6 % on the CP passes.
+constexpr int kWalkWaves = 4;
+
 template <int N, int G, int NB, int TB, typename T, int VEC, int OP>
-__global__ __launch_bounds__(256, (OP == kMttkrp && N == 3 && NB == 1 && G * VEC <= 32) ? 3 : 2) void k_walk(WalkArgs a) {
+__global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 1 && G * VEC <= 32) ? 3 : 2) void k_walk(WalkArgs a) {
     static_assert(G == 1 || G == 2 || G == 4 || G == 8, "row groups of 1..8 lanes");
     static_assert(G % TB == 0, "steps per batch divide the steps of a chunk");
     static_assert(VEC % 4 == 0, "rows are written as float4");
@@ -207,7 +213,6 @@ __global__ __launch_bounds__(256, (OP == kMttkrp && N == 3 && NB == 1 && G * VEC
     const uint64_t total = a.cost[chunks];
     const uint32_t cb = wave_lower(a.cost, chunks, (uint32_t)(wv * total / waves));
     const uint32_t ce = wv + 1 == waves ? chunks : wave_lower(a.cost, chunks, (uint32_t)((wv + 1) * total / waves));
-    if (cb >= ce) return;  // the whole wave leaves together
     const int R = a.R;
     const uint32_t rowBytes = (uint32_t)R * (uint32_t)sizeof(T);
     // byte offset of this lane's columns in block b; blocks past R read columns 0..
@@ -225,24 +230,9 @@ __global__ __launch_bounds__(256, (OP == kMttkrp && N == 3 && NB == 1 && G * VEC
     [[maybe_unused]] const __amdgpu_buffer_rsrc_t rs2 = table_rsrc(a.U[2], a.tabBytes[2]);
     const uint32_t *__restrict__ ptrL = a.ptr[LF];
 
-    // leaf fiber (and 4-D level-1 entry) of the nonzero before the run; the
-    // unsigned wrap at x0 = 0 stands for -1
-    const uint32_t x0 = (uint32_t)(cb * 64);
-    const uint32_t f0 = wave_upper(ptrL, a.cnt[LF], x0);  // leaf fiber of x0
-    const uint32_t fcur = x0 == 0 ? kNone : (a.ptr[LF][f0] == x0 ? f0 - 1 : f0);
-    uint32_t jcur = kNone, j0 = f0;
-    if constexpr (N == 4) {
-        j0 = wave_upper(a.ptr[1], a.cnt[1], f0);
-        jcur = fcur == kNone ? kNone : (a.ptr[1][j0] == f0 && fcur != f0 ? j0 - 1 : j0);
-    }
     // the open slice (leaf fiber for TTM): its partial row from earlier
     // chunks is the carry `acc`, summed over the groups' shares
-    uint32_t scur = OP == kTtm ? f0 : a.slc[j0];
-    // whether the open slice began inside this wave's run: then every
-    // contribution to it passes through this wave, and its row is stored
-    // instead of added (the output starts zeroed)
-    bool inside = false;
-
+    uint32_t scur = kNone;
     float acc[NB][VEC];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -263,6 +253,34 @@ __global__ __launch_bounds__(256, (OP == kMttkrp && N == 3 && NB == 1 && G * VEC
             for (int e = 0; e < VEC; ++e) unsafeAtomicAdd(o + e, v[e]);
         }
     };
+
+    [[maybe_unused]] __shared__ float tail[kWalkWaves][kGrad ? NB * BW : 1];
+    [[maybe_unused]] __shared__ uint32_t tailRow[kWalkWaves];
+    if (cb >= ce) {
+        // no run: nothing to join (each wave passes one barrier, here or at the
+        // end; a condition around the whole run costs 6 registers more, and
+        // the widest case then a wave per SIMD)
+        if constexpr (kGrad) {
+            if (lane == 0) tailRow[threadIdx.x >> 6] = kNone;
+            __syncthreads();
+        }
+        return;
+    }
+    // leaf fiber (and 4-D level-1 entry) of the nonzero before the run; the
+    // unsigned wrap at x0 = 0 stands for -1
+    const uint32_t x0 = (uint32_t)(cb * 64);
+    const uint32_t f0 = wave_upper(ptrL, a.cnt[LF], x0);  // leaf fiber of x0
+    const uint32_t fcur = x0 == 0 ? kNone : (a.ptr[LF][f0] == x0 ? f0 - 1 : f0);
+    uint32_t jcur = kNone, j0 = f0;
+    if constexpr (N == 4) {
+        j0 = wave_upper(a.ptr[1], a.cnt[1], f0);
+        jcur = fcur == kNone ? kNone : (a.ptr[1][j0] == f0 && fcur != f0 ? j0 - 1 : j0);
+    }
+    scur = OP == kTtm ? f0 : a.slc[j0];
+    // whether the open slice began inside this wave's run: then every
+    // contribution to it passes through this wave, and its row is stored
+    // instead of added (the output starts zeroed)
+    bool inside = false;
 
     // Software pipeline over the chunks of the run.  A chunk's entries come
     // from three dependent reads: its words (leaf index, value, fiber-start
@@ -764,14 +782,39 @@ __global__ __launch_bounds__(256, (OP == kMttkrp && N == 3 && NB == 1 && G * VEC
         step(c + 2, w2, e2, w0, e0, w1);
     }
     if constexpr (kGrad) {
-        // the last slice may continue in the next wave
+        // The slice left open may continue in the next wave.  The waves of a
+        // block are neighbours in the tree, so on a hot slice all of them end
+        // in it: their rows are summed in float64 in LDS and the block adds
+        // each distinct row once.  A quarter of the float32 additions to a hot
+        // row's total: relative error of skewed modes 2.4e-7 -> 1.1e-7 (100M
+        // nonzeros, Zipf(1.2)), and fewer atomics waiting on one another.
+        const int w = threadIdx.x >> 6;
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
 #pragma unroll
             for (int off = G; off < 64; off <<= 1)
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) acc[b][e] += __shfl_xor(acc[b][e], off, 64);
-            if (g == 0) put(b, scur, acc[b], false);
+            if (g == 0)
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) tail[w][b * BW + k * VEC + e] = acc[b][e];
+        }
+        if (lane == 0) tailRow[w] = scur;
+        __syncthreads();
+        if (g == 0 && (w == 0 || tailRow[w - 1] != scur)) {
+            int we = w + 1;
+            while (we < (int)wavesPerBlock && tailRow[we] == scur) ++we;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                float v[VEC];
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) {
+                    double t = 0.0;
+                    for (int q = w; q < we; ++q) t += (double)tail[q][b * BW + k * VEC + e];
+                    v[e] = (float)t;
+                }
+                put(b, scur, v, false);
+            }
         }
     }
     if constexpr (kModel) {
@@ -809,12 +852,14 @@ void go(const WalkArgs &a, hipStream_t s) {
     int perCU = 0;
     MMCSF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fn, 256, 0));
     perCU = std::max(perCU, 1);
+    const uint64_t cus = (uint64_t)device_cu_count();
     const uint64_t chunks = ((uint64_t)a.nnz + 63) / 64;
-    uint64_t blocks = (uint64_t)device_cu_count() * perCU;
-    blocks = std::min(blocks, std::max<uint64_t>(1, (chunks + 3) / 4));
-    // a wave start is found by a search over the cost prefix; more waves
-    // than chunks would give empty waves only
-    fn<<<dim3((unsigned)blocks), dim3(256), 0, s>>>(a);
+    // a wave start is found by a search over the cost prefix; more waves than
+    // chunks would give empty waves only.  The waves of a small tensor are
+    // spread over the CUs.
+    const uint64_t block = std::min<uint64_t>(kWalkWaves, (chunks + cus - 1) / cus);
+    const uint64_t blocks = std::min<uint64_t>(cus * perCU, (chunks + block - 1) / block);
+    fn<<<dim3((unsigned)blocks), dim3((unsigned)(64 * block)), 0, s>>>(a);
     MMCSF_HIP(hipGetLastError());
 }
 
