@@ -331,9 +331,9 @@ void mttkrp_coo(const Format &f, const Factors &F, float *out, hipStream_t s);
 // through the mode's root tree when the format has one
 void mttkrp_mode(const Format &f, int mode, const Factors &F, float *out, hipStream_t s,
                  hipEvent_t evStart = nullptr, hipEvent_t evEnd = nullptr, bool zeroed = false);
-// root-level MTTKRP over 64-nonzero chunks (walk.hip); needs R % 4 == 0 and
-// the start bitmasks of the tree
-bool walk_supports(const Csf &c, int R);
+// root-level MTTKRP over 64-nonzero chunks (walk.hip); needs R >= 4 (a multiple
+// of four for bfloat16 rows) and the start bitmasks of the tree
+bool walk_supports(const Csf &c, int R, int dtype);
 void mttkrp_root(const Csf &c, const Factors &F, float *out, hipStream_t s, bool accumulate = false);
 // the walk's row loads are 16 bytes wide (8 for bfloat16 with R % 8 != 0):
 // factor tables of every level but skipLevel, and `out`, must be aligned to that

@@ -525,7 +525,7 @@ void mttkrp_csf(const Csf &c, const uint64_t *dims, int outLevel, const Factors 
     a.nnz = (uint32_t)c.nnz;
     a.R = F.R;
     a.perGroup = per_group_for(c.nnz, g.G);
-    if (outLevel == 0 && walk_supports(c, F.R)) {
+    if (outLevel == 0 && walk_supports(c, F.R, F.dtype)) {
         mttkrp_root(c, F, out, s, accumulate);  // checks the alignment its row loads need
         return;
     }
@@ -623,8 +623,8 @@ void mttkrp_hyb(const Hyb &h, const uint64_t *dims, const Factors &F, float *out
     }
     // the CSF part's walk loads wider rows than the COO / CSL kernels: refuse
     // its misaligned factors before any part is launched
-    if (h.csf.nnz && walk_supports(h.csf, F.R)) check_walk_align(h.csf, F, 0, out);
-    if (h.cslWalk.nnz && walk_supports(h.cslWalk, F.R)) check_walk_align(h.cslWalk, F, 0, out);
+    if (h.csf.nnz && walk_supports(h.csf, F.R, F.dtype)) check_walk_align(h.csf, F, 0, out);
+    if (h.cslWalk.nnz && walk_supports(h.cslWalk, F.R, F.dtype)) check_walk_align(h.cslWalk, F, 0, out);
     fill_zero(out, dims[h.order[0]] * (uint64_t)F.R, s);
     // COO part: slices with one nonzero; each output row is written once
     if (h.cooNnz) {
@@ -649,8 +649,8 @@ void mttkrp_hyb(const Hyb &h, const uint64_t *dims, const Factors &F, float *out
         }
     }
     // CSL part (3-D): walked as a tree of one-nonzero fibers; the CSL kernel
-    // where the walk cannot run (R % 4 != 0, tables above 4 GiB)
-    if (h.cslNnz && h.cslWalk.nnz && walk_supports(h.cslWalk, F.R)) {
+    // where the walk cannot run (R < 4, tables above 4 GiB)
+    if (h.cslNnz && h.cslWalk.nnz && walk_supports(h.cslWalk, F.R, F.dtype)) {
         mttkrp_root(h.cslWalk, F, out, s);
     } else if (h.cslNnz) {
         CslArgs a{};
@@ -689,7 +689,7 @@ void mttkrp_hyb(const Hyb &h, const uint64_t *dims, const Factors &F, float *out
         a.nnz = (uint32_t)c.nnz;
         a.R = F.R;
         a.perGroup = per_group_for(c.nnz, g.G);
-        if (walk_supports(c, F.R)) mttkrp_root(c, F, out, s);
+        if (walk_supports(c, F.R, F.dtype)) mttkrp_root(c, F, out, s);
         else if (N == 3) launch_csf_t<3, 0>(g, a, F.dtype, s);
         else launch_csf_t<4, 0>(g, a, F.dtype, s);
     }

@@ -56,9 +56,12 @@ static bool tables_fit(const Csf &c, int R) {
 }
 
 // row loads of the walk are VEC elements wide (16 bytes, or 8 bytes for
-// bfloat16 rows with R % 8 != 0); rows of `out` are written as float4
+// bfloat16 rows with R % 8 != 0); rows of `out` are written as float4.  At
+// ranks that four does not divide both are 16-byte accesses at 4-byte
+// boundaries.
 void check_walk_align(const Csf &c, const Factors &F, int skipLevel, const float *out) {
-    const uintptr_t need = (F.dtype == MMCSF_BF16 && F.R % 8 != 0) ? 8 : 16;
+    const bool ragged = F.R % 4 != 0;
+    const uintptr_t need = ragged ? 4 : (F.dtype == MMCSF_BF16 && F.R % 8 != 0) ? 8 : 16;
     for (int l = 0; l < c.ndims; ++l) {
         if (l == skipLevel) continue;
         const void *p = F.U[c.order[l]];
@@ -66,19 +69,23 @@ void check_walk_align(const Csf &c, const Factors &F, int skipLevel, const float
         MMCSF_REQUIRE(reinterpret_cast<uintptr_t>(p) % need == 0, MMCSF_ERR_ARG,
                       "factor pointer is not aligned to " + std::to_string(need) + " bytes");
     }
-    MMCSF_REQUIRE(!out || reinterpret_cast<uintptr_t>(out) % 16 == 0, MMCSF_ERR_ARG,
-                  "output pointer is not aligned to 16 bytes");
+    MMCSF_REQUIRE(!out || reinterpret_cast<uintptr_t>(out) % (ragged ? 4 : 16) == 0, MMCSF_ERR_ARG,
+                  ragged ? "output pointer is not aligned to 4 bytes" : "output pointer is not aligned to 16 bytes");
 }
 
-bool walk_supports(const Csf &c, int R) {
-    return R >= 1 && R <= 256 && R % 4 == 0 && tables_fit(c, R) &&
+// Ranks: every multiple of four, and any float32 rank from 4 on.  Below 4 the
+// row is narrower than one lane's load and the per-group kernel serves it.  At
+// R = 10 (HB-CSF, 3.3M nonzeros, 123457 x 70001 x 9973) the per-group kernel,
+// one column a lane in groups of 64, takes 324 us; the whole call 334 -> 53 us.
+bool walk_supports(const Csf &c, int R, int dtype) {
+    return R >= 4 && R <= 256 && (R % 4 == 0 || dtype == MMCSF_F32) && tables_fit(c, R) &&
            (c.nnz == 0 || (c.fbit.p && c.chunkCost.p && (c.ndims == 3 || c.sbit.p)));
 }
 
 void mttkrp_root(const Csf &c, const Factors &F, float *out, hipStream_t s, bool accumulate) {
     if (c.nnz == 0) return;
-    MMCSF_REQUIRE(walk_supports(c, F.R), MMCSF_ERR_UNSUPPORTED,
-                  "root walk needs R % 4 == 0, start bitmasks and factor tables below 4 GiB");
+    MMCSF_REQUIRE(walk_supports(c, F.R, F.dtype), MMCSF_ERR_UNSUPPORTED,
+                  "root walk needs R >= 4, start bitmasks and factor tables below 4 GiB");
     check_walk_align(c, F, 0, out);
     WalkArgs a = args_of(c, F);
     a.out = out;
@@ -120,7 +127,7 @@ void cp_gradient(const Csf &c, const Factors &F, const float *weights, float alp
 
 void ttm_fibers(const Csf &c, const Factors &F, float *Y, hipStream_t s) {
     if (c.nnz == 0) return;
-    MMCSF_REQUIRE(walk_supports(c, F.R), MMCSF_ERR_UNSUPPORTED, "TTM needs R % 4 == 0, R <= 256 and factor tables below 4 GiB");
+    MMCSF_REQUIRE(F.R % 4 == 0 && walk_supports(c, F.R, F.dtype), MMCSF_ERR_UNSUPPORTED, "TTM needs R % 4 == 0, R <= 256 and factor tables below 4 GiB");
     const int leaf = c.ndims - 1;
     const uintptr_t need = (F.dtype == MMCSF_BF16 && F.R % 8 != 0) ? 8 : 16;
     MMCSF_REQUIRE(F.U[c.order[leaf]] && reinterpret_cast<uintptr_t>(F.U[c.order[leaf]]) % need == 0, MMCSF_ERR_ARG,

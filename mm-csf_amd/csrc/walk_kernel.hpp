@@ -64,14 +64,17 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t table_rsrc(const void *p, uint
 // zeros without touching memory.
 template <typename T, int VEC>
 struct Raw;
+// four floats at a 4-byte boundary: rows whose rank no vector width divides
+// start anywhere, and a 16-byte global access needs 4-byte alignment only
+typedef float F4 __attribute__((ext_vector_type(4), aligned(4)));
 template <>
 struct Raw<float, 4> {
-    float4 q;
+    F4 q;
     __device__ __forceinline__ void load(const float *U, uint32_t off) {
-        q = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(U) + off);
+        q = *reinterpret_cast<const F4 *>(reinterpret_cast<const char *>(U) + off);
     }
     __device__ __forceinline__ void loadb(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-        q = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+        q = __builtin_bit_cast(F4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
     }
     __device__ __forceinline__ void get(float *o) const { o[0] = q.x; o[1] = q.y; o[2] = q.z; o[3] = q.w; }
     __device__ __forceinline__ void from_lane(const Raw &o, int src) {
@@ -174,7 +177,9 @@ constexpr bool kFactorOf = OP == kMttkrp && NB <= 2 && G >= 2 && !(N == 4 && G =
 // cost 5 % on 4-D trees and 6 % on the CP passes.
 constexpr int kWalkWaves = 4;
 
-template <int N, int G, int NB, int TB, typename T, int VEC, int OP>
+// RAG: ranks that VEC does not divide (float32 MTTKRP; its own instances, since
+// the column arithmetic costs the widest cases a wave per SIMD)
+template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG>
 __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 1 && G * VEC <= 32) ? 3 : 2) void k_walk(WalkArgs a) {
     static_assert(G == 1 || G == 2 || G == 4 || G == 8, "row groups of 1..8 lanes");
     static_assert(G % TB == 0, "steps per batch divide the steps of a chunk");
@@ -215,13 +220,16 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
     const uint32_t ce = wv + 1 == waves ? chunks : wave_lower(a.cost, chunks, (uint32_t)((wv + 1) * total / waves));
     const int R = a.R;
     const uint32_t rowBytes = (uint32_t)R * (uint32_t)sizeof(T);
-    // byte offset of this lane's columns in block b; blocks past R read columns 0..
+    // First of this lane's columns in block b.  RAG: the row's last lane has
+    // fewer than VEC columns of its own; it takes the last VEC columns of the
+    // row instead, and computes the ones that it shares with the lane before it
+    // alike.  Blocks past R read columns 0..
+    auto colOf = [&](int b) { return RAG ? std::min(b * BW + k * VEC, R - VEC) : b * BW + k * VEC; };
+    // byte offset of the columns
     uint32_t colBytes[NB];
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        const int col = b * BW + k * VEC;
-        colBytes[b] = col < R ? (uint32_t)col * (uint32_t)sizeof(T) : 0u;
-    }
+    for (int b = 0; b < NB; ++b)
+        colBytes[b] = b * BW + k * VEC < R ? (uint32_t)colOf(b) * (uint32_t)sizeof(T) : 0u;
     const T *U0 = static_cast<const T *>(a.U[0]);
     const T *U1 = static_cast<const T *>(a.U[1]);
     const T *U2 = static_cast<const T *>(a.U[2]);
@@ -244,13 +252,15 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
     auto put = [&](int b, uint32_t row, const float *v, bool store) {
         const int col = b * BW + k * VEC;
         if (row == kNone || col >= R) return;
-        float *o = a.out + (size_t)row * R + col;
+        const int c0 = colOf(b);
+        float *o = a.out + (size_t)row * R + c0;
         if (store && !a.accum) {
 #pragma unroll
-            for (int e = 0; e < VEC; e += 4) *reinterpret_cast<float4 *>(o + e) = make_float4(v[e], v[e + 1], v[e + 2], v[e + 3]);
+            for (int e = 0; e < VEC; e += 4) *reinterpret_cast<F4 *>(o + e) = F4{v[e], v[e + 1], v[e + 2], v[e + 3]};
         } else {
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) unsafeAtomicAdd(o + e, v[e]);
+            for (int e = 0; e < VEC; ++e)
+                if (!RAG || c0 + e >= col) unsafeAtomicAdd(o + e, v[e]);  // shared columns are the other lane's
         }
     };
 
@@ -846,9 +856,9 @@ Cfg pick(int R, int dtype) {
     return c;
 }
 
-template <int N, int G, int NB, int TB, typename T, int VEC, int OP>
+template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG>
 void go(const WalkArgs &a, hipStream_t s) {
-    auto fn = k_walk<N, G, NB, TB, T, VEC, OP>;
+    auto fn = k_walk<N, G, NB, TB, T, VEC, OP, RAG>;
     int perCU = 0;
     MMCSF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fn, 256, 0));
     perCU = std::max(perCU, 1);
@@ -867,7 +877,12 @@ template <int N, typename T, int VEC, int OP>
 void dispatch(const Cfg &c, const WalkArgs &a, hipStream_t s) {
 #define MMCSF_WALK(GG, BB, TT)                       \
     if (c.G == GG && c.NB == BB && c.TB == TT) {     \
-        go<N, GG, BB, TT, T, VEC, OP>(a, s);         \
+        if constexpr (OP == kMttkrp && std::is_same_v<T, float>)  \
+            if (a.R % VEC != 0) {                    \
+                go<N, GG, BB, TT, T, VEC, OP, true>(a, s); \
+                return;                              \
+            }                                        \
+        go<N, GG, BB, TT, T, VEC, OP, false>(a, s);  \
         return;                                      \
     }
     MMCSF_WALK(1, 1, 1)
@@ -894,7 +909,7 @@ void dispatch(const Cfg &c, const WalkArgs &a, hipStream_t s) {
 template <int OP>
 void walk_preload() {
     hipFuncAttributes attr;
-    MMCSF_HIP(hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(k_walk<3, 8, 1, 8, float, 4, OP>)));
+    MMCSF_HIP(hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(k_walk<3, 8, 1, 8, float, 4, OP, false>)));
 }
 
 template <int OP>

@@ -108,3 +108,40 @@ def test_sort_key_widths(cuda, dims, fmt_type):
     t = mmcsf.Tensor.from_numpy(dims, inds, vals)
     for mode in ([2] if fmt_type == 12 else range(len(dims))):
         check_format(mmcsf, t, fmt_type, dims, inds, vals, mode, 128)
+
+
+# ---- MTTKRP at ranks that no vector width divides ---------------------------------
+
+def offset_copy(t, off):
+    """A contiguous device copy of t that starts `off` floats into its storage."""
+    import torch
+    s = torch.empty(t.numel() + off, dtype=t.dtype, device=t.device)
+    v = s[off:].view(t.shape)
+    v.copy_(t)
+    return v
+
+
+@pytest.mark.parametrize("R", [1, 3, 4, 5, 6, 7, 8, 9, 10, 15, 17, 25, 31, 33, 50, 63, 65, 127, 129, 253, 255])
+@pytest.mark.parametrize("dims,skew,nnz", [([211, 90, 57], [1.2, None, 1.1], 9000),
+                                           ([60, 37, 25, 14], [1.1, None, 1.2, None], 7001)])
+def test_mttkrp_ragged_ranks(cuda, dims, skew, nnz, R):
+    """Each side of the row groups' widths (4, 8, 16, 32, 64, 128, 256 columns);
+    factors and output at 4-byte boundaries where the rank allows them."""
+    import torch
+    import mmcsf
+    import oracle as O
+    rng = np.random.default_rng(R)
+    inds, vals = random_tensor(rng, dims, nnz, skew)
+    t = mmcsf.Tensor.from_numpy(dims, inds, vals)
+    U = [rng.random((d, R)).astype(np.float32) for d in dims]
+    off = 1 if R % 4 else 0
+    Ud = [offset_copy(torch.from_numpy(u).to(cuda), off) for u in U]
+    ref = [O.mttkrp_coo_f64(inds, vals, m, U) for m in range(len(dims))]
+    f = mmcsf.Format(t, 12, fbr_threshold=16)
+    for m in range(len(dims)):
+        out = offset_copy(torch.full((dims[m], R), 7.0, device=cuda), off)
+        mmcsf.mttkrp(f, m, Ud, out=out)
+        assert rel(out.cpu().numpy(), ref[m]) < 1e-5, f"mode {m}"
+    for fmt_type in (8, 10):
+        g = mmcsf.Format(t, fmt_type, mode=1, fbr_threshold=16)
+        assert rel(mmcsf.mttkrp(g, 1, Ud).cpu().numpy(), ref[1]) < 1e-5, f"type {fmt_type}"
