@@ -442,7 +442,7 @@ uint64_t csf_bytes(const mmcsf::Csf &c) {
 }
 
 uint64_t format_bytes(const mmcsf::Format &f) {
-    uint64_t b = csf_bytes(f.csf) + bytes_of(f.cooVals) + csf_bytes(f.hyb.csf) + csf_bytes(f.hyb.cslWalk) + bytes_of(f.hyb.cooVal) +
+    uint64_t b = csf_bytes(f.csf) + bytes_of(f.cooVals) + bytes_of(f.cooCost) + csf_bytes(f.hyb.csf) + csf_bytes(f.hyb.cslWalk) + bytes_of(f.hyb.cooVal) +
                  bytes_of(f.hyb.cslPtr) + bytes_of(f.hyb.cslIdx) + bytes_of(f.hyb.cslInd1) +
                  bytes_of(f.hyb.cslInd2) + bytes_of(f.hyb.cslVal) + bytes_of(f.hyb.cslBinList);
     for (int l = 0; l < mmcsf::kMaxDims; ++l) {
@@ -846,6 +846,7 @@ int mmcsf_format_build(const mmcsf_tensor *th, int type, const mmcsf_options *op
             if (type == MMCSF_TYPE_COO || type == MMCSF_TYPE_COO_CPU) {
                 for (int l = 0; l < t.ndims; ++l) f.cooOrder[l] = order[l];
                 sort_coo(t, order, f.cooKeys, f.cooVals, s, nullptr, true);
+                build_row_cost(f.cooKeys[0].p, t.nnz, t.dims[order[0]], f.cooCost, s);
             } else {
                 const bool bcsf = type != MMCSF_TYPE_HBCSF;  // types 8, 9, 13, 14
                 DevArray<uint32_t> pos;

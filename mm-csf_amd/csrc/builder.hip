@@ -660,6 +660,33 @@ void build_walk_bits(Csf &c, hipStream_t s) {
     MMCSF_HIP(hipStreamSynchronize(s));
 }
 
+// rows of sorted nonzeros starting in each 64-nonzero chunk, as the chunk's cost
+// (64, and ws per start: row writes and the join of the group runs)
+__global__ void k_row_cost(const uint32_t *__restrict__ key, uint64_t n, bool plain, uint32_t ws,
+                           uint32_t *__restrict__ cost) {
+    const uint64_t x = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+    const bool starts = x < n && (x == 0 || key[x] != key[x - 1]);
+    const uint64_t m = __ballot(starts);
+    if (x < n && (threadIdx.x & 63) == 0) cost[x >> 6] = plain ? 1u : 64u + ws * (uint32_t)__popcll(m);
+}
+
+void build_row_cost(const uint32_t *key, uint64_t n, uint64_t rows, DevArray<uint32_t> &prefix, hipStream_t s) {
+    const uint64_t chunks = (n + 63) / 64;
+    prefix.alloc(chunks + 1);
+    uint64_t total = 0;
+    if (chunks) {
+        Temp tmp;
+        TmpArray<uint32_t> cost(chunks);
+        const uint32_t ws = 24;  // as for the trees
+        const bool plain = chunks * 64 + ws * std::min(n, rows) >= 0xF0000000ull;
+        hipLaunchKernelGGL(k_row_cost, dim3(nblk(n)), dim3(kBS), 0, s, key, n, plain, ws, cost.p);
+        total = exclusive_sum(cost.p, prefix.p, chunks, s, tmp);
+    }
+    hipLaunchKernelGGL(k_set, dim3(1), dim3(1), 0, s, prefix.p, chunks, (uint32_t)total);
+    MMCSF_HIP(hipGetLastError());
+    MMCSF_HIP(hipStreamSynchronize(s));
+}
+
 // ---------------------------------------------------------------------------
 // make_TiledBin (util.h:1887-1952)
 // ---------------------------------------------------------------------------

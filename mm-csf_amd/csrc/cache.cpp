@@ -297,8 +297,10 @@ void format_load(const char *path, Format &f) {
     MMCSF_REQUIRE(r.pod<uint32_t>() == kByteOrder, MMCSF_ERR_IO, "format cache written with another byte order");
     format_fields(r, f);
     st.drain();
-    // derived from the stored CSL arrays: rebuilt, not stored
+    // derived from the stored arrays: rebuilt, not stored
     build_csl_walk(f.hyb, st.s);
+    if (f.cooVals.p && f.cooKeys[0].n == f.nnz)
+        build_row_cost(f.cooKeys[0].p, f.nnz, f.dims[f.cooOrder[0]], f.cooCost, st.s);
     r.bytes(m, 8);
     MMCSF_REQUIRE(std::memcmp(m, kEnd, 8) == 0 && r.left == 0, MMCSF_ERR_IO, "format cache: bad end of file");
     MMCSF_REQUIRE(f.ndims == 3 || f.ndims == 4, MMCSF_ERR_IO, "format cache: bad tensor order");

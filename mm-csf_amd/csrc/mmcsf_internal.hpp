@@ -257,6 +257,7 @@ struct Format {
     int cooOrder[kMaxDims] = {0, 1, 2, 3};
     DevArray<uint32_t> cooKeys[kMaxDims];
     DevArray<float> cooVals;
+    DevArray<uint32_t> cooCost;          // cost prefix over 64-nonzero chunks (derived, not stored)
     // types 8 / 12
     Csf csf;
     // type 12: a root tree per mode other than the partition's root, so every
@@ -295,6 +296,9 @@ void build_csf(int ndims, const uint64_t *dims, uint64_t nnz, const int *order,
                DevArray<uint32_t> *keys, DevArray<float> &&vals, uint64_t fbrThreshold,
                uint64_t fbrSThreshold, Csf &out, hipStream_t s);
 
+// cost prefix over the 64-nonzero chunks of nonzeros sorted by `key` (output
+// rows below `rows`)
+void build_row_cost(const uint32_t *key, uint64_t n, uint64_t rows, DevArray<uint32_t> &cost, hipStream_t s);
 void build_bins_tiled(Csf &c, hipStream_t s);           // make_TiledBin
 void build_hyb(int ndims, const uint64_t *dims, Csf &&src, Hyb &out, hipStream_t s);
 // the CSL part of a built 3-D HB-CSF as a walkable tree (h.cslWalk)
@@ -327,6 +331,9 @@ void mttkrp_csf(const Csf &c, const uint64_t *dims, int outLevel, const Factors 
                 hipStream_t s, hipEvent_t evStart = nullptr, hipEvent_t evEnd = nullptr, bool accumulate = false,
                 bool zeroed = false);
 void mttkrp_coo(const Format &f, const Factors &F, float *out, hipStream_t s);
+// the same as a chunked walk (walk.hip); `out` zeroed by the caller
+bool coo_walk_supports(const Format &f, const Factors &F);
+void mttkrp_coo_walk(const Format &f, const Factors &F, float *out, hipStream_t s);
 // MTTKRP of tensor mode `mode` of a CSF-based format (types 8 and 12),
 // through the mode's root tree when the format has one
 void mttkrp_mode(const Format &f, int mode, const Factors &F, float *out, hipStream_t s,

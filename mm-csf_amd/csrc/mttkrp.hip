@@ -597,6 +597,10 @@ void mttkrp_coo(const Format &f, const Factors &F, float *out, hipStream_t s) {
             check_align(a.U[l], F.dtype, g);
         }
     }
+    if (coo_walk_supports(f, F)) {
+        mttkrp_coo_walk(f, F, out, s);
+        return;
+    }
     a.val = f.cooVals.p;
     a.out = out;
     a.nnz = (uint32_t)f.nnz;

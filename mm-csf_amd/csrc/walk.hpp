@@ -65,6 +65,13 @@ struct WalkArgs {
     int R;
 };
 
+// Where a nonzero's coordinates come from.
+enum WalkSrc : int {
+    kTree = 0,  // a CSF tree rooted at the output mode
+    kCoo = 1,   // sorted COO (MTTKRP only): idx[l] holds level l's coordinate of
+                // every nonzero; every nonzero is a leaf fiber of its own
+};
+
 enum WalkOp : int {
     kMttkrp = 0,      // out += v * product of the other rows
     kLossGrad = 1,    // out += alpha * e * product; sumsq += e^2
@@ -75,9 +82,9 @@ enum WalkOp : int {
 
 // one traversal of the root tree of c; instantiated per operation in its
 // own translation unit (walk_<op>.hip)
-template <int OP>
-void walk_launch(const Csf &c, const Factors &F, const WalkArgs &a, hipStream_t s);
-template <int OP>
+template <int OP, int SRC = kTree>
+void walk_launch(int ndims, const Factors &F, const WalkArgs &a, hipStream_t s);
+template <int OP, int SRC = kTree>
 void walk_preload();
 
 }  // namespace mmcsf

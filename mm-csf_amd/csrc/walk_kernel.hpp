@@ -179,11 +179,12 @@ constexpr int kWalkWaves = 4;
 
 // RAG: ranks that VEC does not divide (float32 MTTKRP; its own instances, since
 // the column arithmetic costs the widest cases a wave per SIMD)
-template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG>
+template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG, int SRC>
 __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 1 && G * VEC <= 32) ? 3 : 2) void k_walk(WalkArgs a) {
     static_assert(G == 1 || G == 2 || G == 4 || G == 8, "row groups of 1..8 lanes");
     static_assert(G % TB == 0, "steps per batch divide the steps of a chunk");
     static_assert(VEC % 4 == 0, "rows are written as float4");
+    static_assert(SRC == kTree || OP == kMttkrp, "only the MTTKRP walks other sources than trees");
     constexpr bool kModel = OP == kLossGrad || OP == kLossResid;
     constexpr bool kGrad = OP != kLossResid;  // writes rows of `out`
     // multiplies the rows of the upper levels; rows of `out` are keyed by
@@ -236,8 +237,6 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
     const T *UL = static_cast<const T *>(a.U[N - 1]);
     [[maybe_unused]] const __amdgpu_buffer_rsrc_t rs1 = table_rsrc(a.U[1], a.tabBytes[1]);
     [[maybe_unused]] const __amdgpu_buffer_rsrc_t rs2 = table_rsrc(a.U[2], a.tabBytes[2]);
-    const uint32_t *__restrict__ ptrL = a.ptr[LF];
-
     // the open slice (leaf fiber for TTM): its partial row from earlier
     // chunks is the carry `acc`, summed over the groups' shares
     uint32_t scur = kNone;
@@ -276,17 +275,23 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
         }
         return;
     }
-    // leaf fiber (and 4-D level-1 entry) of the nonzero before the run; the
-    // unsigned wrap at x0 = 0 stands for -1
     const uint32_t x0 = (uint32_t)(cb * 64);
-    const uint32_t f0 = wave_upper(ptrL, a.cnt[LF], x0);  // leaf fiber of x0
-    const uint32_t fcur = x0 == 0 ? kNone : (a.ptr[LF][f0] == x0 ? f0 - 1 : f0);
-    uint32_t jcur = kNone, j0 = f0;
-    if constexpr (N == 4) {
-        j0 = wave_upper(a.ptr[1], a.cnt[1], f0);
-        jcur = fcur == kNone ? kNone : (a.ptr[1][j0] == f0 && fcur != f0 ? j0 - 1 : j0);
+    [[maybe_unused]] uint32_t fcur = kNone, jcur = kNone;
+    if constexpr (SRC == kTree) {
+        // leaf fiber (and 4-D level-1 entry) of the nonzero before the run; the
+        // unsigned wrap at x0 = 0 stands for -1
+        const uint32_t *__restrict__ ptrL = a.ptr[LF];
+        const uint32_t f0 = wave_upper(ptrL, a.cnt[LF], x0);  // leaf fiber of x0
+        fcur = x0 == 0 ? kNone : (a.ptr[LF][f0] == x0 ? f0 - 1 : f0);
+        uint32_t j0 = f0;
+        if constexpr (N == 4) {
+            j0 = wave_upper(a.ptr[1], a.cnt[1], f0);
+            jcur = fcur == kNone ? kNone : (a.ptr[1][j0] == f0 && fcur != f0 ? j0 - 1 : j0);
+        }
+        scur = OP == kTtm ? f0 : a.slc[j0];
+    } else {
+        scur = a.idx[0][x0];
     }
-    scur = OP == kTtm ? f0 : a.slc[j0];
     // whether the open slice began inside this wave's run: then every
     // contribution to it passes through this wave, and its row is stored
     // instead of added (the output starts zeroed)
@@ -317,9 +322,12 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
         w.lw = a.leaf[x];
         // one 8-byte word per chunk, read through the scalar cache (the chunk
         // index is wave-uniform; chunks past the tensor read the last word)
-        const uint32_t cw = __builtin_amdgcn_readfirstlane(std::min(c, lastC));
-        using ConstU64 = const __attribute__((address_space(4))) uint64_t;
-        w.word = *reinterpret_cast<ConstU64 *>(reinterpret_cast<uintptr_t>(a.fbit + 2 * cw));
+        w.word = 0;
+        if constexpr (SRC == kTree) {
+            const uint32_t cw = __builtin_amdgcn_readfirstlane(std::min(c, lastC));
+            using ConstU64 = const __attribute__((address_space(4))) uint64_t;
+            w.word = *reinterpret_cast<ConstU64 *>(reinterpret_cast<uintptr_t>(a.fbit + 2 * cw));
+        }
         w.ps = 0;
         if constexpr (kPos) w.ps = a.pos[x];
         w.v = 0.f;
@@ -332,6 +340,13 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
     [[maybe_unused]] const uint32_t lastF = a.cnt[LF] - 1, lastJ = a.cnt[1] - 1;
     auto readEntries = [&](uint32_t c, Words &w, Entries &q) {
         const uint32_t x = c * 64 + (uint32_t)lane;
+        if constexpr (SRC == kCoo) {
+            const uint32_t xc = std::min(x, lastX);
+            q.s = a.idx[0][xc];
+            q.i1 = a.idx[1][xc];
+            q.i2 = N == 4 ? a.idx[2][xc] : 0u;
+            return;
+        }
         const bool start = x < a.nnz && ((w.word >> lane) & 1ull);
         const uint64_t fm = __ballot(start);
         const uint32_t f = fB + (uint32_t)__popcll(fm & low_bits((uint32_t)lane + 1));
@@ -856,9 +871,9 @@ Cfg pick(int R, int dtype) {
     return c;
 }
 
-template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG>
+template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG, int SRC>
 void go(const WalkArgs &a, hipStream_t s) {
-    auto fn = k_walk<N, G, NB, TB, T, VEC, OP, RAG>;
+    auto fn = k_walk<N, G, NB, TB, T, VEC, OP, RAG, SRC>;
     int perCU = 0;
     MMCSF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fn, 256, 0));
     perCU = std::max(perCU, 1);
@@ -873,16 +888,16 @@ void go(const WalkArgs &a, hipStream_t s) {
     MMCSF_HIP(hipGetLastError());
 }
 
-template <int N, typename T, int VEC, int OP>
+template <int N, typename T, int VEC, int OP, int SRC>
 void dispatch(const Cfg &c, const WalkArgs &a, hipStream_t s) {
 #define MMCSF_WALK(GG, BB, TT)                       \
     if (c.G == GG && c.NB == BB && c.TB == TT) {     \
         if constexpr (OP == kMttkrp && std::is_same_v<T, float>)  \
             if (a.R % VEC != 0) {                    \
-                go<N, GG, BB, TT, T, VEC, OP, true>(a, s); \
+                go<N, GG, BB, TT, T, VEC, OP, true, SRC>(a, s); \
                 return;                              \
             }                                        \
-        go<N, GG, BB, TT, T, VEC, OP, false>(a, s);  \
+        go<N, GG, BB, TT, T, VEC, OP, false, SRC>(a, s); \
         return;                                      \
     }
     MMCSF_WALK(1, 1, 1)
@@ -906,23 +921,23 @@ void dispatch(const Cfg &c, const WalkArgs &a, hipStream_t s) {
 
 // loads this translation unit's code object on the current device (a kernel
 // attribute query), so that the first traversal does not pay for it
-template <int OP>
+template <int OP, int SRC>
 void walk_preload() {
     hipFuncAttributes attr;
-    MMCSF_HIP(hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(k_walk<3, 8, 1, 8, float, 4, OP, false>)));
+    MMCSF_HIP(hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(k_walk<3, 8, 1, 8, float, 4, OP, false, SRC>)));
 }
 
-template <int OP>
-void walk_launch(const Csf &c, const Factors &F, const WalkArgs &a, hipStream_t s) {
+template <int OP, int SRC>
+void walk_launch(int ndims, const Factors &F, const WalkArgs &a, hipStream_t s) {
     const Cfg cfg = pick(F.R, F.dtype);
-    if (c.ndims == 3) {
-        if (F.dtype == MMCSF_F32) dispatch<3, float, 4, OP>(cfg, a, s);
-        else if (cfg.VEC == 8) dispatch<3, uint16_t, 8, OP>(cfg, a, s);
-        else dispatch<3, uint16_t, 4, OP>(cfg, a, s);
+    if (ndims == 3) {
+        if (F.dtype == MMCSF_F32) dispatch<3, float, 4, OP, SRC>(cfg, a, s);
+        else if (cfg.VEC == 8) dispatch<3, uint16_t, 8, OP, SRC>(cfg, a, s);
+        else dispatch<3, uint16_t, 4, OP, SRC>(cfg, a, s);
     } else {
-        if (F.dtype == MMCSF_F32) dispatch<4, float, 4, OP>(cfg, a, s);
-        else if (cfg.VEC == 8) dispatch<4, uint16_t, 8, OP>(cfg, a, s);
-        else dispatch<4, uint16_t, 4, OP>(cfg, a, s);
+        if (F.dtype == MMCSF_F32) dispatch<4, float, 4, OP, SRC>(cfg, a, s);
+        else if (cfg.VEC == 8) dispatch<4, uint16_t, 8, OP, SRC>(cfg, a, s);
+        else dispatch<4, uint16_t, 4, OP, SRC>(cfg, a, s);
     }
 }
 

@@ -2,6 +2,6 @@
 #include "walk_kernel.hpp"
 
 namespace mmcsf {
-template void walk_launch<kTtm>(const Csf &, const Factors &, const WalkArgs &, hipStream_t);
+template void walk_launch<kTtm>(int, const Factors &, const WalkArgs &, hipStream_t);
 template void walk_preload<kTtm>();
 }  // namespace mmcsf

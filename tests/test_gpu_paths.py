@@ -145,3 +145,32 @@ def test_mttkrp_ragged_ranks(cuda, dims, skew, nnz, R):
     for fmt_type in (8, 10):
         g = mmcsf.Format(t, fmt_type, mode=1, fbr_threshold=16)
         assert rel(mmcsf.mttkrp(g, 1, Ud).cpu().numpy(), ref[1]) < 1e-5, f"type {fmt_type}"
+
+
+# ---- COO type as a walk -------------------------------------------------------------
+
+@pytest.mark.parametrize("nnz", [1, 63, 64, 65, 4097, 40_000])
+@pytest.mark.parametrize("rows", [1, 50, 100_000])  # one slice, slices over many chunks, a slice per nonzero
+@pytest.mark.parametrize("N", [3, 4])
+def test_coo_walk(cuda, N, rows, nnz):
+    import torch
+    import mmcsf
+    import oracle as O
+    rng = np.random.default_rng(nnz + rows)
+    dims = [rows, 300, 170, 90][:N]
+    inds, vals = random_tensor(rng, dims, nnz, [1.3 if rows > 50 else None] + [None] * (N - 1))
+    f = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), 3, mode=0)
+    for R in (3, 4, 10, 16, 32, 64, 136):
+        U = [rng.random((d, R)).astype(np.float32) for d in dims]
+        Ud = [torch.from_numpy(u).to(cuda) for u in U]
+        ref = O.mttkrp_coo_f64(inds, vals, 0, U)
+        out = torch.full((rows, R), 5.0, device=cuda)
+        assert rel(mmcsf.mttkrp(f, 0, Ud, out=out).cpu().numpy(), ref) < 1e-5, R
+        if R % 4 == 0:
+            # bfloat16 rows at 16 and (accepted, per-group kernel) 8 byte boundaries
+            Ub = [u.to(torch.bfloat16) for u in Ud]
+            Ur = [u.float().cpu().numpy() for u in Ub]
+            ref = O.mttkrp_coo_f64(inds, vals, 0, Ur)
+            for off in (0, 4):
+                got = mmcsf.mttkrp(f, 0, [offset_copy(u, off) for u in Ub])
+                assert rel(got.cpu().numpy(), ref) < 1e-5, (R, off)
