@@ -76,7 +76,8 @@ typedef struct mmcsf_options {
     uint64_t seed;            /* -x seed of generated inputs (new flag, 1) */
     int modeTrees;            /* -a 1|0 (new flag, 1): MM-CSF also keeps a root tree per
                                  other mode, so every mode's MTTKRP is a root traversal;
-                                 0 = single tree, non-root modes scatter (the reference) */
+                                 0 = the reference's single tree, the other modes through its
+                                 level maps */
     int mixedPart;            /* -M 1|0 (new flag, 0): MM-CSF partitions the nonzeros by the
                                  reference's heuristic (mm_partition_reuseBased,
                                  util.h:2386-2512, threshold -h) instead of its override
@@ -201,7 +202,7 @@ typedef struct mmcsf_format_info {
                                   mode m traverses (its root tree, else the MM-CSF tree) */
     uint64_t deviceBytes;      /* device memory held by the format (every tree, its
                                   pointer / index / value arrays, start bitmasks, chunk
-                                  costs, bins and hot-row tables) */
+                                  costs, bins and level maps) */
     uint64_t partNnz[4];       /* MM-CSF: nonzeros per partition (X.totnnzPerPart) */
     int mixedPart;             /* MM-CSF built with -M 1 */
     int modeTreeOrder[4][4];   /* MM-CSF and one-tree types: the mode order of the tree
@@ -241,12 +242,13 @@ void mmcsf_format_free(mmcsf_format *f);
  * rebuilds every format from the .tns text on each run, util.h:313-370 and
  * mttkrp.cu:104-395).  mmcsf_format_save writes every array of every tree the
  * format holds (the reference's arrays, the per-mode root trees, the
- * mixed-mode partitions, start bitmasks, chunk costs, bins, hot-row tables)
- * after an 8-byte magic "MMCSFFMT", a uint32 version (1) and a byte-order
- * mark; mmcsf_format_load rebuilds the format from it, equal bit for bit to
- * the one saved, without reading text, sorting or building.  Errors
- * (MMCSF_ERR_IO) on a missing file, another version or byte order, a
- * truncated file or a bad end mark.
+ * mixed-mode partitions, start bitmasks, chunk costs, bins) after an 8-byte
+ * magic "MMCSFFMT", a uint32 version (2) and a byte-order mark;
+ * mmcsf_format_load rebuilds the format from it, equal bit for bit to the one
+ * saved, without reading text or sorting the tensor (level maps are derived
+ * again from the trees).  Version-1 files load too.  Errors (MMCSF_ERR_IO) on
+ * a missing file, another version or byte order, a truncated file or a bad end
+ * mark.
  */
 int mmcsf_format_save(const mmcsf_format *f, const char *path);
 int mmcsf_format_load(const char *path, mmcsf_format **out);
@@ -276,8 +278,8 @@ int mmcsf_format_to_tensor(const mmcsf_format *f, mmcsf_tensor **out);
  *                                    (mttkrp_gpu.h:75-81, mttkrp_gpu.cu:3380, 3860)
  * COO, B-CSF and HB-CSF serve their root mode (modeOrder[0]) only, like
  * the reference; MM-CSF and the one-tree types 9 / 13 / 14 serve every mode
- * (types 9 / 13 / 14: the root mode walks the tree, the other modes scatter
- * from their level, mttkrp_gpu.cu:2131-2528, 2853-3378, and for type 13 the
+ * (types 9 / 13 / 14: the root mode walks the tree, the other modes take their
+ * rows from their level, mttkrp_gpu.cu:2131-2528, 2853-3378, and for type 13 the
  * host routines MTTKRP_HCSR_CPU[_4D] / _mode1 / _mode2, mttkrp_cpu.cpp:160-348,
  * whose 3-D-only mode1 / mode2 roles this generalises to 4-D: every mode of a
  * 4-D type-13 format is its exact MTTKRP).

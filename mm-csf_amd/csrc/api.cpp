@@ -417,7 +417,7 @@ void build_mixed(const Tensor &t, const mmcsf_options *opt, bool nat, Format &f,
         sort_coo(sub, orders[p], keys, vals, s);
         const uint64_t fs = N == 4 ? 128 : kNoSplit;  // util.h:1325-1326
         build_csf(N, t.dims, sub.nnz, orders[p], keys, std::move(vals), opt->fbrThreashold, fs, f.part[p], s);
-        for (int l = 1; l < N; ++l) build_hot_table(f.part[p], l, t.dims[orders[p][l]], f.part[p].hot[l], s);
+        build_level_maps(f.part[p], s);
         MMCSF_HIP(hipStreamSynchronize(s));
     }
     f.partOrder = std::move(walk);
@@ -437,7 +437,8 @@ uint64_t csf_bytes(const mmcsf::Csf &c) {
     uint64_t b = bytes_of(c.leaf) + bytes_of(c.vals) + bytes_of(c.pos) + bytes_of(c.fbrSlc) + bytes_of(c.fbit) +
                  bytes_of(c.sbit) + bytes_of(c.chunkCost) + bytes_of(c.binList);
     for (int l = 0; l < mmcsf::kMaxDims - 1; ++l) b += bytes_of(c.ptr[l]) + bytes_of(c.idx[l]);
-    for (int l = 0; l < mmcsf::kMaxDims; ++l) b += bytes_of(c.hot[l].rows) + bytes_of(c.hot[l].tgt);
+    b += bytes_of(c.frank) + bytes_of(c.jrank);
+    for (int l = 0; l < mmcsf::kMaxDims; ++l) b += bytes_of(c.map[l].ord) + bytes_of(c.map[l].cost);
     return b;
 }
 
@@ -838,8 +839,7 @@ int mmcsf_format_build(const mmcsf_tensor *th, int type, const mmcsf_options *op
                     f.hasTree[m] = true;
                 }
             } else {
-                // privatisation tables of the scatter levels (every level but the root)
-                for (int l = 1; l < t.ndims; ++l) build_hot_table(f.csf, l, t.dims[order[l]], f.csf.hot[l], s);
+                build_level_maps(f.csf, s);  // the other modes, from the one tree
             }
         } else {
             order_tensormode(t.ndims, t.dims, (int)opt->mode, nat, order);
@@ -857,9 +857,8 @@ int mmcsf_format_build(const mmcsf_tensor *th, int type, const mmcsf_options *op
                     f.csf.pos = std::move(pos);
                     // type 13 is create_HCSR alone (mttkrp.cu:244-247): no slice bins
                     if (type != MMCSF_TYPE_SINGLECSF) build_bins_tiled(f.csf, s);
-                    // one-tree all-mode types: the other modes scatter from their level
-                    if (type != MMCSF_TYPE_BCSF)
-                        for (int l = 1; l < t.ndims; ++l) build_hot_table(f.csf, l, t.dims[order[l]], f.csf.hot[l], s);
+                    // one-tree all-mode types: the other modes from their level
+                    if (type != MMCSF_TYPE_BCSF) build_level_maps(f.csf, s);
                 } else {
                     build_hyb(t.ndims, t.dims, std::move(f.csf), f.hyb, s);
                     build_csl_walk(f.hyb, s);

@@ -17,6 +17,7 @@
 #include <numeric>
 
 #include "mmcsf_internal.hpp"
+#include "mttkrp_kernels.hpp"
 
 namespace mmcsf {
 
@@ -1029,65 +1030,62 @@ void build_hyb(int N, const uint64_t *dims, Csf &&src, Hyb &h, hipStream_t s) {
 
 
 // ---------------------------------------------------------------------------
-// Hot-row tables of a scatter level: the rows of level `level` used most
-// often (by nonzeros for the leaf level, by tree entries for fiber levels)
-// are ranked; the level's index array is re-encoded so that a row of rank
-// r < kMaxHot reads kHotBit | r and every other row reads its coordinate.
-// The scatter kernels accumulate ranked rows in LDS.
+// Level maps: the nonzeros of a tree in the order of one level's coordinates.
 // ---------------------------------------------------------------------------
 namespace {
 
-__global__ void k_hist(const uint32_t *__restrict__ idx, uint64_t n, uint32_t *__restrict__ cnt) {
-    uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-    if (i < n) atomicAdd(&cnt[idx[i]], 1u);
+__global__ void k_word_pop(const uint32_t *__restrict__ bits, uint64_t words, uint32_t *__restrict__ cnt) {
+    uint64_t w = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+    if (w < words) cnt[w] = (uint32_t)(__popc(bits[2 * w]) + __popc(bits[2 * w + 1]));
 }
 
-__global__ void k_rank_table(const uint32_t *__restrict__ rowsByCount, uint32_t nhot,
-                             uint32_t *__restrict__ rank) {
-    uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < nhot) rank[rowsByCount[r]] = kHotBit | r;
-}
-
-__global__ void k_encode(const uint32_t *__restrict__ idx, const uint32_t *__restrict__ rank, uint64_t n,
-                         uint32_t *__restrict__ enc) {
-    uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t v = idx[i];
-    uint32_t r = rank[v];
-    enc[i] = r != 0xffffffffu ? r : v;
+// coordinate of level `lvl` (an index level) of every stored nonzero
+__global__ void k_level_coord(int N, int lvl, uint32_t fibers, const uint32_t *__restrict__ fbit,
+                              const uint32_t *__restrict__ frank,
+                              const uint32_t *__restrict__ sbit, const uint32_t *__restrict__ jrank,
+                              const uint32_t *__restrict__ idx, uint32_t entries, uint64_t n,
+                              uint32_t *__restrict__ key, uint32_t *__restrict__ pos) {
+    uint64_t x = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+    if (x >= n) return;
+    pos[x] = (uint32_t)x;
+    if (!idx) return;
+    // (a loaded file's bits are not to be trusted with an index)
+    uint32_t e = min(dev::rank_of(fbit, frank, (uint32_t)x), fibers - 1);
+    if (N == 4 && lvl == 1) e = dev::rank_of(sbit, jrank, e);
+    key[x] = idx[min(e, entries - 1)];
 }
 
 }  // namespace
 
-void build_hot_table(const Csf &c, int level, uint64_t rows, HotTable &h, hipStream_t s) {
-    const uint32_t *idx = level == c.ndims - 1 ? c.leaf.p : c.idx[level].p;
-    const uint64_t n = level == c.ndims - 1 ? c.nnz : c.cnt[level];
+void build_level_maps(Csf &c, hipStream_t s) {
+    const int N = c.ndims;
+    const uint64_t n = c.nnz, nL = c.cnt[N - 2];
+    if (n == 0) return;
     Temp tmp;
-    h.count = 0;
-    h.tgt.alloc(n);
-    if (n == 0 || rows == 0) return;
-    TmpArray<uint32_t> cnt(rows), cnt2(rows), ids(rows), ids2(rows), rank(rows);
-    MMCSF_HIP(hipMemsetAsync(cnt.p, 0, rows * 4, s));
-    hipLaunchKernelGGL(k_hist, dim3(nblk(n)), dim3(kBS), 0, s, idx, n, cnt.p);
-    hipLaunchKernelGGL(k_iota, dim3(nblk(rows)), dim3(kBS), 0, s, ids.p, rows);
-    size_t bytes = 0;
-    MMCSF_HIP(rocprim::radix_sort_pairs_desc(nullptr, bytes, cnt.p, cnt2.p, ids.p, ids2.p, (size_t)rows, 0u,
-                                             32u, s));
-    MMCSF_HIP(rocprim::radix_sort_pairs_desc(tmp.get(bytes), bytes, cnt.p, cnt2.p, ids.p, ids2.p,
-                                             (size_t)rows, 0u, 32u, s));
-    // rows with at least one use, capped at kMaxHot
-    std::vector<uint32_t> top(std::min<uint64_t>(rows, kMaxHot));
-    MMCSF_HIP(hipMemcpyAsync(top.data(), cnt2.p, top.size() * 4, hipMemcpyDeviceToHost, s));
-    MMCSF_HIP(hipStreamSynchronize(s));
-    uint32_t nhot = 0;
-    while (nhot < top.size() && top[nhot] > 0) ++nhot;
-    h.count = nhot;
-    h.rows.alloc(std::max<uint32_t>(nhot, 1));
-    if (nhot) MMCSF_HIP(hipMemcpyAsync(h.rows.p, ids2.p, nhot * 4, hipMemcpyDeviceToDevice, s));
-    MMCSF_HIP(hipMemsetAsync(rank.p, 0xff, rows * 4, s));
-    if (nhot) hipLaunchKernelGGL(k_rank_table, dim3((nhot + 255) / 256), dim3(256), 0, s, ids2.p, nhot, rank.p);
-    hipLaunchKernelGGL(k_encode, dim3(nblk(n)), dim3(kBS), 0, s, idx, rank.p, n, h.tgt.p);
-    MMCSF_HIP(hipStreamSynchronize(s));
+    auto ranks = [&](const DevArray<uint32_t> &bits, uint64_t items, DevArray<uint32_t> &rank) {
+        const uint64_t words = (items + 63) / 64;
+        rank.alloc(words);
+        TmpArray<uint32_t> cnt(words);
+        hipLaunchKernelGGL(k_word_pop, dim3(nblk(words)), dim3(kBS), 0, s, bits.p, words, cnt.p);
+        exclusive_sum(cnt.p, rank.p, words, s, tmp);
+    };
+    ranks(c.fbit, n, c.frank);
+    if (N == 4) ranks(c.sbit, nL, c.jrank);
+    TmpArray<uint32_t> pos(n), key(n), sorted(n);
+    for (int l = 1; l < N; ++l) {
+        const bool leaf = l == N - 1;
+        hipLaunchKernelGGL(k_level_coord, dim3(nblk(n)), dim3(kBS), 0, s, N, l, (uint32_t)nL, c.fbit.p, c.frank.p,
+                           c.sbit.p, c.jrank.p, leaf ? (const uint32_t *)nullptr : c.idx[l].p,
+                           leaf ? 1u : (uint32_t)c.cnt[l], n, key.p, pos.p);
+        c.map[l].ord.alloc(n);
+        const uint32_t *k = leaf ? c.leaf.p : key.p;
+        const unsigned bits = (unsigned)bitwidth(c.rows[l] ? c.rows[l] - 1 : 0);
+        size_t bytes = 0;
+        MMCSF_HIP(rocprim::radix_sort_pairs(nullptr, bytes, k, sorted.p, pos.p, c.map[l].ord.p, (size_t)n, 0u, bits, s));
+        MMCSF_HIP(rocprim::radix_sort_pairs(tmp.get(bytes), bytes, k, sorted.p, pos.p, c.map[l].ord.p, (size_t)n, 0u,
+                                            bits, s));
+        build_row_cost(sorted.p, n, c.rows[l], c.map[l].cost, s);
+    }
 }
 
 namespace {

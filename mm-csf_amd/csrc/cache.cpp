@@ -1,12 +1,15 @@
 // Binary cache of built formats: every array of every tree of a format
 // (pointer / index / value arrays, positions, start bitmasks, chunk cost
-// prefix, bins, hot-row tables, the per-mode root trees and the mixed-mode
+// prefix, bins, the per-mode root trees and the mixed-mode
 // partitions) with its sizes, so a reload skips reading, sorting and building.
 //
 // File layout (little-endian): the 8-byte magic "MMCSFFMT", a uint32 version
 // (kVersion) and a uint32 byte-order mark 0x01020304, then the format's
 // fields in a fixed order (scalars as their bytes, each array as a uint64
 // element count and its elements), then the 8-byte end mark "MMCSFEND".
+// Version 2 notes which levels of a tree have a level map, and a load derives
+// the maps again; version 1 stored ranked-row tables of those levels instead,
+// which a load reads past.
 // Loading checks the magic, version, byte order, every count against the
 // remaining file size and the end mark.
 #include <algorithm>
@@ -23,7 +26,7 @@ namespace {
 
 constexpr char kMagic[8] = {'M', 'M', 'C', 'S', 'F', 'F', 'M', 'T'};
 constexpr char kEnd[8] = {'M', 'M', 'C', 'S', 'F', 'E', 'N', 'D'};
-constexpr uint32_t kVersion = 1;
+constexpr uint32_t kVersion = 2, kOldestVersion = 1;
 constexpr uint32_t kByteOrder = 0x01020304u;
 
 // Two pinned host buffers between the file and the device: the file read or
@@ -109,6 +112,11 @@ struct Reader {
     FILE *f;
     uint64_t left;  // bytes not yet read
     Stage &st;
+    uint32_t version = kVersion;
+    void skip(uint64_t n) {
+        MMCSF_REQUIRE(n <= left && std::fseek(f, (long)n, SEEK_CUR) == 0, MMCSF_ERR_IO, "format cache: file is truncated");
+        left -= n;
+    }
     void bytes(void *p, size_t n) {
         MMCSF_REQUIRE(n <= left, MMCSF_ERR_IO, "format cache: file is truncated");
         if (n && std::fread(p, 1, n, f) != n) fail(MMCSF_ERR_IO, "format cache: read failed");
@@ -155,6 +163,7 @@ struct Reader {
 template <typename W, typename C>
 void csf_fields(W &w, C &c) {
     auto &cc = const_cast<Csf &>(c);
+    [[maybe_unused]] bool mapped = false;  // the tree serves every mode
     if constexpr (std::is_same_v<W, Writer>) {
         w.pod(c.ndims);
         w.bytes(c.order, sizeof(c.order));
@@ -164,7 +173,7 @@ void csf_fields(W &w, C &c) {
         w.pod(c.hasBins);
         w.bytes(c.binCount, sizeof(c.binCount));
         w.pod(c.dropped);
-        for (int l = 0; l < kMaxDims; ++l) w.pod(c.hot[l].count);
+        for (int l = 0; l < kMaxDims; ++l) w.template pod<uint32_t>(c.map[l].ord.p ? 1u : 0u);
     } else {
         cc.ndims = w.template pod<int>();
         w.bytes(cc.order, sizeof(cc.order));
@@ -174,7 +183,7 @@ void csf_fields(W &w, C &c) {
         cc.hasBins = w.template pod<bool>();
         w.bytes(cc.binCount, sizeof(cc.binCount));
         cc.dropped = w.template pod<uint64_t>();
-        for (int l = 0; l < kMaxDims; ++l) cc.hot[l].count = w.template pod<uint32_t>();
+        for (int l = 0; l < kMaxDims; ++l) mapped = w.template pod<uint32_t>() != 0 || mapped;
         MMCSF_REQUIRE(cc.ndims == 0 || cc.ndims == 3 || cc.ndims == 4, MMCSF_ERR_IO, "format cache: bad tree");
     }
     for (int l = 0; l < kMaxDims - 1; ++l) {
@@ -189,9 +198,22 @@ void csf_fields(W &w, C &c) {
     w.dev(cc.sbit);
     w.dev(cc.chunkCost);
     w.dev(cc.binList);
-    for (int l = 0; l < kMaxDims; ++l) {
-        w.dev(cc.hot[l].rows);
-        w.dev(cc.hot[l].tgt);
+    if constexpr (std::is_same_v<W, Reader>) {
+        if (w.version == 1)
+            for (int l = 0; l < 2 * kMaxDims; ++l) {  // the rows and targets of each level's table
+                const uint64_t n = w.count(sizeof(uint32_t));
+                w.skip(n * sizeof(uint32_t));
+            }
+        if (mapped) {
+            // every array of the tree is needed and sized as its counts say
+            const int N = cc.ndims;
+            bool ok = N >= 3 && cc.leaf.n >= cc.nnz && cc.fbit.n >= cc.nnz / 32 + 3 && cc.cnt[N - 1] == cc.nnz;
+            for (int l = 1; ok && l < N - 1; ++l) ok = cc.idx[l].n >= cc.cnt[l];
+            if (ok && N == 4) ok = cc.sbit.n >= cc.cnt[2] / 32 + 3;
+            MMCSF_REQUIRE(ok, MMCSF_ERR_IO, "format cache: bad tree");
+            w.st.drain();
+            build_level_maps(cc, w.st.s);
+        }
     }
 }
 
@@ -291,9 +313,10 @@ void format_load(const char *path, Format &f) {
     r.bytes(m, 8);
     MMCSF_REQUIRE(std::memcmp(m, kMagic, 8) == 0, MMCSF_ERR_IO, "not a format cache file");
     const uint32_t version = r.pod<uint32_t>();
-    MMCSF_REQUIRE(version == kVersion, MMCSF_ERR_IO,
-                  "format cache version " + std::to_string(version) + ", this library reads version " +
-                      std::to_string(kVersion));
+    MMCSF_REQUIRE(version >= kOldestVersion && version <= kVersion, MMCSF_ERR_IO,
+                  "format cache version " + std::to_string(version) + ", this library reads versions " +
+                      std::to_string(kOldestVersion) + " to " + std::to_string(kVersion));
+    r.version = version;
     MMCSF_REQUIRE(r.pod<uint32_t>() == kByteOrder, MMCSF_ERR_IO, "format cache written with another byte order");
     format_fields(r, f);
     st.drain();

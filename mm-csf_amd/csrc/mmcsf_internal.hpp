@@ -181,8 +181,6 @@ struct TmpArray : DevArray<T> {
 // ---------------------------------------------------------------------------
 constexpr int kMaxDims = 4;
 constexpr int kNumBins = 10;             // Options::nBin, util.h:205
-constexpr uint32_t kHotBit = 0x80000000u;  // target-array tag of a privatised row
-constexpr uint32_t kMaxHot = 4096;         // ranked rows per scatter level
 
 // COO tensor: class Tensor (util.h:80-108) without the derived members.
 struct Tensor {
@@ -193,11 +191,13 @@ struct Tensor {
     DevArray<float> vals;
 };
 
-// Top-k rows of a scatter output, privatised in LDS by the scatter kernels.
-struct HotTable {
-    uint32_t count = 0;                  // ranked rows (<= kMaxHot)
-    DevArray<uint32_t> rows;             // rank -> row
-    DevArray<uint32_t> tgt;              // per contribution: row, or kHotBit|rank
+// A tree's nonzeros in the order of one level's coordinates (ties in stored
+// order), so that the MTTKRP of that level's mode sums each output row in one
+// place instead of scattering to it.  Derived from the tree; not stored in
+// format caches.
+struct LevelMap {
+    DevArray<uint32_t> ord;              // stored positions
+    DevArray<uint32_t> cost;             // cost prefix over 64-nonzero chunks of that order
 };
 
 // One compressed-sparse-fiber tree with N-1 index levels (TiledTensor,
@@ -225,8 +225,10 @@ struct Csf {
     DevArray<uint32_t> binList;          // concatenated slcMapperBin[0..9]
     uint64_t binCount[kNumBins] = {0};
     uint64_t dropped = 0;
-    // privatisation tables for the scatter roles, indexed by output level
-    HotTable hot[kMaxDims];               // built for levels 1..N-1 of MM-CSF
+    // orders of the levels below the root, of trees that serve every mode
+    LevelMap map[kMaxDims];
+    DevArray<uint32_t> frank;             // with maps: leaf fibers before each 64-bit word of fbit
+    DevArray<uint32_t> jrank;             // 4-D, with maps: level-1 entries before each word of sbit
 };
 
 // HB-CSF parts (HYBTensor, util.h:141-173)
@@ -303,7 +305,8 @@ void build_bins_tiled(Csf &c, hipStream_t s);           // make_TiledBin
 void build_hyb(int ndims, const uint64_t *dims, Csf &&src, Hyb &out, hipStream_t s);
 // the CSL part of a built 3-D HB-CSF as a walkable tree (h.cslWalk)
 void build_csl_walk(Hyb &h, hipStream_t s);
-void build_hot_table(const Csf &c, int level, uint64_t rows, HotTable &h, hipStream_t s);
+// the orders of every level below the root (c.map, c.frank, c.jrank)
+void build_level_maps(Csf &c, hipStream_t s);
 // hot[m] = the rows of tensor mode m holding `frac` of the nonzeros, most used first
 void hot_footprints(const Tensor &t, double frac, uint64_t *hot, hipStream_t s);
 // mixed-mode partition: level-1 entry of every nonzero of an unsplit CSF (at
@@ -342,6 +345,9 @@ void mttkrp_mode(const Format &f, int mode, const Factors &F, float *out, hipStr
 // of four for bfloat16 rows) and the start bitmasks of the tree
 bool walk_supports(const Csf &c, int R, int dtype);
 void mttkrp_root(const Csf &c, const Factors &F, float *out, hipStream_t s, bool accumulate = false);
+// the MTTKRP of the mode at level outLevel > 0 of a tree with level maps
+bool map_walk_supports(const Csf &c, const Factors &F, int outLevel, const float *out);
+void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, hipStream_t s, bool accumulate);
 // the walk's row loads are 16 bytes wide (8 for bfloat16 with R % 8 != 0):
 // factor tables of every level but skipLevel, and `out`, must be aligned to that
 void check_walk_align(const Csf &c, const Factors &F, int skipLevel, const float *out);
@@ -349,7 +355,7 @@ void mttkrp_hyb(const Hyb &h, const uint64_t *dims, const Factors &F, float *out
 // loads the code objects of the MTTKRP kernels (and, cp, of the CP
 // completion passes) on the current device, once per process
 void preload_kernels(bool cp);
-void preload_scatter_kernels();
+void preload_group_kernels();
 void fill_zero(float *p, uint64_t n, hipStream_t s);
 
 // TTM (walk.hip): Y[leaf fiber] = sum over its nonzeros of v * U_leaf[leaf]

@@ -27,203 +27,154 @@ using dev::upper_index;
 constexpr int kBlock = 256;
 
 // --------------------------------------------------------------------------
-// CSF walker: N = 3 or 4 levels of coordinates, OUT = level of the output mode.
-// Persistent: every group of G lanes owns one contiguous, equal share of the
-// nonzeros.  Scatter roles (OUT > 0) accumulate the top-ranked output rows in
-// LDS and flush them once per block; other rows take global atomics.
+// Root-mode CSF walker for what the chunked walk does not serve (R < 4, tables
+// of 4 GiB and more).  Persistent: every group of G lanes owns one contiguous,
+// equal share of the nonzeros.
 // --------------------------------------------------------------------------
-constexpr int kMaxBlock = 1024;
-
-template <int N, int OUT, int G, int NV, int VEC, int B, typename T>
-__global__ __launch_bounds__(kMaxBlock) void k_csf(CsfArgs a) {
-    extern __shared__ float lds[];
+template <int N, int G, int NV, int VEC, int B, typename T>
+__global__ __launch_bounds__(kBlock) void k_csf(CsfArgs a) {
     using RowT = Row<G, NV, VEC>;
     constexpr int LF = N - 2;  // leaf-fiber level
-    constexpr bool SCATTER = OUT > 0;
     const int R = a.R;
-    const uint32_t nH = SCATTER ? a.nHot : 0u;
-    const uint32_t stride = a.ldsStride;
-    if constexpr (SCATTER) {
-        for (uint32_t i = threadIdx.x; i < nH * stride; i += blockDim.x) lds[i] = 0.f;
-        __syncthreads();
-    }
     const int lane = threadIdx.x % G;
     const uint64_t ngroups = (uint64_t)gridDim.x * blockDim.x / G;
     const uint64_t grp = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / G;
     const uint32_t x0 = (uint32_t)(grp * a.nnz / ngroups);
     const uint32_t x1 = (uint32_t)((grp + 1) * a.nnz / ngroups);
-    float *__restrict__ out = a.out;
+    if (x0 >= x1) return;
+    const T *U1 = static_cast<const T *>(a.U[1]);
+    const T *U2 = static_cast<const T *>(a.U[2]);
+    const T *UL = static_cast<const T *>(a.U[N - 1]);
+    const uint32_t *__restrict__ ptrL = a.ptr[LF];
 
-    // out[target] += v, through LDS for ranked rows
-    auto scatter = [&](uint32_t tgt, const RowT &v) {
-        if (tgt & kHotBit) {
-            uint32_t r = tgt & ~kHotBit;
-            if (r < nH) {
-                v.lds_add(lds + (size_t)r * stride, R, lane);
-                return;
-            }
-            tgt = a.hotRows[r];
+    uint32_t f = upper_index(ptrL, a.cnt[LF], x0);
+    uint32_t fend = ptrL[f + 1];
+    uint32_t j = f, jend = 0;
+    if constexpr (N == 4) {
+        j = upper_index(a.ptr[1], a.cnt[1], f);
+        jend = a.ptr[1][j + 1];
+    }
+    uint32_t slc = a.slc[j];
+
+    RowT aF, aJ, aS, t;
+    aF.zero();
+    aJ.zero();
+    aS.zero();
+    auto end_fiber = [&]() {
+        if constexpr (N == 3) {
+            t.load(U1, a.idx[1][f], R, lane);
+            aS.fma_had(aF, t);
+        } else {
+            t.load(U2, a.idx[2][f], R, lane);
+            aJ.fma_had(aF, t);
         }
-        v.atomic_add(out, tgt, R, lane);
-    };
-
-    if (x0 < x1) {
-        const T *U0 = static_cast<const T *>(a.U[0]);
-        const T *U1 = static_cast<const T *>(a.U[1]);
-        const T *U2 = static_cast<const T *>(a.U[2]);
-        const T *UL = static_cast<const T *>(a.U[N - 1]);
-        const uint32_t *__restrict__ ptrL = a.ptr[LF];
-        const uint32_t *__restrict__ leaf = (OUT == N - 1) ? a.tgt : a.leaf;
-        const uint32_t *__restrict__ tgtF = a.tgt;
-        const float *__restrict__ val = a.val;
-
-        uint32_t f = upper_index(ptrL, a.cnt[LF], x0);
-        uint32_t fend = ptrL[f + 1];
-        uint32_t j = f, jend = 0;
-        if constexpr (N == 4) {
-            j = upper_index(a.ptr[1], a.cnt[1], f);
-            jend = a.ptr[1][j + 1];
-        }
-        uint32_t slc = a.slc[j];
-
-        RowT aF, aJ, aS, PS, PJ, P, t;
         aF.zero();
-        aJ.zero();
+    };
+    auto end_j = [&]() {
+        if constexpr (N == 4) {
+            t.load(U1, a.idx[1][j], R, lane);
+            aS.fma_had(aJ, t);
+            aJ.zero();
+        }
+    };
+    auto next_slice = [&](uint32_t ns) {
+        if (ns == slc) return;
+        aS.atomic_add(a.out, slc, R, lane);
         aS.zero();
-        PS.zero();
-        PJ.zero();
-        P.zero();
-
-        auto begin_slice = [&]() {
-            if constexpr (OUT >= 1) PS.load(U0, slc, R, lane);
-        };
-        auto begin_j = [&]() {  // 4-D: product of slice and fbrS rows
-            if constexpr (N == 4 && OUT >= 2) {
-                t.load(U1, a.idx[1][j], R, lane);
-                PJ.had(PS, t);
-            }
-        };
-        auto begin_fiber = [&]() {
-            if constexpr (OUT == N - 1) {
-                if constexpr (N == 3) {
-                    t.load(U1, a.idx[1][f], R, lane);
-                    P.had(PS, t);
-                } else {
-                    t.load(U2, a.idx[2][f], R, lane);
-                    P.had(PJ, t);
-                }
-            }
-        };
-        auto end_fiber = [&]() {
-            if constexpr (N == 3 && OUT == 0) {
-                t.load(U1, a.idx[1][f], R, lane);
-                aS.fma_had(aF, t);
-            } else if constexpr (N == 3 && OUT == 1) {
-                aF.mul(PS);
-                scatter(tgtF[f], aF);
-            } else if constexpr (N == 4 && (OUT == 0 || OUT == 1)) {
-                t.load(U2, a.idx[2][f], R, lane);
-                aJ.fma_had(aF, t);
-            } else if constexpr (N == 4 && OUT == 2) {
-                aF.mul(PJ);
-                scatter(tgtF[f], aF);
-            }
-            aF.zero();
-        };
-        auto end_j = [&]() {
-            if constexpr (N == 4 && OUT == 0) {
-                t.load(U1, a.idx[1][j], R, lane);
-                aS.fma_had(aJ, t);
-                aJ.zero();
-            } else if constexpr (N == 4 && OUT == 1) {
-                aJ.mul(PS);
-                scatter(tgtF[j], aJ);
-                aJ.zero();
-            }
-        };
-        auto end_slice = [&]() {
-            if constexpr (OUT == 0) {
-                aS.atomic_add(out, slc, R, lane);
-                aS.zero();
-            }
-        };
-
-        begin_slice();
-        begin_j();
-        begin_fiber();
-        for (uint32_t xb = x0; xb < x1; xb += B) {
-            uint32_t li[B];
-            float vv[B];
-            RowT rows[B];
+        slc = ns;
+    };
+    for (uint32_t xb = x0; xb < x1; xb += B) {
+        float vv[B];
+        RowT rows[B];
 #pragma unroll
-            for (int k = 0; k < B; ++k) {
-                uint32_t x = xb + k;
-                li[k] = 0;
-                vv[k] = 0.f;
-                if (x < x1) {
-                    li[k] = leaf[x];
-                    vv[k] = val[x];
-                }
+        for (int k = 0; k < B; ++k) {
+            const uint32_t x = xb + k;
+            vv[k] = 0.f;
+            if (x < x1) {
+                vv[k] = a.val[x];
+                rows[k].load(UL, a.leaf[x], R, lane);
             }
-            if constexpr (OUT != N - 1) {
+        }
 #pragma unroll
-                for (int k = 0; k < B; ++k)
-                    if (xb + k < x1) rows[k].load(UL, li[k], R, lane);
-            }
-#pragma unroll
-            for (int k = 0; k < B; ++k) {
-                uint32_t x = xb + k;
-                if (x >= x1) break;
-                if (x == fend) {
-                    end_fiber();
-                    ++f;
-                    fend = ptrL[f + 1];
-                    if constexpr (N == 4) {
-                        if (f == jend) {
-                            end_j();
-                            ++j;
-                            jend = a.ptr[1][j + 1];
-                            uint32_t ns = a.slc[j];
-                            if (ns != slc) {
-                                end_slice();
-                                slc = ns;
-                                begin_slice();
-                            }
-                            begin_j();
-                        }
-                    } else {
-                        uint32_t ns = a.slc[f];
-                        if (ns != slc) {
-                            end_slice();
-                            slc = ns;
-                            begin_slice();
-                        }
+        for (int k = 0; k < B; ++k) {
+            const uint32_t x = xb + k;
+            if (x >= x1) break;
+            if (x == fend) {
+                end_fiber();
+                ++f;
+                fend = ptrL[f + 1];
+                if constexpr (N == 4) {
+                    if (f == jend) {
+                        end_j();
+                        ++j;
+                        jend = a.ptr[1][j + 1];
+                        next_slice(a.slc[j]);
                     }
-                    begin_fiber();
-                }
-                if constexpr (OUT == N - 1) {
-                    RowT c;
-                    c.zero();
-                    c.fma(vv[k], P);
-                    scatter(li[k], c);
                 } else {
-                    aF.fma(vv[k], rows[k]);
+                    next_slice(a.slc[f]);
                 }
             }
+            aF.fma(vv[k], rows[k]);
         }
-        end_fiber();
-        end_j();
-        end_slice();
     }
+    end_fiber();
+    end_j();
+    aS.atomic_add(a.out, slc, R, lane);
+}
 
-    if constexpr (SCATTER) {
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < nH * (uint32_t)R; i += blockDim.x) {
-            uint32_t r = i / (uint32_t)R, c = i - r * (uint32_t)R;
-            float v = lds[(size_t)r * stride + c];
-            if (v != 0.f) unsafeAtomicAdd(out + (size_t)a.hotRows[r] * R + c, v);
+// --------------------------------------------------------------------------
+// Level-map MTTKRP for what the mapped walk does not serve (R < 4, tables of
+// 4 GiB and more, bfloat16 rows at 8-byte boundaries): every group sums a
+// contiguous run of the nonzeros in the order of the output level.
+// --------------------------------------------------------------------------
+struct MapArgs {
+    const uint32_t *ord, *fbit, *frank, *sbit, *jrank;
+    const uint32_t *slc, *idx1, *idx2, *leaf;
+    const float *val;
+    const void *U[4];  // per level; U[outLevel] is not read
+    float *out;
+    uint32_t nnz, perGroup;
+    int R, outLevel;
+};
+
+template <int N, int G, int NV, int VEC, int B, typename T>
+__global__ __launch_bounds__(kBlock) void k_map(MapArgs a) {
+    using RowT = Row<G, NV, VEC>;
+    const int lane = threadIdx.x % G;
+    const uint64_t grp = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / G;
+    const uint64_t x0 = grp * (uint64_t)a.perGroup;
+    if (x0 >= a.nnz) return;
+    const uint32_t x1 = (uint32_t)min((uint64_t)a.nnz, x0 + a.perGroup);
+    uint32_t cur = 0xffffffffu;
+    RowT acc;
+    acc.zero();
+    for (uint32_t q = (uint32_t)x0; q < x1; ++q) {
+        const uint32_t x = a.ord[q];
+        const uint32_t f = dev::rank_of(a.fbit, a.frank, x);
+        const uint32_t j = N == 4 ? dev::rank_of(a.sbit, a.jrank, f) : f;
+        const uint32_t c[4] = {a.slc[j], a.idx1[j], N == 4 ? a.idx2[f] : a.leaf[x], N == 4 ? a.leaf[x] : 0u};
+        uint32_t row = 0;
+        RowT p, t;
+        bool first = true;
+#pragma unroll
+        for (int l = 0; l < N; ++l) {
+            if (l == a.outLevel) {
+                row = c[l];
+                continue;
+            }
+            t.load(static_cast<const T *>(a.U[l]), c[l], a.R, lane);
+            if (first) p = t;
+            else p.mul(t);
+            first = false;
         }
+        if (row != cur) {
+            if (cur != 0xffffffffu) acc.atomic_add(a.out, cur, a.R, lane);
+            acc.zero();
+            cur = row;
+        }
+        acc.fma(a.val[x], p);
     }
+    acc.atomic_add(a.out, cur, a.R, lane);
 }
 
 // --------------------------------------------------------------------------
@@ -419,42 +370,44 @@ struct CslK {
     }
 };
 
-template <int N, int OUT>
+template <int N>
 struct CsfLaunch {
     template <int G, int NV, int VEC, int B, typename T>
     struct K {
         static void launch(dim3, dim3, hipStream_t s, const CsfArgs &a) {
-            auto fn = k_csf<N, OUT, G, NV, VEC, B, T>;
-            const size_t lds = (size_t)a.nHot * a.ldsStride * sizeof(float);
-            const int block = OUT > 0 ? kMaxBlock : 256;
-            if (lds > 65536) MMCSF_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            auto fn = k_csf<N, G, NV, VEC, B, T>;
             int perCU = 0;
-            MMCSF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fn, block, lds));
-            perCU = std::max(perCU, 1);
-            dim3 grid((unsigned)(device_cu_count() * perCU));
-            fn<<<grid, dim3(block), lds, s>>>(a);
+            MMCSF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fn, kBlock, 0));
+            fn<<<dim3((unsigned)(device_cu_count() * std::max(perCU, 1))), dim3(kBlock), 0, s>>>(a);
         }
     };
 };
 
-template <int N, int OUT>
+template <int N>
+struct MapLaunch {
+    template <int G, int NV, int VEC, int B, typename T>
+    struct K {
+        static void launch(dim3 g, dim3 b, hipStream_t s, const MapArgs &a) {
+            k_map<N, G, NV, VEC, B, T><<<g, b, 0, s>>>(a);
+        }
+    };
+};
+
+template <int N>
 void launch_csf_t(const Geo &g, CsfArgs &a, int dtype, hipStream_t s) {
     if (dtype == MMCSF_F32)
-        run_geo<CsfLaunch<N, OUT>::template K, CsfArgs, float>(g, a, 1, s);
+        run_geo<CsfLaunch<N>::template K, CsfArgs, float>(g, a, 1, s);
     else
-        run_geo<CsfLaunch<N, OUT>::template K, CsfArgs, uint16_t>(g, a, 1, s);
+        run_geo<CsfLaunch<N>::template K, CsfArgs, uint16_t>(g, a, 1, s);
 }
 
-int max_lds_per_block() {
-    static int bytes = 0;
-    if (!bytes) {
-        int dev = 0;
-        MMCSF_HIP(hipGetDevice(&dev));
-        MMCSF_HIP(hipDeviceGetAttribute(&bytes, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-        if (bytes <= 0) bytes = 65536;
-    }
-    return bytes;
+template <int N>
+void launch_map_t(const Geo &g, MapArgs &a, int dtype, hipStream_t s) {
+    const uint64_t groups = (a.nnz + a.perGroup - 1) / a.perGroup;
+    if (dtype == MMCSF_F32)
+        run_geo<MapLaunch<N>::template K, MapArgs, float>(g, a, groups, s);
+    else
+        run_geo<MapLaunch<N>::template K, MapArgs, uint16_t>(g, a, groups, s);
 }
 
 void check_align(const void *p, int dtype, const Geo &g) {
@@ -465,7 +418,7 @@ void check_align(const void *p, int dtype, const Geo &g) {
 
 }  // namespace
 
-void preload_scatter_kernels() {
+void preload_group_kernels() {
     // one kernel of this translation unit: its code object loads with it
     hipFuncAttributes attr;
     MMCSF_HIP(hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(k_zero)));
@@ -489,6 +442,25 @@ void fill_zero(float *p, uint64_t n, hipStream_t s) {
     MMCSF_HIP(hipGetLastError());
 }
 
+static void launch_csf(const Csf &c, const Geo &g, const Factors &F, float *out, hipStream_t s) {
+    CsfArgs a{};
+    for (int l = 0; l < c.ndims - 1; ++l) {
+        a.ptr[l] = c.ptr[l].p;
+        a.idx[l] = c.idx[l].p;
+        a.cnt[l] = (uint32_t)c.cnt[l];
+    }
+    a.cnt[c.ndims - 1] = (uint32_t)c.nnz;
+    a.slc = c.fbrSlc.p;
+    a.leaf = c.leaf.p;
+    a.val = c.vals.p;
+    for (int l = 0; l < c.ndims; ++l) a.U[l] = F.U[c.order[l]];
+    a.out = out;
+    a.nnz = (uint32_t)c.nnz;
+    a.R = F.R;
+    if (c.ndims == 3) launch_csf_t<3>(g, a, F.dtype, s);
+    else launch_csf_t<4>(g, a, F.dtype, s);
+}
+
 void mttkrp_csf(const Csf &c, const uint64_t *dims, int outLevel, const Factors &F, float *out,
                 hipStream_t s, hipEvent_t evStart, hipEvent_t evEnd, bool accumulate, bool zeroed) {
     const int N = c.ndims;
@@ -504,55 +476,44 @@ void mttkrp_csf(const Csf &c, const uint64_t *dims, int outLevel, const Factors 
     if (c.nnz == 0) return;
     Geo g = pick_geometry(F.R, F.dtype);
     check_align(out, MMCSF_F32, g);
-    CsfArgs a{};
-    for (int l = 0; l < N - 1; ++l) {
-        a.ptr[l] = c.ptr[l].p;
-        a.idx[l] = c.idx[l].p;
-        a.cnt[l] = (uint32_t)c.cnt[l];
-    }
-    a.cnt[N - 1] = (uint32_t)c.nnz;
-    a.slc = c.fbrSlc.p;
-    a.leaf = c.leaf.p;
-    a.val = c.vals.p;
-    for (int l = 0; l < N; ++l) {
-        a.U[l] = F.U[c.order[l]];
+    for (int l = 0; l < N; ++l)
         if (l != outLevel) {
-            MMCSF_REQUIRE(a.U[l] != nullptr, MMCSF_ERR_ARG, "missing factor matrix");
-            check_align(a.U[l], F.dtype, g);
+            MMCSF_REQUIRE(F.U[c.order[l]] != nullptr, MMCSF_ERR_ARG, "missing factor matrix");
+            check_align(F.U[c.order[l]], F.dtype, g);
         }
+    if (outLevel > 0) {
+        const LevelMap &map = c.map[outLevel];
+        MMCSF_REQUIRE(map.ord.p != nullptr, MMCSF_ERR_ARG, "this format serves its root mode only");
+        if (map_walk_supports(c, F, outLevel, out)) {
+            mttkrp_map_walk(c, outLevel, F, out, s, accumulate);
+            return;
+        }
+        MapArgs a{};
+        a.ord = map.ord.p;
+        a.fbit = c.fbit.p;
+        a.frank = c.frank.p;
+        a.sbit = c.sbit.p;
+        a.jrank = c.jrank.p;
+        a.slc = c.fbrSlc.p;
+        a.idx1 = c.idx[1].p;
+        a.idx2 = c.idx[2].p;
+        a.leaf = c.leaf.p;
+        a.val = c.vals.p;
+        for (int l = 0; l < N; ++l) a.U[l] = F.U[c.order[l]];
+        a.out = out;
+        a.nnz = (uint32_t)c.nnz;
+        a.perGroup = per_group_for(c.nnz, g.G);
+        a.R = F.R;
+        a.outLevel = outLevel;
+        if (N == 3) launch_map_t<3>(g, a, F.dtype, s);
+        else launch_map_t<4>(g, a, F.dtype, s);
+        return;
     }
-    a.out = out;
-    a.nnz = (uint32_t)c.nnz;
-    a.R = F.R;
-    a.perGroup = per_group_for(c.nnz, g.G);
-    if (outLevel == 0 && walk_supports(c, F.R, F.dtype)) {
+    if (walk_supports(c, F.R, F.dtype)) {
         mttkrp_root(c, F, out, s, accumulate);  // checks the alignment its row loads need
         return;
     }
-    if (outLevel > 0) {
-        const HotTable &h = c.hot[outLevel];
-        MMCSF_REQUIRE(h.tgt.p != nullptr || c.nnz == 0, MMCSF_ERR_ARG,
-                      "this format serves its root mode only");
-        a.tgt = h.tgt.p;
-        a.hotRows = h.rows.p;
-        a.ldsStride = (uint32_t)F.R + 1;
-        const uint64_t cap = (uint64_t)(max_lds_per_block() - 1024) / (a.ldsStride * sizeof(float));
-        a.nHot = (uint32_t)std::min<uint64_t>(h.count, cap);
-    }
-    if (N == 3) {
-        switch (outLevel) {
-            case 0: launch_csf_t<3, 0>(g, a, F.dtype, s); break;
-            case 1: launch_csf_t<3, 1>(g, a, F.dtype, s); break;
-            default: launch_csf_t<3, 2>(g, a, F.dtype, s); break;
-        }
-    } else {
-        switch (outLevel) {
-            case 0: launch_csf_t<4, 0>(g, a, F.dtype, s); break;
-            case 1: launch_csf_t<4, 1>(g, a, F.dtype, s); break;
-            case 2: launch_csf_t<4, 2>(g, a, F.dtype, s); break;
-            default: launch_csf_t<4, 3>(g, a, F.dtype, s); break;
-        }
-    }
+    launch_csf(c, g, F, out, s);
 }
 
 void mttkrp_mode(const Format &f, int mode, const Factors &F, float *out, hipStream_t s, hipEvent_t evStart,
@@ -677,25 +638,8 @@ void mttkrp_hyb(const Hyb &h, const uint64_t *dims, const Factors &F, float *out
     // CSF part: root-mode walker (accumulates on top of the other parts' rows,
     // which are disjoint from its slices)
     if (h.csf.nnz) {
-        const Csf &c = h.csf;
-        CsfArgs a{};
-        for (int l = 0; l < N - 1; ++l) {
-            a.ptr[l] = c.ptr[l].p;
-            a.idx[l] = c.idx[l].p;
-            a.cnt[l] = (uint32_t)c.cnt[l];
-        }
-        a.cnt[N - 1] = (uint32_t)c.nnz;
-        a.slc = c.fbrSlc.p;
-        a.leaf = c.leaf.p;
-        a.val = c.vals.p;
-        for (int l = 0; l < N; ++l) a.U[l] = F.U[c.order[l]];
-        a.out = out;
-        a.nnz = (uint32_t)c.nnz;
-        a.R = F.R;
-        a.perGroup = per_group_for(c.nnz, g.G);
-        if (walk_supports(c, F.R, F.dtype)) mttkrp_root(c, F, out, s);
-        else if (N == 3) launch_csf_t<3, 0>(g, a, F.dtype, s);
-        else launch_csf_t<4, 0>(g, a, F.dtype, s);
+        if (walk_supports(h.csf, F.R, F.dtype)) mttkrp_root(h.csf, F, out, s);
+        else launch_csf(h.csf, g, F, out, s);
     }
 }
 

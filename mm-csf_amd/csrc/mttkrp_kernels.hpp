@@ -8,10 +8,8 @@
 // (equal nonzero counts per group, so heavy slices and long fibers are split
 // across groups automatically) and keeps its partial sums in registers:
 //
-//   output level      per nonzero              per leaf fiber / fbrS / slice
-//   root (0)          aF += v * U_leaf[k]     aS += aF (.) U_fbr[j]; flush aS at a slice end
-//   fiber levels      aF += v * U_leaf[k]     flush aF (.) prod(ancestor rows) at the fiber end
-//   leaf (N-1)        out[k] += v * P          P = prod(ancestor rows), once per fiber
+//   aF += v * U_leaf[k] per nonzero, aS += aF (.) U_fbr[j] per leaf fiber,
+//   aS flushed at a slice end
 //
 // Flushes are float atomics (no return) and happen only where a group's range
 // ends or a tree node ends, i.e. atomics appear only across split fibers and
@@ -101,14 +99,6 @@ struct Row {
 #pragma unroll
             for (int b = 0; b < VEC; ++b) v[a][b] *= y.v[a][b];
     }
-    __device__ __forceinline__ bool nonzero() const {
-        bool nz = false;
-#pragma unroll
-        for (int a = 0; a < NV; ++a)
-#pragma unroll
-            for (int b = 0; b < VEC; ++b) nz |= (v[a][b] != 0.f);
-        return nz;
-    }
     // out[row] += this, one no-return float atomic per column
     __device__ __forceinline__ void atomic_add(float *__restrict__ out, uint32_t row, int R,
                                                int lane) const {
@@ -119,17 +109,6 @@ struct Row {
             if (c < R) {
 #pragma unroll
                 for (int b = 0; b < VEC; ++b) unsafeAtomicAdd(base + c + b, v[a][b]);
-            }
-        }
-    }
-    // lds[c] += this[c] for an LDS-resident row (ds_add_f32)
-    __device__ __forceinline__ void lds_add(float *base, int R, int lane) const {
-#pragma unroll
-        for (int a = 0; a < NV; ++a) {
-            int c = (a * G + lane) * VEC;
-            if (c < R) {
-#pragma unroll
-                for (int b = 0; b < VEC; ++b) atomicAdd(base + c + b, v[a][b]);
             }
         }
     }
@@ -161,6 +140,14 @@ __device__ __forceinline__ uint32_t upper_index(const uint32_t *__restrict__ a, 
     return lo;
 }
 
+// the segment that item i falls in, from the segments' start bits and the
+// number of starts before each 64-bit word
+__device__ __forceinline__ uint32_t rank_of(const uint32_t *__restrict__ bits, const uint32_t *__restrict__ rank,
+                                            uint32_t i) {
+    const uint64_t w = reinterpret_cast<const uint64_t *>(bits)[i >> 6];
+    return rank[i >> 6] + (uint32_t)__popcll(w & (~0ull >> (63 - (i & 63)))) - 1u;
+}
+
 }  // namespace dev
 
 // Kernel argument block for one CSF tree.
@@ -174,13 +161,7 @@ struct CsfArgs {
     float *out;
     uint32_t nnz;
     uint32_t cnt[4];
-    uint32_t perGroup;        // nonzeros per row group (non-persistent launches)
     int R;
-    // scatter roles: output-level index with ranked rows tagged kHotBit|rank
-    const uint32_t *tgt;
-    const uint32_t *hotRows;  // rank -> row
-    uint32_t nHot;            // ranks accumulated in LDS by this launch
-    uint32_t ldsStride;       // floats per LDS row
 };
 
 }  // namespace mmcsf

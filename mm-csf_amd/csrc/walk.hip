@@ -129,6 +129,45 @@ void mttkrp_coo_walk(const Format &f, const Factors &F, float *out, hipStream_t 
     walk_launch<kMttkrp, kCoo>(N, F, a, s);
 }
 
+// The modes below the root of a tree that serves every mode.  A tree holds an
+// output row's nonzeros in many places; scattering each partial row there is
+// bound by the additions (float atomics that meet in the L2, or in LDS on the
+// hottest rows: one row of a Zipf(1.2) mode takes ~18 % of them).  A level map
+// lists the nonzeros by output row, so the same walk as from a root sums every
+// row in registers; it finds a nonzero's fiber by the rank of its start bit and
+// reads coordinates and value where the tree holds them (a few 4-byte reads of
+// their own line each; the price of 4 bytes per nonzero and level instead of a
+// tree per mode).  One tree, 20M nonzeros, 500000 x 200000 x 50000, R = 32, the
+// two modes below the root: 7.19 -> 2.59 ms.  Those reads bound it: each lane's
+// is a line of its own past the L2, ~8.6 CU clocks apiece.
+bool map_walk_supports(const Csf &c, const Factors &F, int outLevel, const float *out) {
+    if (!walk_supports(c, F.R, F.dtype)) return false;
+    const uintptr_t need = F.R % 4 != 0 ? 4 : (F.dtype == MMCSF_BF16 && F.R % 8 != 0) ? 8 : 16;
+    for (int l = 0; l < c.ndims; ++l)
+        if (l != outLevel && reinterpret_cast<uintptr_t>(F.U[c.order[l]]) % need != 0) return false;
+    return reinterpret_cast<uintptr_t>(out) % (F.R % 4 != 0 ? 4 : 16) == 0;
+}
+
+void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, hipStream_t s, bool accumulate) {
+    WalkArgs a = args_of(c, F);
+    a.ord = c.map[outLevel].ord.p;
+    a.cost = c.map[outLevel].cost.p;
+    a.frank = c.frank.p;
+    a.jrank = c.jrank.p;
+    a.outLevel = outLevel;
+    // the other levels, in tree order, as the walk's levels 1..N-1
+    const uint64_t es = F.dtype == MMCSF_F32 ? 4 : 2;
+    for (int l = 0, to = 1; l < c.ndims; ++l) {
+        if (l == outLevel) continue;
+        a.U[to] = F.U[c.order[l]];
+        a.tabBytes[to] = (uint32_t)(c.rows[l] * (uint64_t)F.R * es);
+        ++to;
+    }
+    a.out = out;
+    a.accum = accumulate ? 1 : 0;
+    walk_launch<kMttkrp, kMap>(c.ndims, F, a, s);
+}
+
 bool cp_supports(int R) { return R >= 1 && R <= 128 && R % 4 == 0; }
 
 void cp_forward(const Csf &c, const Factors &F, float *resid, double *loss, hipStream_t s) {
@@ -184,7 +223,8 @@ void preload_kernels(bool cp) {
     if (!done[dev][0]) {
         walk_preload<kMttkrp>();
         walk_preload<kMttkrp, kCoo>();
-        preload_scatter_kernels();
+        walk_preload<kMttkrp, kMap>();
+        preload_group_kernels();
         done[dev][0] = true;
     }
     if (cp && !done[dev][1]) {

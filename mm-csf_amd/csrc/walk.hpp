@@ -51,6 +51,10 @@ struct WalkArgs {
     const uint32_t *fbit;  // leaf-fiber starts over nonzeros
     const uint32_t *sbit;  // 4-D: level-1 starts over leaf fibers
     const uint32_t *cost;  // exclusive cost prefix over chunks (chunks + 1 entries)
+    const uint32_t *ord;   // kMap: stored position of every nonzero in walk order
+    const uint32_t *frank; // kMap: leaf fibers starting before each word of fbit
+    const uint32_t *jrank; // kMap, 4-D: level-1 entries starting before each word of sbit
+    int outLevel;          // kMap: the tree level of the output mode
     const uint32_t *pos;   // tensor-order position of every stored nonzero
     const float *wts;      // weights in tensor order
     const void *U[4];      // factor of each level
@@ -70,6 +74,10 @@ enum WalkSrc : int {
     kTree = 0,  // a CSF tree rooted at the output mode
     kCoo = 1,   // sorted COO (MTTKRP only): idx[l] holds level l's coordinate of
                 // every nonzero; every nonzero is a leaf fiber of its own
+    kMap = 2,   // a CSF tree whose output mode sits at level `outLevel` below the
+                // root (MTTKRP only), its nonzeros taken in the order `ord` of
+                // that level's coordinates.  The output row is the walk's slice,
+                // the other levels take its levels 1..N-1 in their tree order.
 };
 
 enum WalkOp : int {

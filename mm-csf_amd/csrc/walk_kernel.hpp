@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "mttkrp_kernels.hpp"
 #include "walk.hpp"
 
 namespace mmcsf {
@@ -237,6 +238,29 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
     const T *UL = static_cast<const T *>(a.U[N - 1]);
     [[maybe_unused]] const __amdgpu_buffer_rsrc_t rs1 = table_rsrc(a.U[1], a.tabBytes[1]);
     [[maybe_unused]] const __amdgpu_buffer_rsrc_t rs2 = table_rsrc(a.U[2], a.tabBytes[2]);
+    // kMap: the coordinates of the nonzero stored at x, from the entries that
+    // hold it: output row, levels 1 (and 2, 4-D) and leaf of the walk
+    [[maybe_unused]] auto mapCoords = [&](uint32_t x, uint32_t &row, uint32_t &c1, uint32_t &c2, uint32_t &cl) {
+        const uint32_t f = dev::rank_of(a.fbit, a.frank, x), lf = a.leaf[x];
+        if constexpr (N == 3) {
+            const uint32_t mid = a.idx[1][f];
+            c1 = a.slc[f];
+            c2 = 0;
+            row = a.outLevel == 1 ? mid : lf;
+            cl = a.outLevel == 1 ? lf : mid;
+        } else {
+            const uint32_t j = dev::rank_of(a.sbit, a.jrank, f), low = a.idx[2][f], mid = a.idx[1][j];
+            c1 = a.slc[j];
+            row = a.outLevel == 1 ? mid : a.outLevel == 2 ? low : lf;
+            c2 = a.outLevel == 1 ? low : mid;
+            cl = a.outLevel == 3 ? low : lf;
+        }
+    };
+    [[maybe_unused]] auto mapRow = [&](uint32_t x) {
+        uint32_t row, c1, c2, cl;
+        mapCoords(x, row, c1, c2, cl);
+        return row;
+    };
     // the open slice (leaf fiber for TTM): its partial row from earlier
     // chunks is the carry `acc`, summed over the groups' shares
     uint32_t scur = kNone;
@@ -289,8 +313,10 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
             jcur = fcur == kNone ? kNone : (a.ptr[1][j0] == f0 && fcur != f0 ? j0 - 1 : j0);
         }
         scur = OP == kTtm ? f0 : a.slc[j0];
-    } else {
+    } else if constexpr (SRC == kCoo) {
         scur = a.idx[0][x0];
+    } else {
+        scur = mapRow(a.ord[x0]);
     }
     // whether the open slice began inside this wave's run: then every
     // contribution to it passes through this wave, and its row is stored
@@ -319,7 +345,8 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
     const uint32_t lastC = chunks - 1;
     auto readWords = [&](uint32_t c, Words &w) {
         const uint32_t x = std::min(c * 64 + (uint32_t)lane, lastX);
-        w.lw = a.leaf[x];
+        // kMap: the stored position, replaced by the leaf index with the entries
+        w.lw = SRC == kMap ? a.ord[x] : a.leaf[x];
         // one 8-byte word per chunk, read through the scalar cache (the chunk
         // index is wave-uniform; chunks past the tensor read the last word)
         w.word = 0;
@@ -331,7 +358,7 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
         w.ps = 0;
         if constexpr (kPos) w.ps = a.pos[x];
         w.v = 0.f;
-        if constexpr (OP != kWeightGrad) w.v = a.val[x];
+        if constexpr (OP != kWeightGrad && SRC != kMap) w.v = a.val[x];
     };
     // level-1 entries of chunk c; fB / jB: the leaf fiber and level-1 entry
     // of the nonzero before chunk c, advanced past it.  Chunks past the run
@@ -345,6 +372,11 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
             q.s = a.idx[0][xc];
             q.i1 = a.idx[1][xc];
             q.i2 = N == 4 ? a.idx[2][xc] : 0u;
+            return;
+        }
+        if constexpr (SRC == kMap) {
+            w.v = a.val[w.lw];
+            mapCoords(w.lw, q.s, q.i1, q.i2, w.lw);
             return;
         }
         const bool start = x < a.nnz && ((w.word >> lane) & 1ull);

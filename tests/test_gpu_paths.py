@@ -174,3 +174,70 @@ def test_coo_walk(cuda, N, rows, nnz):
             for off in (0, 4):
                 got = mmcsf.mttkrp(f, 0, [offset_copy(u, off) for u in Ub])
                 assert rel(got.cpu().numpy(), ref) < 1e-5, (R, off)
+
+
+# ---- modes below the root of a tree that serves every mode ------------------------
+
+ONE_TREE = [(9, {}), (13, {}), (14, {}), (12, {"mode_trees": False}), (12, {"mixed": True})]
+
+
+@pytest.mark.parametrize("dims,skew,nnz", [
+    ([40, 30, 20], [None, None, None], 1),
+    ([40, 30, 20], [None, None, None], 64),
+    ([300, 20, 9], [1.2, None, 1.1], 65),
+    ([500, 400, 60], [1.2, 1.2, None], 20_000),
+    ([3000, 1, 700], [None, None, 1.3], 4097),  # one row takes everything
+    ([30, 25, 20, 15], [None, None, None, None], 129),
+    ([60, 37, 25, 14], [1.1, None, 1.2, None], 12_000),
+])
+@pytest.mark.parametrize("fmt_type,kw", ONE_TREE)
+def test_one_tree_every_mode(cuda, dims, skew, nnz, fmt_type, kw):
+    import torch
+    import mmcsf
+    import oracle as O
+    if kw.get("mixed") and (nnz < 1000 or 1 in dims):
+        pytest.skip("the mixed-mode partition refuses tensors of one slice")
+    rng = np.random.default_rng(nnz + fmt_type)
+    inds, vals = random_tensor(rng, dims, nnz, skew)
+    f = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), fmt_type, mode=0, fbr_threshold=16, **kw)
+    for R in (1, 3, 4, 10, 16, 32, 64, 136):
+        U = [rng.random((d, R)).astype(np.float32) for d in dims]
+        Ud = [torch.from_numpy(u).to(cuda) for u in U]
+        outs, _ = mmcsf.mttkrp_allmode(f, Ud)
+        for m in range(len(dims)):
+            assert rel(outs[m].cpu().numpy(), O.mttkrp_coo_f64(inds, vals, m, U)) < 1e-5, (R, m)
+        if R % 8 == 0:
+            # bfloat16 rows at 16 byte boundaries, and at 8 (per-group kernel; the
+            # root mode's walk refuses those)
+            Ub = [u.to(torch.bfloat16) for u in Ud]
+            Ur = [u.float().cpu().numpy() for u in Ub]
+            root = f.info()["modeOrder"][0]
+            for off in (0, 4):
+                for m in range(len(dims)):
+                    if off and (m == root or kw.get("mixed")):
+                        continue
+                    got = mmcsf.mttkrp(f, m, [offset_copy(u, off) for u in Ub])
+                    assert rel(got.cpu().numpy(), O.mttkrp_coo_f64(inds, vals, m, Ur)) < 1e-5, (R, m, off)
+
+
+@pytest.mark.parametrize("name,dims,fmt_type,kw", [("one_tree_3d", [17, 11, 9], 14, {}),
+                                                   ("single_tree_4d", [9, 7, 6, 5], 12, {"mode_trees": False}),
+                                                   ("mixed_3d", [17, 11, 9], 12, {"mixed": True})])
+def test_version_1_caches_load(cuda, golden_dir, tmp_path, name, dims, fmt_type, kw):
+    """Files of the cache's first version hold ranked-row tables where a format
+    now derives level maps; they load and equal a fresh build."""
+    import torch
+    import mmcsf
+    import oracle as O
+    rng = np.random.default_rng(11)
+    inds, vals = random_tensor(rng, dims, 150, [1.4] + [None] * (len(dims) - 1))
+    f = mmcsf.Format.load(f"{golden_dir}/{name}_v1.fmt")
+    fresh = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), fmt_type, mode=1, fbr_threshold=4, **kw)
+    assert f.info() == fresh.info()
+    f.save(tmp_path / "a.fmt")
+    fresh.save(tmp_path / "b.fmt")
+    assert (tmp_path / "a.fmt").read_bytes() == (tmp_path / "b.fmt").read_bytes()
+    U = [rng.random((d, 12)).astype(np.float32) for d in dims]
+    Ud = [torch.from_numpy(u).to(cuda) for u in U]
+    for m in range(len(dims)):
+        assert rel(mmcsf.mttkrp(f, m, Ud).cpu().numpy(), O.mttkrp_coo_f64(inds, vals, m, U)) < 1e-5
