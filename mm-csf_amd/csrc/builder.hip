@@ -615,6 +615,27 @@ void build_csf(int N, const uint64_t *dims, uint64_t n, const int *order, DevArr
     build_walk_bits(c, s);
 }
 
+__global__ void k_word_pop(const uint32_t *__restrict__ bits, uint64_t words, uint32_t *__restrict__ cnt) {
+    uint64_t w = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+    if (w < words) cnt[w] = (uint32_t)(__popc(bits[2 * w]) + __popc(bits[2 * w + 1]));
+}
+
+void build_walk_ranks(Csf &c, hipStream_t s) {
+    const int N = c.ndims;
+    const uint64_t n = c.nnz, nL = c.cnt[N - 2];
+    if (n == 0) return;
+    Temp tmp;
+    auto ranks = [&](const DevArray<uint32_t> &bits, uint64_t items, DevArray<uint32_t> &rank) {
+        const uint64_t words = (items + 63) / 64;
+        rank.alloc(words);
+        TmpArray<uint32_t> cnt(words);
+        hipLaunchKernelGGL(k_word_pop, dim3(nblk(words)), dim3(kBS), 0, s, bits.p, words, cnt.p);
+        exclusive_sum(cnt.p, rank.p, words, s, tmp);
+    };
+    ranks(c.fbit, n, c.frank);
+    if (N == 4) ranks(c.sbit, nL, c.jrank);
+}
+
 // ---------------------------------------------------------------------------
 // start bitmasks for the chunked root traversal: bit x of fbit = nonzero x
 // starts a leaf fiber; 4-D: bit f of sbit = leaf fiber f starts a level-1
@@ -634,6 +655,7 @@ void build_walk_bits(Csf &c, hipStream_t s) {
     };
     mark(c.fbit, n, c.ptr[N - 2].p, nL);
     if (N == 4) mark(c.sbit, nL, c.ptr[1].p, c.cnt[1]);
+    build_walk_ranks(c, s);
     // cost prefix over chunks: waves split the traversal by cost, not by
     // nonzeros (chunks where many slices start take longer)
     const uint64_t chunks = (n + 63) / 64;
@@ -1034,11 +1056,6 @@ void build_hyb(int N, const uint64_t *dims, Csf &&src, Hyb &h, hipStream_t s) {
 // ---------------------------------------------------------------------------
 namespace {
 
-__global__ void k_word_pop(const uint32_t *__restrict__ bits, uint64_t words, uint32_t *__restrict__ cnt) {
-    uint64_t w = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-    if (w < words) cnt[w] = (uint32_t)(__popc(bits[2 * w]) + __popc(bits[2 * w + 1]));
-}
-
 // coordinate of level `lvl` (an index level) of every stored nonzero
 __global__ void k_level_coord(int N, int lvl, uint32_t fibers, const uint32_t *__restrict__ fbit,
                               const uint32_t *__restrict__ frank,
@@ -1062,15 +1079,6 @@ void build_level_maps(Csf &c, hipStream_t s) {
     const uint64_t n = c.nnz, nL = c.cnt[N - 2];
     if (n == 0) return;
     Temp tmp;
-    auto ranks = [&](const DevArray<uint32_t> &bits, uint64_t items, DevArray<uint32_t> &rank) {
-        const uint64_t words = (items + 63) / 64;
-        rank.alloc(words);
-        TmpArray<uint32_t> cnt(words);
-        hipLaunchKernelGGL(k_word_pop, dim3(nblk(words)), dim3(kBS), 0, s, bits.p, words, cnt.p);
-        exclusive_sum(cnt.p, rank.p, words, s, tmp);
-    };
-    ranks(c.fbit, n, c.frank);
-    if (N == 4) ranks(c.sbit, nL, c.jrank);
     TmpArray<uint32_t> pos(n), key(n), sorted(n);
     for (int l = 1; l < N; ++l) {
         const bool leaf = l == N - 1;

@@ -204,15 +204,17 @@ void csf_fields(W &w, C &c) {
                 const uint64_t n = w.count(sizeof(uint32_t));
                 w.skip(n * sizeof(uint32_t));
             }
-        if (mapped) {
-            // every array of the tree is needed and sized as its counts say
+        if (cc.fbit.p && cc.nnz) {
+            // derived again; every array read for that has to be there and as
+            // long as the counts say
             const int N = cc.ndims;
             bool ok = N >= 3 && cc.leaf.n >= cc.nnz && cc.fbit.n >= cc.nnz / 32 + 3 && cc.cnt[N - 1] == cc.nnz;
-            for (int l = 1; ok && l < N - 1; ++l) ok = cc.idx[l].n >= cc.cnt[l];
+            for (int l = 1; ok && l < N - 1; ++l) ok = cc.idx[l].n >= cc.cnt[l] && cc.cnt[l] > 0;
             if (ok && N == 4) ok = cc.sbit.n >= cc.cnt[2] / 32 + 3;
             MMCSF_REQUIRE(ok, MMCSF_ERR_IO, "format cache: bad tree");
             w.st.drain();
-            build_level_maps(cc, w.st.s);
+            build_walk_ranks(cc, w.st.s);
+            if (mapped) build_level_maps(cc, w.st.s);
         }
     }
 }

@@ -219,6 +219,9 @@ struct Csf {
     DevArray<uint32_t> fbrSlc;           // fbrLikeSlcInds: slice coord per level-1 entry
     DevArray<uint32_t> fbit;             // bit x: nonzero x starts a leaf fiber
     DevArray<uint32_t> sbit;             // 4-D, bit f: leaf fiber f starts a level-1 entry
+    DevArray<uint32_t> frank;            // leaf fibers starting before each 64-bit word of fbit
+    DevArray<uint32_t> jrank;            // 4-D: level-1 entries starting before each word of sbit
+                                         // (both derived; not stored in format caches)
     DevArray<uint32_t> chunkCost;        // exclusive prefix of the cost of 64-nonzero chunks
     // slice bins (make_TiledBin / make_HybBin)
     bool hasBins = false;
@@ -227,8 +230,6 @@ struct Csf {
     uint64_t dropped = 0;
     // orders of the levels below the root, of trees that serve every mode
     LevelMap map[kMaxDims];
-    DevArray<uint32_t> frank;             // with maps: leaf fibers before each 64-bit word of fbit
-    DevArray<uint32_t> jrank;             // 4-D, with maps: level-1 entries before each word of sbit
 };
 
 // HB-CSF parts (HYBTensor, util.h:141-173)
@@ -287,6 +288,8 @@ void order_tensormode(int ndims, const uint64_t *dims, int mode, bool nat, int *
 // keys[l] = coordinate of order[l], and permuted values.
 // start bitmasks of a built tree (called by build_csf and build_hyb)
 void build_walk_bits(Csf &c, hipStream_t s);
+// c.frank and c.jrank from the start bitmasks
+void build_walk_ranks(Csf &c, hipStream_t s);
 // pos (optional) receives the tensor-order position of every sorted nonzero.
 // keepKeys: the caller keeps every key array (else only the last level's, which
 // becomes a tree's leaf array; the others are temporaries).
@@ -305,7 +308,7 @@ void build_bins_tiled(Csf &c, hipStream_t s);           // make_TiledBin
 void build_hyb(int ndims, const uint64_t *dims, Csf &&src, Hyb &out, hipStream_t s);
 // the CSL part of a built 3-D HB-CSF as a walkable tree (h.cslWalk)
 void build_csl_walk(Hyb &h, hipStream_t s);
-// the orders of every level below the root (c.map, c.frank, c.jrank)
+// the orders of every level below the root (c.map)
 void build_level_maps(Csf &c, hipStream_t s);
 // hot[m] = the rows of tensor mode m holding `frac` of the nonzeros, most used first
 void hot_footprints(const Tensor &t, double frac, uint64_t *hot, hipStream_t s);

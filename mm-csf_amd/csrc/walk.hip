@@ -13,7 +13,6 @@ WalkArgs args_of(const Csf &c, const Factors &F) {
     const int N = c.ndims;
     WalkArgs a{};
     for (int l = 0; l < N - 1; ++l) {
-        a.ptr[l] = c.ptr[l].p;
         a.idx[l] = c.idx[l].p;
         a.cnt[l] = (uint32_t)c.cnt[l];
     }
@@ -23,6 +22,8 @@ WalkArgs args_of(const Csf &c, const Factors &F) {
     a.val = c.vals.p;
     a.fbit = c.fbit.p;
     a.sbit = c.sbit.p;
+    a.frank = c.frank.p;
+    a.jrank = c.jrank.p;
     a.cost = c.chunkCost.p;
     a.pos = c.pos.p;
     const uint64_t es = F.dtype == MMCSF_F32 ? 4 : 2;
@@ -79,7 +80,7 @@ void check_walk_align(const Csf &c, const Factors &F, int skipLevel, const float
 // one column a lane in groups of 64, takes 324 us; the whole call 334 -> 53 us.
 bool walk_supports(const Csf &c, int R, int dtype) {
     return R >= 4 && R <= 256 && (R % 4 == 0 || dtype == MMCSF_F32) && tables_fit(c, R) &&
-           (c.nnz == 0 || (c.fbit.p && c.chunkCost.p && (c.ndims == 3 || c.sbit.p)));
+           (c.nnz == 0 || (c.fbit.p && c.frank.p && c.chunkCost.p && (c.ndims == 3 || (c.sbit.p && c.jrank.p))));
 }
 
 void mttkrp_root(const Csf &c, const Factors &F, float *out, hipStream_t s, bool accumulate) {
@@ -152,8 +153,6 @@ void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, h
     WalkArgs a = args_of(c, F);
     a.ord = c.map[outLevel].ord.p;
     a.cost = c.map[outLevel].cost.p;
-    a.frank = c.frank.p;
-    a.jrank = c.jrank.p;
     a.outLevel = outLevel;
     // the other levels, in tree order, as the walk's levels 1..N-1
     const uint64_t es = F.dtype == MMCSF_F32 ? 4 : 2;

@@ -43,7 +43,6 @@
 namespace mmcsf {
 
 struct WalkArgs {
-    const uint32_t *ptr[3];
     const uint32_t *idx[3];
     const uint32_t *slc;   // slice coordinate of each level-1 entry
     const uint32_t *leaf;
@@ -51,9 +50,9 @@ struct WalkArgs {
     const uint32_t *fbit;  // leaf-fiber starts over nonzeros
     const uint32_t *sbit;  // 4-D: level-1 starts over leaf fibers
     const uint32_t *cost;  // exclusive cost prefix over chunks (chunks + 1 entries)
+    const uint32_t *frank; // leaf fibers starting before each 64-bit word of fbit
+    const uint32_t *jrank; // 4-D: level-1 entries starting before each word of sbit
     const uint32_t *ord;   // kMap: stored position of every nonzero in walk order
-    const uint32_t *frank; // kMap: leaf fibers starting before each word of fbit
-    const uint32_t *jrank; // kMap, 4-D: level-1 entries starting before each word of sbit
     int outLevel;          // kMap: the tree level of the output mode
     const uint32_t *pos;   // tensor-order position of every stored nonzero
     const float *wts;      // weights in tensor order

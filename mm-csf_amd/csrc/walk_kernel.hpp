@@ -11,25 +11,9 @@
 namespace mmcsf {
 namespace {
 
-// Largest i < n with a[i] <= key (a non-decreasing, a[0] <= key), searched by
-// the whole wave: each round probes 64 evenly spaced entries and keeps the
-// slot of the last probe <= key, so 2^26 entries take 5 rounds of one load.
-// Every lane must call it with the same arguments.
-__device__ __forceinline__ uint32_t wave_upper(const uint32_t *__restrict__ a, uint32_t n, uint32_t key) {
-    const uint32_t lane = threadIdx.x & 63;
-    uint32_t lo = 0, hi = n;
-    while (hi - lo > 1) {
-        const uint32_t step = (hi - lo + 63) / 64;
-        const uint32_t probe = lo + lane * step;
-        const bool le = lane == 0 || (probe < hi && a[probe] <= key);
-        const uint64_t m = __ballot(le);
-        const uint32_t last = 63u - (uint32_t)__builtin_clzll(m);
-        lo += last * step;
-        hi = std::min(hi, lo + step);
-    }
-    return lo;
-}
-
+// Searches by the whole wave: each round probes 64 evenly spaced entries, so
+// 2^24 entries take 4 rounds of one load.  Every lane must call it with the
+// same arguments.
 // first i in [0, n] with a[i] >= key (a non-decreasing over n + 1 entries)
 __device__ __forceinline__ uint32_t wave_lower(const uint32_t *__restrict__ a, uint32_t n, uint32_t key) {
     const uint32_t lane = threadIdx.x & 63;
@@ -214,12 +198,23 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
                             ? blockIdx.x
                             : ((blockIdx.x & 7u) + 8u * ((blockIdx.x >> 3) / spanBlocks)) * spanBlocks +
                                   (blockIdx.x >> 3) % spanBlocks;
-    const uint64_t wv = (uint64_t)lb * wavesPerBlock + (threadIdx.x >> 6);
+    // (the wave's index in a scalar register: so are its run and the tree
+    // positions at its start)
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint64_t wv = (uint64_t)lb * wavesPerBlock + w;
     const uint32_t chunks = (uint32_t)(((uint64_t)a.nnz + 63) / 64);
-    // this wave's chunks: an equal share of the total traversal cost
-    const uint64_t total = a.cost[chunks];
-    const uint32_t cb = wave_lower(a.cost, chunks, (uint32_t)(wv * total / waves));
-    const uint32_t ce = wv + 1 == waves ? chunks : wave_lower(a.cost, chunks, (uint32_t)((wv + 1) * total / waves));
+    // this wave's chunks: an equal share of the total traversal cost, or one
+    // chunk where there is a wave for each (the search is two dependent reads
+    // or more, of the ~8 that such a short run waits for)
+    uint32_t cb, ce;
+    if (chunks <= waves) {
+        cb = (uint32_t)std::min<uint64_t>(wv, chunks);
+        ce = std::min(cb + 1, chunks);
+    } else {
+        const uint64_t total = a.cost[chunks];
+        cb = wave_lower(a.cost, chunks, (uint32_t)(wv * total / waves));
+        ce = wv + 1 == waves ? chunks : wave_lower(a.cost, chunks, (uint32_t)((wv + 1) * total / waves));
+    }
     const int R = a.R;
     const uint32_t rowBytes = (uint32_t)R * (uint32_t)sizeof(T);
     // First of this lane's columns in block b.  RAG: the row's last lane has
@@ -294,7 +289,7 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
         // end; a condition around the whole run costs 6 registers more, and
         // the widest case then a wave per SIMD)
         if constexpr (kGrad) {
-            if (lane == 0) tailRow[threadIdx.x >> 6] = kNone;
+            if (lane == 0) tailRow[w] = kNone;
             __syncthreads();
         }
         return;
@@ -302,15 +297,14 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
     const uint32_t x0 = (uint32_t)(cb * 64);
     [[maybe_unused]] uint32_t fcur = kNone, jcur = kNone;
     if constexpr (SRC == kTree) {
-        // leaf fiber (and 4-D level-1 entry) of the nonzero before the run; the
-        // unsigned wrap at x0 = 0 stands for -1
-        const uint32_t *__restrict__ ptrL = a.ptr[LF];
-        const uint32_t f0 = wave_upper(ptrL, a.cnt[LF], x0);  // leaf fiber of x0
-        fcur = x0 == 0 ? kNone : (a.ptr[LF][f0] == x0 ? f0 - 1 : f0);
+        // leaf fiber (and 4-D level-1 entry) of the nonzero before the run, by
+        // the ranks of the start bits; the unsigned wrap at x0 = 0 stands for -1
+        fcur = a.frank[cb] - 1u;
+        const uint32_t f0 = fcur + (a.fbit[2 * cb] & 1u);  // leaf fiber of x0
         uint32_t j0 = f0;
         if constexpr (N == 4) {
-            j0 = wave_upper(a.ptr[1], a.cnt[1], f0);
-            jcur = fcur == kNone ? kNone : (a.ptr[1][j0] == f0 && fcur != f0 ? j0 - 1 : j0);
+            j0 = dev::rank_of(a.sbit, a.jrank, f0);
+            jcur = fcur == kNone ? kNone : dev::rank_of(a.sbit, a.jrank, fcur);
         }
         scur = OP == kTtm ? f0 : a.slc[j0];
     } else if constexpr (SRC == kCoo) {
@@ -845,7 +839,6 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
         // each distinct row once.  A quarter of the float32 additions to a hot
         // row's total: relative error of skewed modes 2.4e-7 -> 1.1e-7 (100M
         // nonzeros, Zipf(1.2)), and fewer atomics waiting on one another.
-        const int w = threadIdx.x >> 6;
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
 #pragma unroll
@@ -859,15 +852,15 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
         if (lane == 0) tailRow[w] = scur;
         __syncthreads();
         if (g == 0 && (w == 0 || tailRow[w - 1] != scur)) {
-            int we = w + 1;
-            while (we < (int)wavesPerBlock && tailRow[we] == scur) ++we;
+            uint32_t we = w + 1;
+            while (we < wavesPerBlock && tailRow[we] == scur) ++we;
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 float v[VEC];
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
                     double t = 0.0;
-                    for (int q = w; q < we; ++q) t += (double)tail[q][b * BW + k * VEC + e];
+                    for (uint32_t q = w; q < we; ++q) t += (double)tail[q][b * BW + k * VEC + e];
                     v[e] = (float)t;
                 }
                 put(b, scur, v, false);
