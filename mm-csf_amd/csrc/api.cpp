@@ -1255,8 +1255,6 @@ int mmcsf_ttm(const mmcsf_format *fh, int R, int dtype, const void *factor, floa
         MMCSF_REQUIRE(reinterpret_cast<uintptr_t>(factor) % need == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0,
                       MMCSF_ERR_ARG, "factor / output pointer is not aligned");
         hipStream_t s = static_cast<hipStream_t>(stream);
-        const uint64_t rows = c.cnt[c.ndims - 2];
-        fill_zero(Y, rows * (uint64_t)R, s);
         Factors F{};
         for (int m = 0; m < f.ndims; ++m) F.U[m] = factor;  // only the leaf factor is read
         F.dtype = dtype;

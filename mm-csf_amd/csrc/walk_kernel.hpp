@@ -36,6 +36,42 @@ __device__ __forceinline__ uint32_t wave_lower(const uint32_t *__restrict__ a, u
     return lo;
 }
 
+// Chunks [cb, ce) of wave wv of `waves`: an equal share of the total traversal
+// cost, or one chunk where there is a wave for each (the search is two
+// dependent reads or more, of the ~8 that such a short run waits for).
+__device__ __forceinline__ void wave_run(const uint32_t *__restrict__ cost, uint32_t chunks, uint64_t wv,
+                                         uint64_t waves, uint32_t &cb, uint32_t &ce) {
+    if (chunks <= waves) {
+        cb = (uint32_t)std::min<uint64_t>(wv, chunks);
+        ce = std::min(cb + 1, chunks);
+    } else {
+        const uint64_t total = cost[chunks];
+        cb = wave_lower(cost, chunks, (uint32_t)(wv * total / waves));
+        ce = wv + 1 == waves ? chunks : wave_lower(cost, chunks, (uint32_t)((wv + 1) * total / waves));
+    }
+}
+
+// Clears the rows that waves of a walk keyed by leaf fiber add to instead of
+// storing: the fibers of the first and the last nonzero of each wave's run.
+// Every other row is stored by the one wave that holds its fiber.
+// (An output row per fiber makes clearing all of Y a pass of its own: 10M
+// fibers, R = 32, 217 us of 708; here 10.)
+template <int OP>
+__global__ __launch_bounds__(256) void k_clear_run_ends(WalkArgs a, uint64_t waves) {
+    const uint64_t wv = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    if (wv >= waves) return;  // the whole wave leaves together
+    const uint32_t chunks = (uint32_t)(((uint64_t)a.nnz + 63) / 64);
+    uint32_t cb, ce;
+    wave_run(a.cost, chunks, wv, waves, cb, ce);
+    if (cb >= ce) return;
+    const uint32_t last = (uint32_t)std::min<uint64_t>((uint64_t)ce * 64, a.nnz) - 1;
+    const size_t f0 = dev::rank_of(a.fbit, a.frank, cb * 64), f1 = dev::rank_of(a.fbit, a.frank, last);
+    for (int c = threadIdx.x & 63; c < a.R; c += 64) {
+        a.out[f0 * a.R + c] = 0.f;
+        a.out[f1 * a.R + c] = 0.f;
+    }
+}
+
 // Buffer resource of one factor table (gfx9 raw buffer: stride 0, byte
 // range checked): lanes whose offset is at or past `bytes` read zeros and
 // access no memory.
@@ -203,18 +239,8 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint64_t wv = (uint64_t)lb * wavesPerBlock + w;
     const uint32_t chunks = (uint32_t)(((uint64_t)a.nnz + 63) / 64);
-    // this wave's chunks: an equal share of the total traversal cost, or one
-    // chunk where there is a wave for each (the search is two dependent reads
-    // or more, of the ~8 that such a short run waits for)
     uint32_t cb, ce;
-    if (chunks <= waves) {
-        cb = (uint32_t)std::min<uint64_t>(wv, chunks);
-        ce = std::min(cb + 1, chunks);
-    } else {
-        const uint64_t total = a.cost[chunks];
-        cb = wave_lower(a.cost, chunks, (uint32_t)(wv * total / waves));
-        ce = wv + 1 == waves ? chunks : wave_lower(a.cost, chunks, (uint32_t)((wv + 1) * total / waves));
-    }
+    wave_run(a.cost, chunks, wv, waves, cb, ce);
     const int R = a.R;
     const uint32_t rowBytes = (uint32_t)R * (uint32_t)sizeof(T);
     // First of this lane's columns in block b.  RAG: the row's last lane has
@@ -909,6 +935,11 @@ void go(const WalkArgs &a, hipStream_t s) {
     // spread over the CUs.
     const uint64_t block = std::min<uint64_t>(kWalkWaves, (chunks + cus - 1) / cus);
     const uint64_t blocks = std::min<uint64_t>(cus * perCU, (chunks + block - 1) / block);
+    if constexpr (OP == kTtm) {
+        const uint64_t waves = blocks * block;
+        k_clear_run_ends<OP><<<dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s>>>(a, waves);
+        MMCSF_HIP(hipGetLastError());
+    }
     fn<<<dim3((unsigned)blocks), dim3((unsigned)(64 * block)), 0, s>>>(a);
     MMCSF_HIP(hipGetLastError());
 }

@@ -241,3 +241,29 @@ def test_version_1_caches_load(cuda, golden_dir, tmp_path, name, dims, fmt_type,
     Ud = [torch.from_numpy(u).to(cuda) for u in U]
     for m in range(len(dims)):
         assert rel(mmcsf.mttkrp(f, m, Ud).cpu().numpy(), O.mttkrp_coo_f64(inds, vals, m, U)) < 1e-5
+
+
+# ---- TTM without a cleared output ---------------------------------------------------
+
+@pytest.mark.parametrize("fibers,per_fiber", [(1, 1), (1, 64), (63, 1), (64, 1), (65, 2), (3, 4000), (5000, 1),
+                                              (200_000, 1), (1000, 63), (1000, 64), (777, 65), (90, 3000)])
+def test_ttm_writes_every_row(cuda, fibers, per_fiber):
+    """Fibers shorter and longer than chunks, runs and blocks; the output holds
+    other numbers before the call."""
+    import torch
+    import mmcsf
+    rng = np.random.default_rng(fibers + per_fiber)
+    n = fibers * per_fiber
+    f = np.repeat(np.arange(fibers, dtype=np.int64), per_fiber)
+    leaf = np.tile(np.arange(per_fiber, dtype=np.int64), fibers)
+    dims = [(fibers - 1) // 50 + 1, 50, max(4000, per_fiber)]
+    vals = (rng.random(n) + 0.25).astype(np.float32)
+    t = mmcsf.Tensor.from_numpy(dims, [f // 50, f % 50, leaf], vals)
+    fm = mmcsf.Format(t, 8, mode=0)
+    assert fm.info()["modeOrder"] == [0, 1, 2]
+    for R in (4, 32, 72):
+        U = rng.random((dims[2], R)).astype(np.float32)
+        Y = torch.full((fibers, R), 3.0, device=cuda)
+        mmcsf.ttm(fm, torch.from_numpy(U).to(cuda), out=Y)
+        want = np.einsum("fl,lr->fr", vals.astype(np.float64).reshape(fibers, per_fiber), U[:per_fiber].astype(np.float64))
+        assert rel(Y.cpu().numpy(), want) < 1e-5, R
