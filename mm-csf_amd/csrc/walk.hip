@@ -208,7 +208,12 @@ void ttm_fibers(const Csf &c, const Factors &F, float *Y, hipStream_t s) {
                   "factor pointer is not aligned to " + std::to_string(need) + " bytes");
     WalkArgs a = args_of(c, F);
     a.out = Y;
-    walk_launch<kTtm>(c.ndims, F, a, s);
+    // Y past the 256 MB memory-side cache cannot be read back from it, and its
+    // lines only push the factor rows out: written around the caches (20M
+    // nonzeros, 10M fibers, R = 32, 1.28 GB of rows: 486 -> 459 us).  Smaller
+    // outputs stay where their reader finds them.
+    if (c.cnt[c.ndims - 2] * (uint64_t)F.R * 4u > (256ull << 20)) walk_launch<kTtmStream>(c.ndims, F, a, s);
+    else walk_launch<kTtm>(c.ndims, F, a, s);
 }
 
 void preload_kernels(bool cp) {

@@ -85,6 +85,7 @@ enum WalkOp : int {
     kLossResid = 2,   // sumsq += e^2; resid[pos] = e
     kWeightGrad = 3,  // out += alpha * wts[pos] * product
     kTtm = 4,         // out[leaf fiber] += v * U_leaf[leaf] (tensor-times-matrix)
+    kTtmStream = 5,   // the same, rows written around the caches
 };
 
 // one traversal of the root tree of c; instantiated per operation in its

@@ -210,7 +210,8 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
     constexpr bool kGrad = OP != kLossResid;  // writes rows of `out`
     // multiplies the rows of the upper levels; rows of `out` are keyed by
     // slice (by leaf fiber for TTM, which has no upper levels)
-    constexpr bool kUpper = OP != kTtm;
+    constexpr bool kByFiber = OP == kTtm || OP == kTtmStream;
+    constexpr bool kUpper = !kByFiber;
     constexpr bool kFactor = kFactorOf<N, G, NB, OP>;
     static_assert(!(kFactor && (OP == kLossGrad || OP == kLossResid)), "the CP passes multiply per nonzero");
     // residuals / weights are addressed by tensor-order position
@@ -300,7 +301,13 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
         float *o = a.out + (size_t)row * R + c0;
         if (store && !a.accum) {
 #pragma unroll
-            for (int e = 0; e < VEC; e += 4) *reinterpret_cast<F4 *>(o + e) = F4{v[e], v[e + 1], v[e + 2], v[e + 3]};
+            for (int e = 0; e < VEC; e += 4) {
+                const F4 q{v[e], v[e + 1], v[e + 2], v[e + 3]};
+                // (an operation of its own: a store chosen at run time is merged
+                // with the plain one and loses the hint)
+                if constexpr (OP == kTtmStream) __builtin_nontemporal_store(q, reinterpret_cast<F4 *>(o + e));
+                else *reinterpret_cast<F4 *>(o + e) = q;
+            }
         } else {
 #pragma unroll
             for (int e = 0; e < VEC; ++e)
@@ -332,7 +339,7 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
             j0 = dev::rank_of(a.sbit, a.jrank, f0);
             jcur = fcur == kNone ? kNone : dev::rank_of(a.sbit, a.jrank, fcur);
         }
-        scur = OP == kTtm ? f0 : a.slc[j0];
+        scur = kByFiber ? f0 : a.slc[j0];
     } else if constexpr (SRC == kCoo) {
         scur = a.idx[0][x0];
     } else {
@@ -935,7 +942,7 @@ void go(const WalkArgs &a, hipStream_t s) {
     // spread over the CUs.
     const uint64_t block = std::min<uint64_t>(kWalkWaves, (chunks + cus - 1) / cus);
     const uint64_t blocks = std::min<uint64_t>(cus * perCU, (chunks + block - 1) / block);
-    if constexpr (OP == kTtm) {
+    if constexpr (OP == kTtm || OP == kTtmStream) {
         const uint64_t waves = blocks * block;
         k_clear_run_ends<OP><<<dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s>>>(a, waves);
         MMCSF_HIP(hipGetLastError());

@@ -267,3 +267,24 @@ def test_ttm_writes_every_row(cuda, fibers, per_fiber):
         mmcsf.ttm(fm, torch.from_numpy(U).to(cuda), out=Y)
         want = np.einsum("fl,lr->fr", vals.astype(np.float64).reshape(fibers, per_fiber), U[:per_fiber].astype(np.float64))
         assert rel(Y.cpu().numpy(), want) < 1e-5, R
+
+
+def test_ttm_large_output(cuda):
+    """More than 256 MB of rows, which are written around the caches."""
+    import torch
+    import mmcsf
+    fibers, R = 1_050_001, 64
+    f = np.arange(fibers, dtype=np.int64)
+    inds = [np.concatenate([f // 1000, f[:500] // 1000]), np.concatenate([f % 1000, f[:500] % 1000]),
+            np.concatenate([f % 37, 40 + f[:500] % 9])]
+    rng = np.random.default_rng(5)
+    vals = (rng.random(fibers + 500) + 0.25).astype(np.float32)
+    dims = [fibers // 1000 + 1, 1000, 2000]
+    fm = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), 8, mode=0)
+    assert fm.info()["nLevel"][1] == fibers and fibers * R * 4 > 256 << 20
+    U = rng.random((dims[2], R)).astype(np.float32)
+    Y = torch.full((fibers, R), 3.0, device=cuda)
+    mmcsf.ttm(fm, torch.from_numpy(U).to(cuda), out=Y)
+    want = vals[:fibers, None].astype(np.float64) * U[inds[2][:fibers]]
+    want[:500] += vals[fibers:, None].astype(np.float64) * U[inds[2][fibers:]]
+    assert rel(Y.cpu().numpy(), want) < 1e-5
