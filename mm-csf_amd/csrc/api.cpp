@@ -1147,11 +1147,23 @@ int mmcsf_mttkrp_allmode(const mmcsf_format *fh, int R, int dtype, const void *c
         for (int m = 0; m < f.ndims; ++m) F.U[m] = factors[m];
         F.dtype = dtype;
         F.R = R;
+        // every output cleared by one launch, and (untimed, every mode with a
+        // root tree) every mode walked by one where the walks are short
+        uint64_t count[kMaxDims];
+        const Csf *trees[kMaxDims];
+        bool roots = !ms_per_mode && !f.mixed;
         for (int m = 0; m < f.ndims; ++m) {
             MMCSF_REQUIRE(outs[m] != nullptr, MMCSF_ERR_ARG, "missing output");
-            mttkrp_mode(f, m, F, outs[m], s, ms_per_mode ? ev[2 * m] : nullptr,
-                        ms_per_mode ? ev[2 * m + 1] : nullptr);
+            count[m] = f.dims[m] * (uint64_t)R;
+            trees[m] = f.hasTree[m] ? &f.tree[m] : &f.csf;
+            roots = roots && trees[m]->order[0] == m;
         }
+        MMCSF_REQUIRE(R >= 1 && R <= 256, MMCSF_ERR_UNSUPPORTED, "R must be in 1..256");
+        fill_zero_all(outs, count, f.ndims, s);
+        if (!roots || !mttkrp_roots(trees, f.ndims, F, outs, s))
+            for (int m = 0; m < f.ndims; ++m)
+                mttkrp_mode(f, m, F, outs[m], s, ms_per_mode ? ev[2 * m] : nullptr,
+                            ms_per_mode ? ev[2 * m + 1] : nullptr, true);
         if (ms_per_mode) {
             MMCSF_HIP(hipEventSynchronize(ev[2 * f.ndims - 1]));
             for (int m = 0; m < f.ndims; ++m)

@@ -348,6 +348,9 @@ void mttkrp_mode(const Format &f, int mode, const Factors &F, float *out, hipStr
 // of four for bfloat16 rows) and the start bitmasks of the tree
 bool walk_supports(const Csf &c, int R, int dtype);
 void mttkrp_root(const Csf &c, const Factors &F, float *out, hipStream_t s, bool accumulate = false);
+// the root walks of all modes in one launch, into zeroed outputs; false
+// (nothing launched) when they are better launched one by one
+bool mttkrp_roots(const Csf *const *trees, int modes, const Factors &F, float *const *outs, hipStream_t s);
 // the MTTKRP of the mode at level outLevel > 0 of a tree with level maps
 bool map_walk_supports(const Csf &c, const Factors &F, int outLevel, const float *out);
 void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, hipStream_t s, bool accumulate);
@@ -360,6 +363,8 @@ void mttkrp_hyb(const Hyb &h, const uint64_t *dims, const Factors &F, float *out
 void preload_kernels(bool cp);
 void preload_group_kernels();
 void fill_zero(float *p, uint64_t n, hipStream_t s);
+// up to kMaxDims arrays in one launch
+void fill_zero_all(float *const *p, const uint64_t *n, int arrays, hipStream_t s);
 
 // TTM (walk.hip): Y[leaf fiber] = sum over its nonzeros of v * U_leaf[leaf]
 void ttm_fibers(const Csf &c, const Factors &F, float *Y, hipStream_t s);

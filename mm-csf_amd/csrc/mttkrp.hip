@@ -300,6 +300,24 @@ __global__ void k_zero(float *p, uint64_t n) {
     for (; i < n; i += stride) p[i] = 0.f;
 }
 
+struct ZeroArgs {
+    float *p[kMaxDims];
+    uint64_t n[kMaxDims];
+};
+
+// array blockIdx.y, 16 bytes a lane between its unaligned ends
+__global__ void k_zero_all(ZeroArgs z) {
+    float *p = z.p[blockIdx.y];
+    const uint64_t n = z.n[blockIdx.y];
+    const uint64_t head = min(n, (uint64_t)((16 - (reinterpret_cast<uintptr_t>(p) & 15)) & 15) / 4);
+    const uint64_t quads = (n - head) / 4;
+    const uint64_t t = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
+    float4 *q = reinterpret_cast<float4 *>(p + head);
+    for (uint64_t i = t; i < quads; i += stride) q[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (t < head) p[t] = 0.f;
+    if (t < n - head - 4 * quads) p[head + 4 * quads + t] = 0.f;
+}
+
 // --------------------------------------------------------------------------
 // dispatch over the row geometry
 // --------------------------------------------------------------------------
@@ -459,6 +477,20 @@ static void launch_csf(const Csf &c, const Geo &g, const Factors &F, float *out,
     a.R = F.R;
     if (c.ndims == 3) launch_csf_t<3>(g, a, F.dtype, s);
     else launch_csf_t<4>(g, a, F.dtype, s);
+}
+
+void fill_zero_all(float *const *p, const uint64_t *n, int arrays, hipStream_t s) {
+    ZeroArgs z{};
+    uint64_t most = 0;
+    for (int i = 0; i < arrays; ++i) {
+        z.p[i] = p[i];
+        z.n[i] = n[i];
+        most = std::max(most, n[i]);
+    }
+    if (!most) return;
+    const uint64_t blocks = std::min<uint64_t>((most / 4 + 255) / 256 + 1, 8192);
+    hipLaunchKernelGGL(k_zero_all, dim3((unsigned)blocks, (unsigned)arrays), dim3(256), 0, s, z);
+    MMCSF_HIP(hipGetLastError());
 }
 
 void mttkrp_csf(const Csf &c, const uint64_t *dims, int outLevel, const Factors &F, float *out,

@@ -68,6 +68,12 @@ struct WalkArgs {
     int R;
 };
 
+// several walks launched together, and the blocks of each
+struct WalkSet {
+    WalkArgs walk[kMaxDims];
+    uint32_t blocks[kMaxDims];
+};
+
 // Where a nonzero's coordinates come from.
 enum WalkSrc : int {
     kTree = 0,  // a CSF tree rooted at the output mode
@@ -92,6 +98,10 @@ enum WalkOp : int {
 // own translation unit (walk_<op>.hip)
 template <int OP, int SRC = kTree>
 void walk_launch(int ndims, const Factors &F, const WalkArgs &a, hipStream_t s);
+// several traversals alike but for their trees, in one launch; false (nothing
+// launched) when they are better launched one by one
+template <int OP, int SRC = kTree>
+bool walk_launch_set(int ndims, const Factors &F, WalkSet &set, int walks, hipStream_t s);
 template <int OP, int SRC = kTree>
 void walk_preload();
 

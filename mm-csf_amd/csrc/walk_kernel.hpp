@@ -201,7 +201,7 @@ constexpr int kWalkWaves = 4;
 // RAG: ranks that VEC does not divide (float32 MTTKRP; its own instances, since
 // the column arithmetic costs the widest cases a wave per SIMD)
 template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG, int SRC>
-__global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 1 && G * VEC <= 32) ? 3 : 2) void k_walk(WalkArgs a) {
+__device__ __forceinline__ void walk(const WalkArgs &a, const uint32_t gridBlocks) {
     static_assert(G == 1 || G == 2 || G == 4 || G == 8, "row groups of 1..8 lanes");
     static_assert(G % TB == 0, "steps per batch divide the steps of a chunk");
     static_assert(VEC % 4 == 0, "rows are written as float4");
@@ -224,14 +224,14 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
     const int lane = threadIdx.x & 63;
     const int g = lane / G, k = lane % G;
     const uint64_t wavesPerBlock = blockDim.x >> 6;
-    const uint64_t waves = (uint64_t)gridDim.x * wavesPerBlock;
+    const uint64_t waves = (uint64_t)gridBlocks * wavesPerBlock;
     // Workgroups are dispatched round-robin over the 8 XCDs (block b on XCD
     // b % 8).  Each XCD takes 16 spans of consecutive blocks spread over the
     // tree, so neighbouring waves (which share slices and fiber rows) sit on
     // one L2, while every XCD still sees all parts of the tree.
     constexpr uint32_t kSpans = 16;
-    const uint32_t spanBlocks = gridDim.x / (8u * kSpans);
-    const uint32_t lb = gridDim.x % (8u * kSpans)
+    const uint32_t spanBlocks = gridBlocks / (8u * kSpans);
+    const uint32_t lb = gridBlocks % (8u * kSpans)
                             ? blockIdx.x
                             : ((blockIdx.x & 7u) + 8u * ((blockIdx.x >> 3) / spanBlocks)) * spanBlocks +
                                   (blockIdx.x >> 3) % spanBlocks;
@@ -909,6 +909,21 @@ __global__ __launch_bounds__(64 * kWalkWaves, (OP == kMttkrp && N == 3 && NB == 
     }
 }
 
+template <int N, int G, int NB, int VEC, int OP>
+constexpr int kMinWaves = (OP == kMttkrp && N == 3 && NB == 1 && G * VEC <= 32) ? 3 : 2;
+
+template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG, int SRC>
+__global__ __launch_bounds__(64 * kWalkWaves, (kMinWaves<N, G, NB, VEC, OP>)) void k_walk(WalkArgs a) {
+    walk<N, G, NB, TB, T, VEC, OP, RAG, SRC>(a, gridDim.x);
+}
+
+// The walks of several trees in one launch, a row of the grid each.
+template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG, int SRC>
+__global__ __launch_bounds__(64 * kWalkWaves, (kMinWaves<N, G, NB, VEC, OP>)) void k_walk_set(WalkSet set) {
+    if (blockIdx.x < set.blocks[blockIdx.y])
+        walk<N, G, NB, TB, T, VEC, OP, RAG, SRC>(set.walk[blockIdx.y], set.blocks[blockIdx.y]);
+}
+
 struct Cfg {
     int G, NB, TB, VEC;
 };
@@ -929,39 +944,71 @@ Cfg pick(int R, int dtype) {
     return c;
 }
 
-template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG, int SRC>
-void go(const WalkArgs &a, hipStream_t s) {
-    auto fn = k_walk<N, G, NB, TB, T, VEC, OP, RAG, SRC>;
+// resident blocks of the current device
+template <typename K>
+uint64_t resident_blocks(K fn) {
     int perCU = 0;
-    MMCSF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fn, 256, 0));
-    perCU = std::max(perCU, 1);
-    const uint64_t cus = (uint64_t)device_cu_count();
-    const uint64_t chunks = ((uint64_t)a.nnz + 63) / 64;
-    // a wave start is found by a search over the cost prefix; more waves than
-    // chunks would give empty waves only.  The waves of a small tensor are
-    // spread over the CUs.
-    const uint64_t block = std::min<uint64_t>(kWalkWaves, (chunks + cus - 1) / cus);
-    const uint64_t blocks = std::min<uint64_t>(cus * perCU, (chunks + block - 1) / block);
-    if constexpr (OP == kTtm || OP == kTtmStream) {
-        const uint64_t waves = blocks * block;
-        k_clear_run_ends<OP><<<dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s>>>(a, waves);
-        MMCSF_HIP(hipGetLastError());
-    }
-    fn<<<dim3((unsigned)blocks), dim3((unsigned)(64 * block)), 0, s>>>(a);
-    MMCSF_HIP(hipGetLastError());
+    MMCSF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fn, 64 * kWalkWaves, 0));
+    return (uint64_t)device_cu_count() * std::max(perCU, 1);
 }
 
-template <int N, typename T, int VEC, int OP, int SRC>
-void dispatch(const Cfg &c, const WalkArgs &a, hipStream_t s) {
-#define MMCSF_WALK(GG, BB, TT)                       \
-    if (c.G == GG && c.NB == BB && c.TB == TT) {     \
+template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG, int SRC>
+struct Walk {
+    // one walk: a wave start is found by a search over the cost prefix; more
+    // waves than chunks would give empty waves only.  The waves of a small
+    // tensor are spread over the CUs.
+    static void launch(const WalkArgs &a, hipStream_t s) {
+        auto fn = k_walk<N, G, NB, TB, T, VEC, OP, RAG, SRC>;
+        const uint64_t cus = (uint64_t)device_cu_count();
+        const uint64_t chunks = ((uint64_t)a.nnz + 63) / 64;
+        const uint64_t block = std::min<uint64_t>(kWalkWaves, (chunks + cus - 1) / cus);
+        const uint64_t blocks = std::min<uint64_t>(resident_blocks(fn), (chunks + block - 1) / block);
+        if constexpr (OP == kTtm || OP == kTtmStream) {
+            const uint64_t waves = blocks * block;
+            k_clear_run_ends<OP><<<dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s>>>(a, waves);
+            MMCSF_HIP(hipGetLastError());
+        }
+        fn<<<dim3((unsigned)blocks), dim3((unsigned)(64 * block)), 0, s>>>(a);
+        MMCSF_HIP(hipGetLastError());
+    }
+    // Several walks at once; false when they are better launched one by one.
+    // Side by side / in turn, all modes from the call on: 1M nonzeros 41 / 56 us
+    // (3-D, R = 32), 67 / 104 (4-D, R = 32), 6M 176 / 192 and 377 / 398, 10M
+    // 350 / 361 and 274 / 276 (3-D, R = 16); at 20M 541 / 516 (3-D, R = 16).
+    // The line is drawn at the chunks per resident wave of ~8M nonzeros.
+    static constexpr uint64_t kSetChunks = 96;
+    static bool launch_set(WalkSet &set, int walks, hipStream_t s) {
+        auto fn = k_walk_set<N, G, NB, TB, T, VEC, OP, RAG, SRC>;
+        const uint64_t cus = (uint64_t)device_cu_count();
+        uint64_t chunks = 0, most = 0;
+        for (int i = 0; i < walks; ++i) chunks += ((uint64_t)set.walk[i].nnz + 63) / 64;
+        const uint64_t resident = resident_blocks(fn);
+        if (chunks > kSetChunks * resident * kWalkWaves) return false;
+        const uint64_t block = std::min<uint64_t>(kWalkWaves, (chunks + cus - 1) / cus);
+        for (int i = 0; i < walks; ++i) {
+            const uint64_t c = ((uint64_t)set.walk[i].nnz + 63) / 64;
+            const uint64_t b = std::min<uint64_t>(std::max<uint64_t>(resident / walks, 1), (c + block - 1) / block);
+            set.blocks[i] = (uint32_t)b;
+            most = std::max(most, b);
+        }
+        fn<<<dim3((unsigned)most, (unsigned)walks), dim3((unsigned)(64 * block)), 0, s>>>(set);
+        MMCSF_HIP(hipGetLastError());
+        return true;
+    }
+};
+
+// calls f with the Walk of the configuration
+template <int N, typename T, int VEC, int OP, int SRC, typename F>
+void dispatch(const Cfg &c, int R, F f) {
+#define MMCSF_WALK(GG, BB, TT)                                    \
+    if (c.G == GG && c.NB == BB && c.TB == TT) {                  \
         if constexpr (OP == kMttkrp && std::is_same_v<T, float>)  \
-            if (a.R % VEC != 0) {                    \
-                go<N, GG, BB, TT, T, VEC, OP, true, SRC>(a, s); \
-                return;                              \
-            }                                        \
-        go<N, GG, BB, TT, T, VEC, OP, false, SRC>(a, s); \
-        return;                                      \
+            if (R % VEC != 0) {                                   \
+                f(Walk<N, GG, BB, TT, T, VEC, OP, true, SRC>{});  \
+                return;                                           \
+            }                                                     \
+        f(Walk<N, GG, BB, TT, T, VEC, OP, false, SRC>{});         \
+        return;                                                   \
     }
     MMCSF_WALK(1, 1, 1)
     MMCSF_WALK(2, 1, 2)
@@ -980,6 +1027,20 @@ void dispatch(const Cfg &c, const WalkArgs &a, hipStream_t s) {
     fail(MMCSF_ERR_UNSUPPORTED, "no root-walk kernel for this rank");
 }
 
+template <int OP, int SRC, typename F>
+void dispatch_all(int ndims, const Factors &fac, F f) {
+    const Cfg cfg = pick(fac.R, fac.dtype);
+    if (ndims == 3) {
+        if (fac.dtype == MMCSF_F32) dispatch<3, float, 4, OP, SRC>(cfg, fac.R, f);
+        else if (cfg.VEC == 8) dispatch<3, uint16_t, 8, OP, SRC>(cfg, fac.R, f);
+        else dispatch<3, uint16_t, 4, OP, SRC>(cfg, fac.R, f);
+    } else {
+        if (fac.dtype == MMCSF_F32) dispatch<4, float, 4, OP, SRC>(cfg, fac.R, f);
+        else if (cfg.VEC == 8) dispatch<4, uint16_t, 8, OP, SRC>(cfg, fac.R, f);
+        else dispatch<4, uint16_t, 4, OP, SRC>(cfg, fac.R, f);
+    }
+}
+
 }  // namespace
 
 // loads this translation unit's code object on the current device (a kernel
@@ -992,16 +1053,14 @@ void walk_preload() {
 
 template <int OP, int SRC>
 void walk_launch(int ndims, const Factors &F, const WalkArgs &a, hipStream_t s) {
-    const Cfg cfg = pick(F.R, F.dtype);
-    if (ndims == 3) {
-        if (F.dtype == MMCSF_F32) dispatch<3, float, 4, OP, SRC>(cfg, a, s);
-        else if (cfg.VEC == 8) dispatch<3, uint16_t, 8, OP, SRC>(cfg, a, s);
-        else dispatch<3, uint16_t, 4, OP, SRC>(cfg, a, s);
-    } else {
-        if (F.dtype == MMCSF_F32) dispatch<4, float, 4, OP, SRC>(cfg, a, s);
-        else if (cfg.VEC == 8) dispatch<4, uint16_t, 8, OP, SRC>(cfg, a, s);
-        else dispatch<4, uint16_t, 4, OP, SRC>(cfg, a, s);
-    }
+    dispatch_all<OP, SRC>(ndims, F, [&](auto w) { w.launch(a, s); });
+}
+
+template <int OP, int SRC>
+bool walk_launch_set(int ndims, const Factors &F, WalkSet &set, int walks, hipStream_t s) {
+    bool done = false;
+    dispatch_all<OP, SRC>(ndims, F, [&](auto w) { done = w.launch_set(set, walks, s); });
+    return done;
 }
 
 }  // namespace mmcsf

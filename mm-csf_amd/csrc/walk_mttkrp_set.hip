@@ -1,0 +1,6 @@
+// Chunked root walks of several modes in one launch (all-mode MTTKRP).
+#include "walk_kernel.hpp"
+
+namespace mmcsf {
+template bool walk_launch_set<kMttkrp>(int, const Factors &, WalkSet &, int, hipStream_t);
+}  // namespace mmcsf

@@ -288,3 +288,37 @@ def test_ttm_large_output(cuda):
     want = vals[:fibers, None].astype(np.float64) * U[inds[2][:fibers]]
     want[:500] += vals[fibers:, None].astype(np.float64) * U[inds[2][fibers:]]
     assert rel(Y.cpu().numpy(), want) < 1e-5
+
+
+# ---- all modes in one launch -------------------------------------------------------
+
+@pytest.mark.parametrize("dims,skew,nnz", [
+    ([4, 3, 2], [None] * 3, 1),
+    ([300, 200, 100], [None] * 3, 64),
+    ([300, 1, 100], [None] * 3, 4000),
+    ([5000, 70, 900], [1.2, None, 1.1], 16_384 * 8),   # a chunk per wave and more
+    ([900, 800, 700], [None] * 3, 1_000_000),
+    ([90, 80, 70, 60], [None] * 4, 333),
+    ([900, 80, 70, 600], [1.1, None, None, 1.2], 300_000),
+])
+def test_allmode_in_one_launch(cuda, dims, skew, nnz):
+    """All modes side by side equal each mode by itself, which goes through a
+    launch of its own, and float64; outputs hold other numbers before."""
+    import torch
+    import mmcsf
+    import oracle as O
+    rng = np.random.default_rng(nnz)
+    inds, vals = random_tensor(rng, dims, nnz, skew)
+    f = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), 12, fbr_threshold=128)
+    for R, dt in ((4, "f32"), (10, "f32"), (32, "f32"), (32, "bf16"), (64, "bf16"), (132, "f32")):
+        Ud = [torch.from_numpy(rng.random((d, R)).astype(np.float32)).to(cuda) for d in dims]
+        if dt == "bf16":
+            Ud = [u.to(torch.bfloat16) for u in Ud]
+        outs = [torch.full((d, R), 9.0, device=cuda) for d in dims]
+        mmcsf.mttkrp_allmode(f, Ud, outs=outs)
+        for m in range(len(dims)):
+            one = mmcsf.mttkrp(f, m, Ud)
+            assert rel(outs[m].cpu().numpy(), one.cpu().numpy()) < 1e-6, (R, dt, m)
+            if nnz <= 200_000 and R in (10, 32):
+                ref = O.mttkrp_coo_f64(inds, vals, m, [u.float().cpu().numpy() for u in Ud])
+                assert rel(outs[m].cpu().numpy(), ref) < 1e-5, (R, dt, m)
