@@ -333,9 +333,11 @@ struct Factors {
 // output has been zeroed.
 // accumulate: add to `out` (not zeroed here; every row written with atomics)
 // zeroed: `out` already holds zeros (the caller cleared it); not zeroed again
+// anyAlign: factors that the root walk would refuse for their alignment go to
+// the per-group kernel
 void mttkrp_csf(const Csf &c, const uint64_t *dims, int outLevel, const Factors &F, float *out,
                 hipStream_t s, hipEvent_t evStart = nullptr, hipEvent_t evEnd = nullptr, bool accumulate = false,
-                bool zeroed = false);
+                bool zeroed = false, bool anyAlign = false);
 void mttkrp_coo(const Format &f, const Factors &F, float *out, hipStream_t s);
 // the same as a chunked walk (walk.hip); `out` zeroed by the caller
 bool coo_walk_supports(const Format &f, const Factors &F);
@@ -357,6 +359,7 @@ void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, h
 // the walk's row loads are 16 bytes wide (8 for bfloat16 with R % 8 != 0):
 // factor tables of every level but skipLevel, and `out`, must be aligned to that
 void check_walk_align(const Csf &c, const Factors &F, int skipLevel, const float *out);
+bool walk_aligned(const Csf &c, const Factors &F, int skipLevel, const float *out);
 void mttkrp_hyb(const Hyb &h, const uint64_t *dims, const Factors &F, float *out, hipStream_t s);
 // loads the code objects of the MTTKRP kernels (and, cp, of the CP
 // completion passes) on the current device, once per process

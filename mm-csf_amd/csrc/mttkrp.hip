@@ -494,7 +494,7 @@ void fill_zero_all(float *const *p, const uint64_t *n, int arrays, hipStream_t s
 }
 
 void mttkrp_csf(const Csf &c, const uint64_t *dims, int outLevel, const Factors &F, float *out,
-                hipStream_t s, hipEvent_t evStart, hipEvent_t evEnd, bool accumulate, bool zeroed) {
+                hipStream_t s, hipEvent_t evStart, hipEvent_t evEnd, bool accumulate, bool zeroed, bool anyAlign) {
     const int N = c.ndims;
     if (!accumulate && !zeroed) fill_zero(out, dims[c.order[outLevel]] * (uint64_t)F.R, s);
     if (evStart) MMCSF_HIP(hipEventRecord(evStart, s));
@@ -541,7 +541,7 @@ void mttkrp_csf(const Csf &c, const uint64_t *dims, int outLevel, const Factors 
         else launch_map_t<4>(g, a, F.dtype, s);
         return;
     }
-    if (walk_supports(c, F.R, F.dtype)) {
+    if (walk_supports(c, F.R, F.dtype) && (!anyAlign || walk_aligned(c, F, 0, out))) {
         mttkrp_root(c, F, out, s, accumulate);  // checks the alignment its row loads need
         return;
     }
@@ -566,7 +566,9 @@ void mttkrp_mode(const Format &f, int mode, const Factors &F, float *out, hipStr
         return;
     }
     if (f.hasTree[mode]) {
-        mttkrp_csf(f.tree[mode], f.dims, 0, F, out, s, evStart, evEnd, false, zeroed);
+        // MM-CSF refuses bfloat16 rows at 8-byte boundaries where 16 are needed;
+        // the one-tree types take them in every mode but their root
+        mttkrp_csf(f.tree[mode], f.dims, 0, F, out, s, evStart, evEnd, false, zeroed, f.type != MMCSF_TYPE_MMCSF);
         return;
     }
     int lvl = 0;

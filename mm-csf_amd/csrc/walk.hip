@@ -74,6 +74,13 @@ void check_walk_align(const Csf &c, const Factors &F, int skipLevel, const float
                   ragged ? "output pointer is not aligned to 4 bytes" : "output pointer is not aligned to 16 bytes");
 }
 
+bool walk_aligned(const Csf &c, const Factors &F, int skipLevel, const float *out) {
+    const uintptr_t need = F.R % 4 != 0 ? 4 : (F.dtype == MMCSF_BF16 && F.R % 8 != 0) ? 8 : 16;
+    for (int l = 0; l < c.ndims; ++l)
+        if (l != skipLevel && reinterpret_cast<uintptr_t>(F.U[c.order[l]]) % need != 0) return false;
+    return reinterpret_cast<uintptr_t>(out) % (F.R % 4 != 0 ? 4 : 16) == 0;
+}
+
 // Ranks: every multiple of four, and any float32 rank from 4 on.  Below 4 the
 // row is narrower than one lane's load and the per-group kernel serves it.  At
 // R = 10 (HB-CSF, 3.3M nonzeros, 123457 x 70001 x 9973) the per-group kernel,
@@ -142,11 +149,7 @@ void mttkrp_coo_walk(const Format &f, const Factors &F, float *out, hipStream_t 
 // two modes below the root: 7.19 -> 2.59 ms.  Those reads bound it: each lane's
 // is a line of its own past the L2, ~8.6 CU clocks apiece.
 bool map_walk_supports(const Csf &c, const Factors &F, int outLevel, const float *out) {
-    if (!walk_supports(c, F.R, F.dtype)) return false;
-    const uintptr_t need = F.R % 4 != 0 ? 4 : (F.dtype == MMCSF_BF16 && F.R % 8 != 0) ? 8 : 16;
-    for (int l = 0; l < c.ndims; ++l)
-        if (l != outLevel && reinterpret_cast<uintptr_t>(F.U[c.order[l]]) % need != 0) return false;
-    return reinterpret_cast<uintptr_t>(out) % (F.R % 4 != 0 ? 4 : 16) == 0;
+    return walk_supports(c, F.R, F.dtype) && walk_aligned(c, F, outLevel, out);
 }
 
 void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, hipStream_t s, bool accumulate) {
@@ -175,8 +178,9 @@ bool mttkrp_roots(const Csf *const *trees, int modes, const Factors &F, float *c
     WalkSet set{};
     for (int m = 0; m < modes; ++m) {
         const Csf &c = *trees[m];
-        if (c.nnz == 0 || !walk_supports(c, F.R, F.dtype)) return false;
-        check_walk_align(c, F, 0, outs[m]);
+        for (int l = 0; l < c.ndims; ++l)
+            if (!F.U[l]) return false;
+        if (c.nnz == 0 || !walk_supports(c, F.R, F.dtype) || !walk_aligned(c, F, 0, outs[m])) return false;
         set.walk[m] = args_of(c, F);
         set.walk[m].out = outs[m];
     }

@@ -178,7 +178,8 @@ def test_coo_walk(cuda, N, rows, nnz):
 
 # ---- modes below the root of a tree that serves every mode ------------------------
 
-ONE_TREE = [(9, {}), (13, {}), (14, {}), (12, {"mode_trees": False}), (12, {"mixed": True})]
+ONE_TREE = [(9, {}), (13, {}), (14, {}), (9, {"mode_trees": False}), (13, {"mode_trees": False}),
+            (14, {"mode_trees": False}), (12, {"mode_trees": False}), (12, {"mixed": True})]
 
 
 @pytest.mark.parametrize("dims,skew,nnz", [
@@ -207,8 +208,8 @@ def test_one_tree_every_mode(cuda, dims, skew, nnz, fmt_type, kw):
         for m in range(len(dims)):
             assert rel(outs[m].cpu().numpy(), O.mttkrp_coo_f64(inds, vals, m, U)) < 1e-5, (R, m)
         if R % 8 == 0:
-            # bfloat16 rows at 16 byte boundaries, and at 8 (per-group kernel; the
-            # root mode's walk refuses those)
+            # bfloat16 rows at 16 byte boundaries, and, for modes below the root, at
+            # 8 (per-group kernels)
             Ub = [u.to(torch.bfloat16) for u in Ud]
             Ur = [u.float().cpu().numpy() for u in Ub]
             root = f.info()["modeOrder"][0]
@@ -220,7 +221,7 @@ def test_one_tree_every_mode(cuda, dims, skew, nnz, fmt_type, kw):
                     assert rel(got.cpu().numpy(), O.mttkrp_coo_f64(inds, vals, m, Ur)) < 1e-5, (R, m, off)
 
 
-@pytest.mark.parametrize("name,dims,fmt_type,kw", [("one_tree_3d", [17, 11, 9], 14, {}),
+@pytest.mark.parametrize("name,dims,fmt_type,kw", [("one_tree_3d", [17, 11, 9], 14, {"mode_trees": False}),
                                                    ("single_tree_4d", [9, 7, 6, 5], 12, {"mode_trees": False}),
                                                    ("mixed_3d", [17, 11, 9], 12, {"mixed": True})])
 def test_version_1_caches_load(cuda, golden_dir, tmp_path, name, dims, fmt_type, kw):
