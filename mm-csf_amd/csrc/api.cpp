@@ -1392,15 +1392,23 @@ int mmcsf_cp_loss_grad(const mmcsf_format *fh, int R, int dtype, const void *con
                       "CP completion needs a B-CSF or MM-CSF format");
         MMCSF_REQUIRE(f.csf.pos.p || f.nnz == 0, MMCSF_ERR_ARG, "format holds no nonzero positions");
         hipStream_t s = static_cast<hipStream_t>(stream);
-        cp_zero(loss, s);
-        bool counted = false;
+        // the gradients and the loss (two floats wide) cleared by one launch
+        const Csf *trees[kMaxDims];
+        float *out[kMaxDims + 1];
+        uint64_t count[kMaxDims + 1];
+        int walks = 0;
         for (int m = 0; m < f.ndims; ++m) {
             if (!grads[m]) continue;
-            fill_zero(grads[m], f.dims[m] * (uint64_t)R, s);
-            cp_gradient(*root_tree(f, m), F, nullptr, alpha, grads[m], counted ? nullptr : loss, s);
-            counted = true;
+            trees[walks] = root_tree(f, m);
+            out[walks] = grads[m];
+            count[walks++] = f.dims[m] * (uint64_t)R;
         }
-        if (counted) cp_half(loss, s);
+        out[walks] = reinterpret_cast<float *>(loss);
+        count[walks] = 2;
+        fill_zero_all(out, count, walks + 1, s);
+        for (int i = 0; i < walks; ++i)
+            cp_gradient(*trees[i], F, nullptr, alpha, out[i], i == 0 ? loss : nullptr, s);
+        if (walks) cp_half(loss, s);
         else cp_forward(f.csf, F, nullptr, loss, s);
     });
 }

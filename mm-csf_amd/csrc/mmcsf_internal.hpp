@@ -366,7 +366,7 @@ void mttkrp_hyb(const Hyb &h, const uint64_t *dims, const Factors &F, float *out
 void preload_kernels(bool cp);
 void preload_group_kernels();
 void fill_zero(float *p, uint64_t n, hipStream_t s);
-// up to kMaxDims arrays in one launch
+// up to kMaxDims + 1 arrays in one launch
 void fill_zero_all(float *const *p, const uint64_t *n, int arrays, hipStream_t s);
 
 // TTM (walk.hip): Y[leaf fiber] = sum over its nonzeros of v * U_leaf[leaf]
@@ -379,7 +379,6 @@ void cp_forward(const Csf &c, const Factors &F, float *resid, double *loss, hipS
 void cp_gradient(const Csf &c, const Factors &F, const float *weights, float alpha, float *grad, double *loss,
                  hipStream_t s);
 void cp_half(double *loss, hipStream_t s);
-void cp_zero(double *loss, hipStream_t s);
 
 // binary cache of built formats (cache.cpp)
 void format_save(const Format &f, const char *path);

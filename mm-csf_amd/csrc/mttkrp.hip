@@ -301,8 +301,8 @@ __global__ void k_zero(float *p, uint64_t n) {
 }
 
 struct ZeroArgs {
-    float *p[kMaxDims];
-    uint64_t n[kMaxDims];
+    float *p[kMaxDims + 1];
+    uint64_t n[kMaxDims + 1];
 };
 
 // array blockIdx.y, 16 bytes a lane between its unaligned ends

@@ -264,9 +264,4 @@ void cp_half(double *loss, hipStream_t s) {
     MMCSF_HIP(hipGetLastError());
 }
 
-void cp_zero(double *loss, hipStream_t s) {
-    hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(64), 0, s, loss);
-    MMCSF_HIP(hipGetLastError());
-}
-
 }  // namespace mmcsf
