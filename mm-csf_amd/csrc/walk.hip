@@ -1,6 +1,7 @@
 // Entry points of the chunked root walk (the kernel is in walk_kernel.hpp,
 // instantiated per operation in walk_mttkrp.hip, walk_loss.hip,
 // walk_lossgrad.hip, walk_wgrad.hip and walk_ttm.hip).
+#include <algorithm>
 #include <mutex>
 
 #include "walk.hpp"
@@ -33,8 +34,65 @@ WalkArgs args_of(const Csf &c, const Factors &F) {
     }
     a.nnz = (uint32_t)c.nnz;
     a.R = F.R;
+    a.cols = F.R;
     a.alpha = 1.f;
     return a;
+}
+
+// Columns that one MTTKRP pass takes.  A pass holds a group's rows, partial sums
+// and loads in flight in registers.  Past two column blocks (64 float32
+// columns) it runs at two waves per SIMD, and past four (128) it spills: passes
+// over 64 columns, which read the tree again, take over.  All modes, one pass /
+// passes of 64, float32: 30M nonzeros, 3-D (500000 x 200000 x 50000) R = 96
+// 4.06 / 3.22 ms, 128 4.62 / 4.26, 160 9.4 / 5.4, 256 11.7 / 8.6; 2M nonzeros
+// (3000 x 2000 x 1000) R = 96 246 / 243 us, 128 251 / 294, 160 499 / 378, 256
+// 595 / 567.  So from 97 to 128 columns it is one pass, but for 3-D tables past
+// the L2s (4 MB per XCD), which passes bring closer to fitting.  A 4-D walk
+// does not factor at two column blocks and waits on such tables' lines most:
+// there passes of 32 columns win from R = 64 on (30M nonzeros, tables of 43 MB:
+// 4.70 / 4.57 ms, R = 128 9.9 / 9.0).  Bfloat16 rows are half as wide and stay
+// in one pass (R = 128: 2.38 / 2.45 ms, 2M nonzeros R = 256 284 / 410 us).
+int pass_columns(int N, const WalkArgs &a, const Factors &F) {
+    const int R = F.R;
+    if (F.dtype != MMCSF_F32) return R;
+    uint64_t bytes = 0;
+    for (int l = 1; l < N; ++l) bytes += a.tabBytes[l];
+    const bool far = bytes >= (24ull << 20);
+    if (N == 4 && far && R > 32 && R % 32 == 0) return 32;
+    if (R > 128 || (R > 64 && R <= 96) || (R > 96 && far && N == 3)) return 64;
+    return R;
+}
+
+// the pass that starts at column `at`: `width` columns, fewer at the end, but
+// never fewer than four left over (a lane's load)
+int pass_width(int R, int at, int width) {
+    const int left = R - at;
+    if (left <= width) return left;
+    return left - width < 4 ? width - 4 : width;
+}
+
+// moves a walk to the columns from `at` on
+void take_columns(int N, WalkArgs &a, const Factors &F, int at, int cols) {
+    const uint32_t skip = (uint32_t)at * (F.dtype == MMCSF_F32 ? 4u : 2u);
+    for (int l = 0; l < N; ++l) {
+        if (a.U[l]) a.U[l] = static_cast<const char *>(a.U[l]) + skip;
+        a.tabBytes[l] -= std::min(a.tabBytes[l], skip);
+    }
+    a.out += at;
+    a.cols = cols;
+}
+
+// launches an MTTKRP walk once per pass over columns
+template <typename L>
+void walk_columns(int N, const WalkArgs &a, const Factors &F, L launch) {
+    const int width = pass_columns(N, a, F);
+    for (int at = 0; at < F.R;) {
+        WalkArgs p = a;
+        const int cols = pass_width(F.R, at, width);
+        take_columns(N, p, F, at, cols);
+        launch(p);
+        at += cols;
+    }
 }
 
 __global__ void k_zero_f64(double *p) {
@@ -98,7 +156,7 @@ void mttkrp_root(const Csf &c, const Factors &F, float *out, hipStream_t s, bool
     WalkArgs a = args_of(c, F);
     a.out = out;
     a.accum = accumulate ? 1 : 0;
-    walk_launch<kMttkrp>(c.ndims, F, a, s);
+    walk_columns(c.ndims, a, F, [&](const WalkArgs &p) { walk_launch<kMttkrp>(c.ndims, F, p, s); });
 }
 
 // The COO type's root-mode MTTKRP as a walk: the coordinates are read once per
@@ -132,9 +190,10 @@ void mttkrp_coo_walk(const Format &f, const Factors &F, float *out, hipStream_t 
     }
     a.nnz = (uint32_t)f.nnz;
     a.R = F.R;
+    a.cols = F.R;
     a.alpha = 1.f;
     a.out = out;
-    walk_launch<kMttkrp, kCoo>(N, F, a, s);
+    walk_columns(N, a, F, [&](const WalkArgs &p) { walk_launch<kMttkrp, kCoo>(N, F, p, s); });
 }
 
 // The modes below the root of a tree that serves every mode.  A tree holds an
@@ -167,7 +226,7 @@ void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, h
     }
     a.out = out;
     a.accum = accumulate ? 1 : 0;
-    walk_launch<kMttkrp, kMap>(c.ndims, F, a, s);
+    walk_columns(c.ndims, a, F, [&](const WalkArgs &p) { walk_launch<kMttkrp, kMap>(c.ndims, F, p, s); });
 }
 
 // The root walks of every mode in one launch, into zeroed outputs.  A walk of
@@ -184,7 +243,17 @@ bool mttkrp_roots(const Csf *const *trees, int modes, const Factors &F, float *c
         set.walk[m] = args_of(c, F);
         set.walk[m].out = outs[m];
     }
-    return walk_launch_set<kMttkrp>(trees[0]->ndims, F, set, modes, s);
+    const int N = trees[0]->ndims, R = F.R;
+    // passes over columns as for one walk; the first decides for all of them
+    const int width = pass_columns(N, set.walk[0], F);
+    for (int at = 0; at < R;) {
+        WalkSet p = set;
+        const int cols = pass_width(R, at, width);
+        for (int m = 0; m < modes; ++m) take_columns(N, p.walk[m], F, at, cols);
+        if (!walk_launch_set<kMttkrp>(N, F, p, modes, at > 0, s)) return false;
+        at += cols;
+    }
+    return true;
 }
 
 bool cp_supports(int R) { return R >= 1 && R <= 128 && R % 4 == 0; }

@@ -65,7 +65,8 @@ struct WalkArgs {
     int accum;             // add every row with atomics (other writers share `out`)
     uint32_t nnz;
     uint32_t cnt[4];
-    int R;
+    int R;                 // rank: the width of every factor and output row
+    int cols;              // columns of this pass, from U and out on
 };
 
 // several walks launched together, and the blocks of each
@@ -99,9 +100,9 @@ enum WalkOp : int {
 template <int OP, int SRC = kTree>
 void walk_launch(int ndims, const Factors &F, const WalkArgs &a, hipStream_t s);
 // several traversals alike but for their trees, in one launch; false (nothing
-// launched) when they are better launched one by one
+// launched) when they are better launched one by one, unless `always`
 template <int OP, int SRC = kTree>
-bool walk_launch_set(int ndims, const Factors &F, WalkSet &set, int walks, hipStream_t s);
+bool walk_launch_set(int ndims, const Factors &F, WalkSet &set, int walks, bool always, hipStream_t s);
 template <int OP, int SRC = kTree>
 void walk_preload();
 

@@ -242,8 +242,8 @@ __device__ __forceinline__ void walk(const WalkArgs &a, const uint32_t gridBlock
     const uint32_t chunks = (uint32_t)(((uint64_t)a.nnz + 63) / 64);
     uint32_t cb, ce;
     wave_run(a.cost, chunks, wv, waves, cb, ce);
-    const int R = a.R;
-    const uint32_t rowBytes = (uint32_t)R * (uint32_t)sizeof(T);
+    const int R = a.cols;  // columns of this pass; rows are a.R wide
+    const uint32_t rowBytes = (uint32_t)a.R * (uint32_t)sizeof(T);
     // First of this lane's columns in block b.  RAG: the row's last lane has
     // fewer than VEC columns of its own; it takes the last VEC columns of the
     // row instead, and computes the ones that it shares with the lane before it
@@ -298,7 +298,7 @@ __device__ __forceinline__ void walk(const WalkArgs &a, const uint32_t gridBlock
         const int col = b * BW + k * VEC;
         if (row == kNone || col >= R) return;
         const int c0 = colOf(b);
-        float *o = a.out + (size_t)row * R + c0;
+        float *o = a.out + (size_t)row * a.R + c0;
         if (store && !a.accum) {
 #pragma unroll
             for (int e = 0; e < VEC; e += 4) {
@@ -930,14 +930,14 @@ struct Cfg {
 
 // row groups of G lanes x VEC columns per load; NB column blocks; TB steps
 // of loads in flight (at most 32 row elements per lane and row kind)
-Cfg pick(int R, int dtype) {
+Cfg pick(int R, int cols, int dtype) {
     const int vec = (dtype == MMCSF_BF16 && R % 8 == 0) ? 8 : 4;
     Cfg c{8, 1, 8, vec};
-    if (R <= vec) c = {1, 1, 1, vec};
-    else if (R <= 2 * vec) c = {2, 1, 2, vec};
-    else if (R <= 4 * vec) c = {4, 1, 4, vec};
+    if (cols <= vec) c = {1, 1, 1, vec};
+    else if (cols <= 2 * vec) c = {2, 1, 2, vec};
+    else if (cols <= 4 * vec) c = {4, 1, 4, vec};
     else {
-        const int nb = (R + 8 * vec - 1) / (8 * vec);
+        const int nb = (cols + 8 * vec - 1) / (8 * vec);
         c.NB = nb <= 1 ? 1 : nb <= 2 ? 2 : nb <= 4 ? 4 : 8;
     }
     c.TB = std::max(1, std::min(c.G, 32 / (c.NB * vec)));
@@ -977,13 +977,13 @@ struct Walk {
     // 350 / 361 and 274 / 276 (3-D, R = 16); at 20M 541 / 516 (3-D, R = 16).
     // The line is drawn at the chunks per resident wave of ~8M nonzeros.
     static constexpr uint64_t kSetChunks = 96;
-    static bool launch_set(WalkSet &set, int walks, hipStream_t s) {
+    static bool launch_set(WalkSet &set, int walks, bool always, hipStream_t s) {
         auto fn = k_walk_set<N, G, NB, TB, T, VEC, OP, RAG, SRC>;
         const uint64_t cus = (uint64_t)device_cu_count();
         uint64_t chunks = 0, most = 0;
         for (int i = 0; i < walks; ++i) chunks += ((uint64_t)set.walk[i].nnz + 63) / 64;
         const uint64_t resident = resident_blocks(fn);
-        if (chunks > kSetChunks * resident * kWalkWaves) return false;
+        if (!always && chunks > kSetChunks * resident * kWalkWaves) return false;
         const uint64_t block = std::min<uint64_t>(kWalkWaves, (chunks + cus - 1) / cus);
         for (int i = 0; i < walks; ++i) {
             const uint64_t c = ((uint64_t)set.walk[i].nnz + 63) / 64;
@@ -1017,7 +1017,9 @@ void dispatch(const Cfg &c, int R, F f) {
         MMCSF_WALK(8, 1, 8)
         MMCSF_WALK(8, 2, 4)
         MMCSF_WALK(8, 4, 2)
-        MMCSF_WALK(8, 8, 1)
+        if constexpr (!(OP == kMttkrp && std::is_same_v<T, float>)) {  // (its passes end at 128 columns)
+            MMCSF_WALK(8, 8, 1)
+        }
     } else {
         MMCSF_WALK(8, 1, 4)
         MMCSF_WALK(8, 2, 2)
@@ -1028,8 +1030,8 @@ void dispatch(const Cfg &c, int R, F f) {
 }
 
 template <int OP, int SRC, typename F>
-void dispatch_all(int ndims, const Factors &fac, F f) {
-    const Cfg cfg = pick(fac.R, fac.dtype);
+void dispatch_all(int ndims, const Factors &fac, int cols, F f) {
+    const Cfg cfg = pick(fac.R, cols, fac.dtype);
     if (ndims == 3) {
         if (fac.dtype == MMCSF_F32) dispatch<3, float, 4, OP, SRC>(cfg, fac.R, f);
         else if (cfg.VEC == 8) dispatch<3, uint16_t, 8, OP, SRC>(cfg, fac.R, f);
@@ -1053,13 +1055,13 @@ void walk_preload() {
 
 template <int OP, int SRC>
 void walk_launch(int ndims, const Factors &F, const WalkArgs &a, hipStream_t s) {
-    dispatch_all<OP, SRC>(ndims, F, [&](auto w) { w.launch(a, s); });
+    dispatch_all<OP, SRC>(ndims, F, a.cols, [&](auto w) { w.launch(a, s); });
 }
 
 template <int OP, int SRC>
-bool walk_launch_set(int ndims, const Factors &F, WalkSet &set, int walks, hipStream_t s) {
+bool walk_launch_set(int ndims, const Factors &F, WalkSet &set, int walks, bool always, hipStream_t s) {
     bool done = false;
-    dispatch_all<OP, SRC>(ndims, F, [&](auto w) { done = w.launch_set(set, walks, s); });
+    dispatch_all<OP, SRC>(ndims, F, set.walk[0].cols, [&](auto w) { done = w.launch_set(set, walks, always, s); });
     return done;
 }
 

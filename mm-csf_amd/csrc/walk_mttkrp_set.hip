@@ -2,5 +2,5 @@
 #include "walk_kernel.hpp"
 
 namespace mmcsf {
-template bool walk_launch_set<kMttkrp>(int, const Factors &, WalkSet &, int, hipStream_t);
+template bool walk_launch_set<kMttkrp>(int, const Factors &, WalkSet &, int, bool, hipStream_t);
 }  // namespace mmcsf

@@ -323,3 +323,38 @@ def test_allmode_in_one_launch(cuda, dims, skew, nnz):
             if nnz <= 200_000 and R in (10, 32):
                 ref = O.mttkrp_coo_f64(inds, vals, m, [u.float().cpu().numpy() for u in Ud])
                 assert rel(outs[m].cpu().numpy(), ref) < 1e-5, (R, dt, m)
+
+
+# ---- MTTKRP in passes over columns ---------------------------------------------------
+
+@pytest.mark.parametrize("R,dt", [(64, "f32"), (65, "f32"), (66, "f32"), (67, "f32"), (68, "f32"), (72, "bf16"),
+                                  (76, "bf16"), (96, "f32"), (127, "f32"), (128, "f32"), (128, "bf16"), (129, "f32"),
+                                  (136, "bf16"), (140, "bf16"), (200, "bf16"), (255, "f32"), (256, "f32"),
+                                  (256, "bf16")])
+@pytest.mark.parametrize("dims,skew", [([800, 300, 90], [1.2, None, 1.1]),
+                                       ([90, 30_000, 200, 60_000], [1.2, None, None, 1.2])])
+def test_mttkrp_column_passes(cuda, dims, skew, R, dt):
+    """Widths around the passes' 64 columns; the 4-D tensor's tables are past
+    24 MB from R = 68 on, where R = 96, 128 and 256 go 32 columns at a time;
+    bfloat16 rows go in one pass.  Trees, COO and level maps; one launch per mode and all
+    modes in one."""
+    import torch
+    import mmcsf
+    import oracle as O
+    rng = np.random.default_rng(R)
+    inds, vals = random_tensor(rng, dims, 9001, skew)
+    t = mmcsf.Tensor.from_numpy(dims, inds, vals)
+    Ud = [torch.from_numpy(rng.random((d, R)).astype(np.float32)).to(cuda) for d in dims]
+    if dt == "bf16":
+        Ud = [u.to(torch.bfloat16) for u in Ud]
+    U = [u.float().cpu().numpy() for u in Ud]
+    ref = [O.mttkrp_coo_f64(inds, vals, m, U) for m in range(len(dims))]
+    for fmt_type, kw in ((12, {}), (14, {"mode_trees": False}), (12, {"mixed": True})):
+        f = mmcsf.Format(t, fmt_type, fbr_threshold=64, **kw)
+        outs, _ = mmcsf.mttkrp_allmode(f, Ud)
+        for m in range(len(dims)):
+            assert rel(outs[m].cpu().numpy(), ref[m]) < 1e-5, (fmt_type, m)
+            assert rel(mmcsf.mttkrp(f, m, Ud).cpu().numpy(), ref[m]) < 1e-5, (fmt_type, m)
+    for fmt_type in (3, 8, 10):
+        f = mmcsf.Format(t, fmt_type, mode=1)
+        assert rel(mmcsf.mttkrp(f, 1, Ud).cpu().numpy(), ref[1]) < 1e-5, fmt_type
