@@ -350,9 +350,10 @@ void mttkrp_mode(const Format &f, int mode, const Factors &F, float *out, hipStr
 // of four for bfloat16 rows) and the start bitmasks of the tree
 bool walk_supports(const Csf &c, int R, int dtype);
 void mttkrp_root(const Csf &c, const Factors &F, float *out, hipStream_t s, bool accumulate = false);
-// the root walks of all modes in one launch, into zeroed outputs; false
-// (nothing launched) when they are better launched one by one
-bool mttkrp_roots(const Csf *const *trees, int modes, const Factors &F, float *const *outs, hipStream_t s);
+// the root walks of several trees in one launch, into zeroed outputs (which may
+// be one output for trees without a root row in common); false (nothing
+// launched) when they are better launched one by one
+bool mttkrp_roots(const Csf *const *trees, int walks, const Factors &F, float *const *outs, hipStream_t s);
 // the MTTKRP of the mode at level outLevel > 0 of a tree with level maps
 bool map_walk_supports(const Csf &c, const Factors &F, int outLevel, const float *out);
 void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, hipStream_t s, bool accumulate);

@@ -647,6 +647,13 @@ void mttkrp_hyb(const Hyb &h, const uint64_t *dims, const Factors &F, float *out
             else run_geo<CooSel<4>::template K, CooArgs, uint16_t>(g, a, groups, s);
         }
     }
+    // The walked parts, which share no slice, in one launch where the walks are
+    // short (3.3M nonzeros, R = 10: 49 -> 47 us the call).
+    if (h.cslWalk.nnz && h.csf.nnz) {
+        const Csf *trees[2] = {&h.csf, &h.cslWalk};
+        float *const outs[2] = {out, out};
+        if (mttkrp_roots(trees, 2, F, outs, s)) return;
+    }
     // CSL part (3-D): walked as a tree of one-nonzero fibers; the CSL kernel
     // where the walk cannot run (R < 4, tables above 4 GiB)
     if (h.cslNnz && h.cslWalk.nnz && walk_supports(h.cslWalk, F.R, F.dtype)) {

@@ -229,16 +229,16 @@ void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, h
     walk_columns(c.ndims, a, F, [&](const WalkArgs &p) { walk_launch<kMttkrp, kMap>(c.ndims, F, p, s); });
 }
 
-// The root walks of every mode in one launch, into zeroed outputs.  A walk of
+// The root walks of several trees in one launch, into zeroed outputs.  A walk of
 // few chunks per wave is a chain of ~8 memory latencies and a launch; the modes'
 // chains then run side by side (300 x 200 x 100, 20000 nonzeros, R = 32: six
 // launches for the outputs and the walks, 34 us a call, are two, 20 us).
-bool mttkrp_roots(const Csf *const *trees, int modes, const Factors &F, float *const *outs, hipStream_t s) {
+bool mttkrp_roots(const Csf *const *trees, int walks, const Factors &F, float *const *outs, hipStream_t s) {
     WalkSet set{};
-    for (int m = 0; m < modes; ++m) {
+    for (int m = 0; m < walks; ++m) {
         const Csf &c = *trees[m];
-        for (int l = 0; l < c.ndims; ++l)
-            if (!F.U[l]) return false;
+        for (int l = 1; l < c.ndims; ++l)
+            if (!F.U[c.order[l]]) return false;
         if (c.nnz == 0 || !walk_supports(c, F.R, F.dtype) || !walk_aligned(c, F, 0, outs[m])) return false;
         set.walk[m] = args_of(c, F);
         set.walk[m].out = outs[m];
@@ -249,8 +249,8 @@ bool mttkrp_roots(const Csf *const *trees, int modes, const Factors &F, float *c
     for (int at = 0; at < R;) {
         WalkSet p = set;
         const int cols = pass_width(R, at, width);
-        for (int m = 0; m < modes; ++m) take_columns(N, p.walk[m], F, at, cols);
-        if (!walk_launch_set<kMttkrp>(N, F, p, modes, at > 0, s)) return false;
+        for (int m = 0; m < walks; ++m) take_columns(N, p.walk[m], F, at, cols);
+        if (!walk_launch_set<kMttkrp>(N, F, p, walks, at > 0, s)) return false;
         at += cols;
     }
     return true;

@@ -987,7 +987,8 @@ struct Walk {
         const uint64_t block = std::min<uint64_t>(kWalkWaves, (chunks + cus - 1) / cus);
         for (int i = 0; i < walks; ++i) {
             const uint64_t c = ((uint64_t)set.walk[i].nnz + 63) / 64;
-            const uint64_t b = std::min<uint64_t>(std::max<uint64_t>(resident / walks, 1), (c + block - 1) / block);
+            // the resident blocks, shared by chunks
+            const uint64_t b = std::min<uint64_t>(std::max<uint64_t>(resident * c / chunks, 1), (c + block - 1) / block);
             set.blocks[i] = (uint32_t)b;
             most = std::max(most, b);
         }
