@@ -4,7 +4,9 @@
 // iteration) and the solve statuses, after each iteration when a tolerance can
 // stop the loop, else in batches.  Arithmetic per step:
 //   MTTKRP                 the MM-CSF kernels (float32 accumulation)
-//   Gram  A^T A            MFMA v_mfma_f32_16x16x4f32 over row chunks, chunk sums
+//   Gram  A^T A            R <= 32: v_mfma_f64_16x16x4f64 inside the row solve;
+//                          wider ranks and the initial factors:
+//                          v_mfma_f32_16x16x4f32 over row chunks, chunk sums
 //                          reduced in float64
 //   Hadamard of Grams, the R x R inverse (Cholesky, in LDS for R <= 36; LU
 //   with partial pivoting when the matrix is not SPD),
@@ -226,112 +228,140 @@ __global__ void k_normal_inverse(const double *__restrict__ G, int N, int skip, 
     }
 }
 
-// U[i][j] = sum_k M[i][k] Hinv[k][j] (float64 accumulation); each thread
-// computes four columns of one row, reading M[i][k] once for all four
-// The same product for R <= 32 with R % 4 == 0: one row per thread (the grid
-// covers the rows once, so nothing is loop-invariant across rows and the
-// Hinv reads stay in the k loop), read with eight 16-byte loads; Hinv
-// zero-padded to 32 x 32 in LDS (every lane of a wave reads the same entry),
-// 32 float64 sums per thread.
-// U = M H^-1 for R <= 32 (R % 4 == 0), one row per thread, fused with the
-// column norms of the new rows: kind 0 adds float64 sums of squares to sq,
-// kind 1 the largest non-negative entry (order-preserving bits) to mx.  The
-// block's rows are one contiguous run of M and U: they are read and written
-// as consecutive float4 and pass through LDS (33 floats per row), where each
-// thread solves its row and the block reduces the columns, so that each block
-// adds one value per column.  H^-1 (Hpad: zero-padded to 32 x 32) is the same
-// for every lane: it is read with scalar loads and enters the float64 FMAs as
-// scalar operands.  Block 0 also clears Gz, the R x R Gram that
-// k_scale_gram32 accumulates next.
-constexpr int kSolveThreads = 512;
-__global__ __launch_bounds__(kSolveThreads) void k_solve_rows32(const float *__restrict__ M,
-                                                                const double *__restrict__ Hpad, uint32_t rows,
-                                                                int R, float *__restrict__ U, int kind,
-                                                                double *__restrict__ sq, uint32_t *__restrict__ mx,
-                                                                double *__restrict__ Gz) {
-    __shared__ float tile[kSolveThreads * 33];
-    __shared__ double ps[kSolveThreads];
-    using ConstD = const __attribute__((address_space(4))) double;
-    const ConstD *H = reinterpret_cast<const ConstD *>(reinterpret_cast<uintptr_t>(Hpad));
-    if (blockIdx.x == 0)
-        for (int e = threadIdx.x; e < R * R; e += blockDim.x) Gz[e] = 0.0;
-    const uint64_t row0 = (uint64_t)blockIdx.x * kSolveThreads;
-    const uint32_t nrows = (uint32_t)min((uint64_t)kSolveThreads, rows - row0);
-    const int q4 = R / 4;  // float4 per row
-    const uint32_t n4 = nrows * (uint32_t)q4;
-    // at most 8 float4 per thread (n4 <= 512 rows x 8): every read is issued
-    // before the first is waited for
-    constexpr int kPer = 8;
-    const float4 *m4 = reinterpret_cast<const float4 *>(M + row0 * R);
-    float4 v[kPer];
+// The row solve of a mode at R <= 32 (R % 4 == 0, 16-byte rows): U = M H^-1 with
+// the column norms of the new rows (kind 0 adds float64 sums of squares to sq,
+// kind 1 takes the largest non-negative entry, as order-preserving bits, into
+// mx) and their Gram.  All three products run on v_mfma_f64_16x16x4f64, 16
+// rows at a time:
+//   A  lane l: row l % 16, k = 8 (l / 16) + s at step s of 8 (the two float4
+//      that the lane reads; the order of k is free as long as B's is the same)
+//   B  lane l: H^-1[8 (l / 16) + s][l % 16 (+ 16)], held for all rows (Hpad:
+//      zero-padded to 32 x 32)
+//   D  lane l, register r: row 4 r + l / 16, column l % 16 (+ 16)
+// D's registers are the Gram's operands as they are: register r of every lane
+// is four rows of the transposed tile.  What bounds it is latency, not rate:
+// 200000 rows are 0.4 GFLOP and 51 MB.  The vector version (one row per thread
+// through LDS, H^-1 as scalar operands, 32 float64 sums a thread) took 28 / 25 /
+// 23 us at 200000 / 100000 / 20000 rows without the Gram, which was made in the
+// normalisation; this takes 27 / 17 / 15 us with it.  A block per CU at most, in
+// whole rounds of spans: at 200000 rows a block per span took 33 us, most of the
+// difference in adding the blocks' Grams.  Every block adds its norms and its Gram once; the Gram goes to one of
+// kGramCopies copies (zeroed by k_scale32), which shortens the chains of
+// additions to one address.
+constexpr int kSolveWaves = 8, kSolveTiles = 4;  // 64 rows per wave and span, 512 per block
+constexpr int kSolveRows = kSolveWaves * kSolveTiles * 16;
+constexpr int kGramCopies = 3;
+typedef double v4d __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(64 * kSolveWaves) void k_solve32(const float *__restrict__ M,
+                                                              const double *__restrict__ Hpad, uint32_t rows, int R,
+                                                              float *__restrict__ U, int kind,
+                                                              double *__restrict__ sq, uint32_t *__restrict__ mx,
+                                                              double *__restrict__ Gc) {
+    __shared__ double gram[3][256];   // tiles (0,0), (0,1), (1,1)
+    __shared__ double nsq[kSolveWaves][32];
+    __shared__ float nmx[kSolveWaves][32];
+    for (int e = threadIdx.x; e < 3 * 256; e += blockDim.x) gram[e / 256][e % 256] = 0.0;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int q = lane >> 4, c = lane & 15;
+    const bool two = R > 16;
+    double b0[8], b1[8];
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        const uint32_t e = threadIdx.x + q * kSolveThreads;
-        v[q] = e < n4 ? m4[e] : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s = 0; s < 8; ++s) {
+        b0[s] = Hpad[(8 * q + s) * 32 + c];
+        b1[s] = Hpad[(8 * q + s) * 32 + 16 + c];
+    }
+    uint64_t r0 = 0;
+    // this lane's columns 8q .. 8q+7 of row r0 + 16 t + c (zeros past R and past the rows)
+    auto read = [&](int t, float4 &x, float4 &y) {
+        const uint64_t row = r0 + 16 * t + c;
+        x = y = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (row < rows) {
+            const float *m = M + row * R + 8 * q;
+            if (8 * q < R) x = *reinterpret_cast<const float4 *>(m);
+            if (8 * q + 4 < R) y = *reinterpret_cast<const float4 *>(m + 4);
+        }
+    };
+    v4d g00 = {0, 0, 0, 0}, g01 = g00, g11 = g00;
+    double ss0 = 0.0, ss1 = 0.0;
+    float mm0 = 0.f, mm1 = 0.f;
+    for (uint64_t span = blockIdx.x; span * kSolveRows < rows; span += gridDim.x) {
+        r0 = span * kSolveRows + (uint64_t)w * (kSolveTiles * 16);
+        float4 x[kSolveTiles], y[kSolveTiles];
+#pragma unroll
+        for (int t = 0; t < kSolveTiles; ++t) read(t, x[t], y[t]);
+#pragma unroll
+        for (int t = 0; t < kSolveTiles; ++t) {
+            const float av[8] = {x[t].x, x[t].y, x[t].z, x[t].w, y[t].x, y[t].y, y[t].z, y[t].w};
+            v4d d0 = {0, 0, 0, 0}, d1 = d0;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                d0 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)av[s], b0[s], d0, 0, 0, 0);
+                if (two) d1 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)av[s], b1[s], d1, 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint64_t row = r0 + 16 * t + 4 * r + q;
+                const float u0 = (float)d0[r], u1 = (float)d1[r];
+                if (row < rows) {
+                    if (c < R) U[row * R + c] = u0;
+                    if (16 + c < R) U[row * R + 16 + c] = u1;
+                }
+                ss0 += (double)u0 * u0;
+                ss1 += (double)u1 * u1;
+                mm0 = fmaxf(mm0, u0);
+                mm1 = fmaxf(mm1, u1);
+                g00 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)u0, (double)u0, g00, 0, 0, 0);
+                if (two) {
+                    g01 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)u0, (double)u1, g01, 0, 0, 0);
+                    g11 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)u1, (double)u1, g11, 0, 0, 0);
+                }
+            }
+        }
     }
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        const uint32_t e = threadIdx.x + q * kSolveThreads;
-        if (e < n4) {
-            float *t = tile + (e / q4) * 33 + (e % q4) * 4;
-            t[0] = v[q].x; t[1] = v[q].y; t[2] = v[q].z; t[3] = v[q].w;
+    for (int off = 16; off < 64; off <<= 1) {
+        ss0 += __shfl_xor(ss0, off, 64);
+        ss1 += __shfl_xor(ss1, off, 64);
+        mm0 = fmaxf(mm0, __shfl_xor(mm0, off, 64));
+        mm1 = fmaxf(mm1, __shfl_xor(mm1, off, 64));
+    }
+    if (q == 0) {
+        nsq[w][c] = ss0;
+        nsq[w][16 + c] = ss1;
+        nmx[w][c] = mm0;
+        nmx[w][16 + c] = mm1;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int e = (4 * r + q) * 16 + c;
+        unsafeAtomicAdd(&gram[0][e], g00[r]);
+        if (two) {
+            unsafeAtomicAdd(&gram[1][e], g01[r]);
+            unsafeAtomicAdd(&gram[2][e], g11[r]);
         }
     }
     __syncthreads();
-    const bool live = threadIdx.x < nrows;
-    float *mine = tile + threadIdx.x * 33;
-    // the row times H^-1, 16 columns at a time (16 float64 sums live)
-    float out[32];
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        double s[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) s[j] = 0.0;
-#pragma unroll 4
-        for (int k = 0; k < 32; ++k) {
-            const double mk = k < R ? (double)mine[k] : 0.0;
-#pragma unroll
-            for (int j = 0; j < 16; ++j) s[j] = fma(mk, H[k * 32 + half * 16 + j], s[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) out[half * 16 + j] = (float)s[j];
+    double *G = Gc + (size_t)(blockIdx.x % kGramCopies) * R * R;
+    for (int e = threadIdx.x; e < R * R; e += blockDim.x) {
+        const int i = e / R, j = e % R;
+        // the (1,0) tile is the (0,1) tile's transpose
+        const int hi = max(i, j), lo = min(i, j);
+        const double v = i < 16 && j < 16 ? gram[0][i * 16 + j]
+                         : lo >= 16       ? gram[2][(i - 16) * 16 + j - 16]
+                                          : gram[1][lo * 16 + hi - 16];
+        unsafeAtomicAdd(G + e, v);
     }
-    // the new row replaces the thread's own row (rows past the factor and
-    // columns past R hold zero)
-#pragma unroll
-    for (int j = 0; j < 32; ++j) mine[j] = (live && j < R) ? out[j] : 0.f;
-    __syncthreads();
-    float4 *u4 = reinterpret_cast<float4 *>(U + row0 * R);
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        const uint32_t e = threadIdx.x + q * kSolveThreads;
-        if (e < n4) {
-            const float *t = tile + (e / q4) * 33 + (e % q4) * 4;
-            u4[e] = make_float4(t[0], t[1], t[2], t[3]);
+    if (threadIdx.x < R) {
+        const int j = threadIdx.x;
+        double s2 = 0.0;
+        float m2 = 0.f;
+        for (int v = 0; v < kSolveWaves; ++v) {
+            s2 += nsq[v][j];
+            m2 = fmaxf(m2, nmx[v][j]);
         }
-    }
-    // thread t: column t % 32 over rows t / 32, t / 32 + 16, ...
-    constexpr int kSubs = kSolveThreads / 32;
-    const int j = threadIdx.x % 32, sub = threadIdx.x / 32;
-    double ss = 0.0;
-    float mm = 0.f;
-    for (int r = sub; r < kSolveThreads; r += kSubs) {
-        const float v = tile[r * 33 + j];
-        ss += (double)v * v;
-        mm = fmaxf(mm, v);
-    }
-    __syncthreads();  // rows no longer read: the maxima reuse the front of the tile
-    float *pm = tile;
-    ps[sub * 32 + j] = ss;
-    pm[sub * 32 + j] = mm;
-    __syncthreads();
-    if (threadIdx.x < R) {  // sub 0, column j
-        for (int q = 1; q < kSubs; ++q) {
-            ss += ps[q * 32 + j];
-            mm = fmaxf(mm, pm[q * 32 + j]);
-        }
-        if (kind == 0) unsafeAtomicAdd(sq + j, ss);
-        else atomicMax(mx + j, __float_as_uint(mm));
+        if (kind == 0) unsafeAtomicAdd(sq + j, s2);
+        else atomicMax(mx + j, __float_as_uint(m2));
     }
 }
 
@@ -347,104 +377,72 @@ __device__ inline uint16_t to_bf16(float x) {
     return (uint16_t)(u >> 16);
 }
 
-// The normalisation and Gram of a factor (R <= 32): lambda from the column
-// norms, U[:, c] /= lambda_c in place, Ub (optional) = its bfloat16 copy, and
-// G += U^T U of the normalised rows.  Every wave owns kScaleRows rows and
-// all their columns (the 16 x 16 tiles cols 0-15 x 0-15, 0-15 x 16-31 and
-// 16-31 x 16-31, MFMA operands laid out as in k_gram), so each element is
-// read, scaled and written by one lane.  The block's 16 waves are summed in
-// LDS before the block adds its tiles to G.  Block 0 writes lambda and clears
-// sqNext / mxNext, the norm accumulators of the next update.  Mz (optional):
-// the first nz floats of the MTTKRP output, cleared for the next mode's
-// MTTKRP (nothing reads them after the row solve).
-constexpr int kScaleThreads = 1024;
-constexpr int kScaleRows = 64;
-__global__ __launch_bounds__(kScaleThreads) void k_scale_gram32(float *__restrict__ U, uint32_t rows, int R,
-                                                      int kind, const double *__restrict__ sq,
-                                                      const uint32_t *__restrict__ mx, double *__restrict__ lam,
-                                                      double *__restrict__ sqNext, uint32_t *__restrict__ mxNext,
-                                                      uint16_t *__restrict__ Ub, double *__restrict__ G,
-                                                      float *__restrict__ Mz, uint64_t nz) {
-    constexpr int kWaves = kScaleThreads / 64;
-    if (Mz) {
-        float4 *z4 = reinterpret_cast<float4 *>(Mz);
-        const uint64_t n4 = nz / 4, stride = (uint64_t)gridDim.x * blockDim.x;
-        for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n4; i += stride)
-            z4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (uint64_t i = n4 * 4 + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nz; i += stride) Mz[i] = 0.f;
-    }
-    __shared__ float part[3][kWaves][256];
-    if (blockIdx.x == 0 && threadIdx.x < R) {
-        lam[threadIdx.x] = lambda_of(kind, sq, mx, threadIdx.x);
-        sqNext[threadIdx.x] = 0.0;
-        mxNext[threadIdx.x] = 0u;
-    }
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const bool two = R > 16;
-    const int c0 = lane & 15, c1 = 16 + (lane & 15);
-    const bool ok0 = c0 < R, ok1 = c1 < R;
-    double d0 = ok0 ? lambda_of(kind, sq, mx, c0) : 1.0, d1 = ok1 ? lambda_of(kind, sq, mx, c1) : 1.0;
-    if (d0 == 0.0) d0 = 1.0;
-    if (d1 == 0.0) d1 = 1.0;
-    const uint64_t wave = (uint64_t)blockIdx.x * kWaves + wid;
-    const uint64_t r0 = wave * kScaleRows;
-    const uint64_t r1 = min((uint64_t)rows, r0 + kScaleRows);
-    const int kk = lane >> 4;
-    v4f a00 = {0.f, 0.f, 0.f, 0.f}, a01 = a00, a11 = a00;
-    for (uint64_t k = r0; k < r1; k += 16) {
-        float x0[4], x1[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint64_t row = k + 4 * q + kk;
-            const bool in = row < r1;
-            x0[q] = in && ok0 ? U[row * R + c0] : 0.f;
-            x1[q] = in && ok1 ? U[row * R + c1] : 0.f;
+// The normalisation of a factor after k_solve32: lambda from the column norms,
+// U[:, c] /= lambda_c in place, Ub (optional) = its bfloat16 copy.  Block 0
+// writes lambda, clears sqNext / mxNext, the norm accumulators of the next
+// update, and turns the Gram of the rows before the division, in kGramCopies
+// parts, into that of the normalised rows, G = D^-1 (sum of parts) D^-1 in
+// float64, clearing the parts.  Mz (optional): the first nz floats of the MTTKRP
+// output, cleared for the next mode's MTTKRP (nothing reads them after the row
+// solve).  One streaming pass (200000 rows, with the next output: 77 MB; the
+// version that also made the Gram took 29 / 21 / 17 us at 200000 / 100000 / 20000
+// rows, this one 10 / 7 / 5 us).
+constexpr int kScaleThreads = 256;
+__global__ __launch_bounds__(kScaleThreads) void k_scale32(float *__restrict__ U, uint32_t rows, int R, int kind,
+                                                           const double *__restrict__ sq,
+                                                           const uint32_t *__restrict__ mx, double *__restrict__ lam,
+                                                           double *__restrict__ sqNext, uint32_t *__restrict__ mxNext,
+                                                           uint16_t *__restrict__ Ub, double *__restrict__ Gc,
+                                                           double *__restrict__ G, float *__restrict__ Mz,
+                                                           uint64_t nz) {
+    __shared__ double inv[32];
+    if (threadIdx.x < R) {
+        const double d = lambda_of(kind, sq, mx, threadIdx.x);
+        inv[threadIdx.x] = d == 0.0 ? 1.0 : 1.0 / d;
+        if (blockIdx.x == 0) {
+            lam[threadIdx.x] = d;
+            sqNext[threadIdx.x] = 0.0;
+            mxNext[threadIdx.x] = 0u;
         }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint64_t row = k + 4 * q + kk;
-            const bool in = row < r1;
-            x0[q] = (float)((double)x0[q] / d0);
-            x1[q] = (float)((double)x1[q] / d1);
-            if (in && ok0) {
-                U[row * R + c0] = x0[q];
-                if (Ub) Ub[row * R + c0] = to_bf16(x0[q]);
-            }
-            if (in && ok1) {
-                U[row * R + c1] = x1[q];
-                if (Ub) Ub[row * R + c1] = to_bf16(x1[q]);
-            }
-            a00 = __builtin_amdgcn_mfma_f32_16x16x4f32(x0[q], x0[q], a00, 0, 0, 0);
-            if (two) {
-                a01 = __builtin_amdgcn_mfma_f32_16x16x4f32(x0[q], x1[q], a01, 0, 0, 0);
-                a11 = __builtin_amdgcn_mfma_f32_16x16x4f32(x1[q], x1[q], a11, 0, 0, 0);
-            }
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        part[0][wid][lane * 4 + r] = a00[r];
-        part[1][wid][lane * 4 + r] = a01[r];
-        part[2][wid][lane * 4 + r] = a11[r];
     }
     __syncthreads();
-    // tile t of the wave: t = 0 (0,0), 1 (0,1), 2 (1,1)
-    if (wid < (two ? 3 : 1)) {
-        const int bi = wid == 2 ? 1 : 0, bj = wid == 0 ? 0 : 1;
+    if (blockIdx.x == 0)
+        for (int e = threadIdx.x; e < R * R; e += kScaleThreads) {
+            double g = 0.0;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            float v = 0.f;
-            for (int w = 0; w < kWaves; ++w) v += part[wid][w][lane * 4 + r];
-            const int i = 16 * bi + 4 * (lane >> 4) + r;
-            const int j = 16 * bj + (lane & 15);
-            if (i < R && j < R) {
-                unsafeAtomicAdd(G + (size_t)i * R + j, (double)v);
-                if (bi != bj) unsafeAtomicAdd(G + (size_t)j * R + i, (double)v);
+            for (int p = 0; p < kGramCopies; ++p) {
+                g += Gc[(size_t)p * R * R + e];
+                Gc[(size_t)p * R * R + e] = 0.0;
             }
+            G[e] = g * inv[e / R] * inv[e % R];
         }
+    const uint64_t t = blockIdx.x * (uint64_t)kScaleThreads + threadIdx.x, stride = (uint64_t)gridDim.x * kScaleThreads;
+    float4 *u4 = reinterpret_cast<float4 *>(U);
+    const uint64_t n4 = (uint64_t)rows * R / 4;  // R % 4 == 0
+    const uint32_t per = (uint32_t)R / 4;
+    for (uint64_t i = t; i < n4; i += stride) {
+        const int c = (int)(i % per) * 4;
+        float4 v = u4[i];
+        v.x = (float)((double)v.x * inv[c]);
+        v.y = (float)((double)v.y * inv[c + 1]);
+        v.z = (float)((double)v.z * inv[c + 2]);
+        v.w = (float)((double)v.w * inv[c + 3]);
+        u4[i] = v;
+        if (Ub) {
+            ushort4 h = make_ushort4(to_bf16(v.x), to_bf16(v.y), to_bf16(v.z), to_bf16(v.w));
+            reinterpret_cast<ushort4 *>(Ub)[i] = h;
+        }
+    }
+    if (Mz) {
+        float4 *z4 = reinterpret_cast<float4 *>(Mz);
+        const uint64_t m4 = nz / 4;
+        for (uint64_t i = t; i < m4; i += stride) z4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (uint64_t i = m4 * 4 + t; i < nz; i += stride) Mz[i] = 0.f;
     }
 }
 
+// U[i][j] = sum_k M[i][k] Hinv[k][j] (float64 accumulation); each thread
+// computes four columns of one row, reading M[i][k] once for all four
 __global__ __launch_bounds__(256) void k_apply_inverse(const float *__restrict__ M, const double *__restrict__ Hinv,
                                                        uint32_t rows, int R, float *__restrict__ U) {
     extern __shared__ double hs[];
@@ -770,6 +768,11 @@ static void cpd_als_on(const Format &f, int R, int iters, double tol, int dtype,
     uint64_t upd = 0;  // factor updates so far (selects the half of the norm accumulators)
     bool mZeroed = false;  // the MTTKRP output was cleared for the next mode by the previous update
     clear_norms();
+    // the fused updates (R <= 32: the normal matrices then sit in LDS and leave
+    // W free) collect the Gram's parts there
+    static_assert(kGramCopies <= 3, "W holds 3 R x R matrices");
+    if (R <= 32)
+        hipLaunchKernelGGL(k_zero_d, dim3(grid_for(3 * RR)), dim3(256), 0, s, st.W, (uint64_t)(3 * RR));
     auto t0 = std::chrono::steady_clock::now();
     bool stop = false;
     while (it < iters && !stop) {
@@ -801,23 +804,22 @@ static void cpd_als_on(const Format &f, int R, int iters, double tol, int dtype,
                 }
                 const int kind = cur == 0 ? 0 : 1;  // 2-norm at iteration 0, max-norm after
                 if (fused) {
-                    // two launches: the row solve with the column norms, then lambda,
-                    // the normalisation, the bfloat16 copy and the Gram
+                    // two launches: the row solve with the column norms and the Gram,
+                    // then lambda, the normalisation and the bfloat16 copy
                     const int h = (int)(upd & 1);
-                    const unsigned solveBlocks = (unsigned)((f.dims[m] + kSolveThreads - 1) / kSolveThreads);
-                    hipLaunchKernelGGL(k_solve_rows32, dim3(solveBlocks), dim3(kSolveThreads), 0, s, st.M, st.Hpad,
-                                       (uint32_t)f.dims[m], R, U[m], kind, st.sq + h * R, st.mx + h * R,
-                                       st.G + m * RR);
+                    // whole rounds of spans over at most a block per CU
+                    const uint64_t spans = (f.dims[m] + kSolveRows - 1) / kSolveRows;
+                    const uint64_t rounds = (spans + device_cu_count() - 1) / device_cu_count();
+                    hipLaunchKernelGGL(k_solve32, dim3((unsigned)((spans + rounds - 1) / rounds)),
+                                       dim3(64 * kSolveWaves), 0, s, st.M, st.Hpad, (uint32_t)f.dims[m], R, U[m], kind,
+                                       st.sq + h * R, st.mx + h * R, st.W);
                     // modes before the last also clear the next mode's MTTKRP output
                     // (the last mode's output feeds the inner product of the fit)
                     const bool clearNext = m + 1 < N;
-                    const uint64_t waves = (f.dims[m] + kScaleRows - 1) / kScaleRows;
-                    const uint64_t wavesPerBlock = kScaleThreads / 64;
-                    hipLaunchKernelGGL(k_scale_gram32, dim3((unsigned)((waves + wavesPerBlock - 1) / wavesPerBlock)),
-                                       dim3(kScaleThreads), 0, s, U[m],
-                                       (uint32_t)f.dims[m], R, kind, st.sq + h * R, st.mx + h * R, st.lam,
+                    hipLaunchKernelGGL(k_scale32, dim3(grid_for(f.dims[m] * R / 4, 2048)), dim3(kScaleThreads), 0, s,
+                                       U[m], (uint32_t)f.dims[m], R, kind, st.sq + h * R, st.mx + h * R, st.lam,
                                        st.sq + (1 - h) * R, st.mx + (1 - h) * R,
-                                       dtype == MMCSF_BF16 ? st.Ub[m] : (uint16_t *)nullptr, st.G + m * RR,
+                                       dtype == MMCSF_BF16 ? st.Ub[m] : (uint16_t *)nullptr, st.W, st.G + m * RR,
                                        clearNext ? st.M : (float *)nullptr,
                                        clearNext ? f.dims[m + 1] * (uint64_t)R : 0ull);
                     mZeroed = clearNext;

@@ -358,3 +358,34 @@ def test_mttkrp_column_passes(cuda, dims, skew, R, dt):
     for fmt_type in (3, 8, 10):
         f = mmcsf.Format(t, fmt_type, mode=1)
         assert rel(mmcsf.mttkrp(f, 1, Ud).cpu().numpy(), ref[1]) < 1e-5, fmt_type
+
+
+# ---- CP-ALS row solve and Gram on float64 matrix instructions -----------------------
+
+@pytest.mark.parametrize("dims", [[513, 512, 17], [511, 64, 65], [1025, 33, 15], [131_073, 40, 30]])
+@pytest.mark.parametrize("R", [4, 12, 16, 20, 28, 32])
+def test_cpd_row_solve_edges(cuda, dims, R):
+    """Rows at the edges of 16-row tiles, 64-row waves, 512-row spans and of a
+    second round of spans; one and two column tiles, full and partial.  Bounds of
+    test_gpu_cpd.py: fits within 1e-4 of the float64 ALS, the model on the
+    observed entries within 1e-3."""
+    import torch
+    import mmcsf
+    from oracle import dense as D
+    from test_gpu_cpd import planted_tensor
+    rng = np.random.default_rng(R + dims[0])
+    inds, vals = planted_tensor(rng, dims, 40_000, R)
+    U0 = [(rng.random((d, R)) * 6 - 3).astype(np.float32) for d in dims]
+    fmt = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), 12, fbr_threshold=128)
+    iters = 4
+    Ud = [torch.from_numpy(u.copy()).to(cuda) for u in U0]
+    lam, st = mmcsf.cpd_als(fmt, Ud, iters=iters, tol=0.0)
+    fits, U64, lam64 = D.cpd_als(inds, vals, dims, [u.astype(np.float64) for u in U0], iters, tol=0.0)
+    np.testing.assert_allclose(st["fit_history"], fits, atol=1e-4, rtol=0)
+    mg = D.cp_model_values(inds, [u.cpu().double().numpy() * (lam if m == 0 else 1.0) for m, u in enumerate(Ud)])
+    m64 = D.cp_model_values(inds, [u * (lam64 if m == 0 else 1.0) for m, u in enumerate(U64)])
+    assert np.linalg.norm(mg - m64) / np.linalg.norm(m64) < 1e-3
+    # the allocation-free call takes the same path
+    Un = [torch.from_numpy(u.copy()).to(cuda) for u in U0]
+    lamn, stn = mmcsf.cpd_als(fmt, Un, iters=iters, tol=0.0, no_alloc=True)
+    np.testing.assert_allclose(stn["fit_history"], fits, atol=1e-4, rtol=0)
