@@ -426,11 +426,26 @@ void build_mixed(const Tensor &t, const mmcsf_options *opt, bool nat, Format &f,
 
 // A root tree for every mode but `root`: each MTTKRP becomes a root traversal.
 // These trees are internal, so their level order is free.  The leaf level is
-// gathered once per nonzero, the level-1 rows once per fiber segment: a 3-D
-// tree puts at its leaf the mode whose used rows concentrate in a clearly
-// smaller working set (rows holding 90% of the nonzeros; those stay in the
-// L2), and otherwise takes the order with fewer level-1 entries (fewer
-// fiber-level gathers).  One tree and 20M nonzeros (500000 x 200000 x 50000),
+// gathered once per nonzero, the level-1 rows once per fiber.  For a 3-D tree:
+//   - where neither other mode's used rows are clearly more concentrated (the
+//     rows holding 90% of the nonzeros, within a factor of 2), the order with
+//     fewer fibers.
+//   - else the concentrated mode, whose rows stay in the L2, is the leaf: at
+//     100M nonzeros (500000 x 200000 x 50000, Zipf(1.2) x Zipf(1.2) x uniform)
+//     the root 1 tree takes 1110 us so, with 0.41 fibers per nonzero, and
+//     1305 us with 0.19 the other way round.
+//   - but if nearly every nonzero would then be a fiber of its own (0.9 and
+//     more) the spread rows are gathered for every nonzero in either order, and
+//     the concentrated mode goes to level 1 if that saves a good part of its
+//     gathers: 200000 (Zipf(1.2)) x 100000 x 20000, 20M nonzeros, root 1: 269 us
+//     with 0.50 fibers per nonzero, 299 us with 0.995 and the concentrated leaf;
+//     1.02-1.38x over ranks 8 to 128, both storages and 2000 to 60000 rows of the
+//     spread mode at 0.5 and 0.63.  At 0.75 and 0.85 (2M nonzeros) it is
+//     0.94-1.01x, so the line is at 0.65.
+// The fibers are counted by pair_counts before anything is sorted; with both
+// trees built and one kept, a uniform tensor of 20M nonzeros took 18.0 ms to
+// build instead of 13.9, one of 20000 1.35 ms instead of 1.15.
+// One tree and 20M nonzeros (500000 x 200000 x 50000),
 // R = 32, all modes: 2.87 ms through level maps, 0.77 ms through root trees,
 // for 0.95 GB of structure instead of 0.54 and a build of 20 ms instead of 8.
 void build_mode_trees(const Tensor &t, const mmcsf_options *opt, bool nat, int root, bool positions, Format &f,
@@ -445,26 +460,31 @@ void build_mode_trees(const Tensor &t, const mmcsf_options *opt, bool nat, int r
         c.pos = std::move(p);
     };
     uint64_t hot[kMaxDims] = {0, 0, 0, 0};
-    if (t.ndims == 3) hot_footprints(t, 0.9, hot, s);
+    double pairs[3] = {0, 0, 0};
+    if (t.ndims == 3) {
+        hot_footprints(t, 0.9, hot, s);
+        pair_counts(t, pairs, s);
+    }
     for (int m = 0; m < t.ndims; ++m) {
         if (m == root) continue;
-        int o2[kMaxDims];
-        order_tensormode(t.ndims, t.dims, m, nat, o2);
+        int o[kMaxDims];
+        order_tensormode(t.ndims, t.dims, m, nat, o);
         if (t.ndims == 3) {
-            int o3[kMaxDims] = {o2[0], o2[2], o2[1], 0};
-            if (2 * hot[o3[2]] < hot[o2[2]]) {
-                build_tree(o3, f.tree[m]);
-            } else if (2 * hot[o2[2]] < hot[o3[2]]) {
-                build_tree(o2, f.tree[m]);
+            // fibers of the trees with x at level 1
+            const auto fibers = [&](int x) { return pairs[3 - m - x]; };
+            const int x = o[1], y = o[2];
+            bool swap;  // order m, y, x
+            if (2 * hot[x] < hot[y] || 2 * hot[y] < hot[x]) {
+                const int dense = hot[x] < hot[y] ? x : y, spread = x + y - dense;
+                const double n = (double)t.nnz;
+                const bool up = fibers(spread) >= 0.9 * n && fibers(dense) <= 0.65 * n;
+                swap = (up ? dense : spread) == y;
             } else {
-                build_tree(o2, f.tree[m]);
-                Csf alt;
-                build_tree(o3, alt);
-                if (alt.cnt[1] < f.tree[m].cnt[1]) f.tree[m] = std::move(alt);
+                swap = fibers(y) < fibers(x);
             }
-        } else {
-            build_tree(o2, f.tree[m]);
+            if (swap) std::swap(o[1], o[2]);
         }
+        build_tree(o, f.tree[m]);
         f.hasTree[m] = true;
     }
 }

@@ -10,6 +10,7 @@
 //   create_HYB / _4D, make_HybBin  852-1142, 1786-1885
 #include <cstdio>
 #include <cstdlib>
+#include <cmath>
 #include <cstring>
 #include <rocprim/rocprim.hpp>
 
@@ -1142,6 +1143,103 @@ __global__ void k_reach(const uint64_t *__restrict__ prefix, uint64_t rows, doub
     if (before < want && (i + 1 == rows || (double)prefix[i] >= want)) *out = (uint32_t)(i + 1);
 }
 
+// The distinct pairs of two modes' coordinates among the nonzeros, for the mode
+// pairs (0,1), (0,2), (1,2), estimated from the pairs whose hash starts with
+// `shift` zero bits: a pair is in the sample or not with all its nonzeros, so
+// the sample's distinct pairs times 2^shift is the estimate, and with about
+// 2^kPairBits of them it is good to a fraction of a percent.  One pass over the
+// index arrays, four nonzeros per lane and load.  Sampled pairs wait in an LDS
+// queue per wave (coordinates are below 2^31: the mode pair fits above the key)
+// and go 64 at a time into an open-addressing table of mask + 1 slots (key + 1;
+// 0 is free), at least twice the sample; a pair that finds no slot within
+// kPairProbes counts as new.  Without the queue nearly every hash of a wave
+// waited for some lane's trip to the table, past the L2: 20M nonzeros took
+// 350 us, with it 160 us (three hashes per nonzero); a tree built to be compared
+// and dropped takes 4.5 ms.
+constexpr int kPairBits = 16, kPairProbes = 64;
+constexpr int kPairQueue = 2 * 3 * 256;  // a wave's step adds 3 x 256 at most
+__global__ __launch_bounds__(kBS) void k_pair_count(const uint32_t *__restrict__ i0, const uint32_t *__restrict__ i1,
+                                                    const uint32_t *__restrict__ i2, uint64_t dim1, uint64_t dim2,
+                                                    uint64_t n, int shift, unsigned long long *table, uint32_t mask,
+                                                    uint32_t *found) {
+    __shared__ uint64_t queues[kBS / 64][kPairQueue];
+    const int lane = threadIdx.x & 63;
+    volatile uint64_t *const queue = queues[threadIdx.x / 64];
+    int held = 0;  // the same in every lane
+    uint32_t fresh[3] = {0, 0, 0};
+    auto drain = [&] {
+        __builtin_amdgcn_wave_barrier();
+        for (int e = lane; e < held; e += 64) {
+            const uint64_t key = queue[e];
+            uint64_t h = key * 0x9e3779b97f4a7c15ull;
+            h ^= h >> 32;
+            uint32_t at = (uint32_t)h & mask;
+            bool isNew = true;
+            for (int probe = 0; probe < kPairProbes; ++probe, at = (at + 1) & mask) {
+                unsigned long long have = __hip_atomic_load(table + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (have == 0) {
+                    have = atomicCAS(table + at, 0ull, (unsigned long long)key + 1);
+                    if (have == 0) break;
+                }
+                if (have == key + 1) {
+                    isNew = false;
+                    break;
+                }
+            }
+            const int pair = (int)(key >> 62);
+            fresh[0] += isNew && pair == 0;
+            fresh[1] += isNew && pair == 1;
+            fresh[2] += isNew && pair == 2;
+        }
+        __builtin_amdgcn_wave_barrier();
+        held = 0;
+    };
+    auto offer = [&](bool in, uint32_t a, uint32_t b, uint64_t width, uint64_t pair) {
+        uint32_t h = a * 0x9e3779b1u + b * 0x85ebca77u;
+        h ^= h >> 15;
+        h *= 0x2c1b3c6du;
+        h ^= h >> 13;
+        h *= 0x297a2d39u;
+        h ^= h >> 16;
+        in = in && (shift == 0 || h >> (32 - shift) == 0);
+        const uint64_t who = __ballot(in);
+        if (in) queue[held + __popcll(who & ((1ull << lane) - 1))] = (a * width + b) | pair << 62;
+        held += __popcll(who);
+    };
+    auto count = [&](bool in, uint32_t a, uint32_t b, uint32_t c) {
+        offer(in, a, b, dim1, 0);
+        offer(in, a, c, dim2, 1);
+        offer(in, b, c, dim2, 2);
+    };
+    const uint64_t t = blockIdx.x * (uint64_t)kBS + threadIdx.x, threads = (uint64_t)gridDim.x * kBS;
+    const uint64_t n4 = n / 4, steps = (n4 + threads - 1) / threads;
+    for (uint64_t k = 0; k < steps; ++k) {
+        const uint64_t i = k * threads + t;
+        const bool in = i < n4;
+        uint4 a = make_uint4(0, 0, 0, 0), b = a, c = a;
+        if (in) {
+            a = reinterpret_cast<const uint4 *>(i0)[i];
+            b = reinterpret_cast<const uint4 *>(i1)[i];
+            c = reinterpret_cast<const uint4 *>(i2)[i];
+        }
+        count(in, a.x, b.x, c.x);
+        count(in, a.y, b.y, c.y);
+        count(in, a.z, b.z, c.z);
+        count(in, a.w, b.w, c.w);
+        if (held > kPairQueue / 2) drain();
+    }
+    if (blockIdx.x == 0) {  // the last n % 4 nonzeros
+        const uint64_t i = n4 * 4 + threadIdx.x;
+        const bool in = i < n;
+        count(in, in ? i0[i] : 0, in ? i1[i] : 0, in ? i2[i] : 0);
+    }
+    drain();
+    for (int p = 0; p < 3; ++p) {
+        for (int off = 32; off; off >>= 1) fresh[p] += __shfl_down(fresh[p], off, 64);
+        if (lane == 0 && fresh[p]) atomicAdd(found + p, fresh[p]);
+    }
+}
+
 }  // namespace
 
 // Per mode m, the rows that hold `frac` of the nonzeros, most used rows first:
@@ -1179,6 +1277,32 @@ void hot_footprints(const Tensor &t, double frac, uint64_t *hot, hipStream_t s) 
     MMCSF_HIP(hipMemcpyAsync(h, found.p, sizeof(h), hipMemcpyDeviceToHost, s));
     MMCSF_HIP(hipStreamSynchronize(s));
     for (int m = 0; m < t.ndims; ++m) hot[m] = h[m];
+}
+
+// pairs[m] = the distinct coordinate pairs of the two modes other than m of a
+// 3-D tensor, which is the level-1 entries of the trees that have the one at
+// the root and the other below (an estimate past 2^kPairBits nonzeros)
+void pair_counts(const Tensor &t, double *pairs, hipStream_t s) {
+    const uint64_t n = t.nnz;
+    pairs[0] = pairs[1] = pairs[2] = 0.0;
+    if (n == 0) return;
+    int shift = 0;
+    while ((n >> shift) > (1ull << kPairBits)) ++shift;
+    uint32_t slots = 1024;
+    while (slots < 6 * (n >> shift)) slots *= 2;
+    TmpArray<unsigned long long> table(slots);
+    TmpArray<uint32_t> found(3);
+    hipLaunchKernelGGL(k_zero_words, dim3(nblk(2ull * slots)), dim3(kBS), 0, s, reinterpret_cast<uint32_t *>(table.p),
+                       2ull * slots);
+    hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(kBS), 0, s, found.p, (uint64_t)3);
+    const unsigned blocks = (unsigned)std::min<uint64_t>(3ull * device_cu_count(), (n + 4 * kBS - 1) / (4 * kBS));
+    hipLaunchKernelGGL(k_pair_count, dim3(blocks), dim3(kBS), 0, s, t.inds[0].p, t.inds[1].p, t.inds[2].p, t.dims[1],
+                       t.dims[2], n, shift, table.p, slots - 1, found.p);
+    MMCSF_HIP(hipGetLastError());
+    uint32_t h[3];
+    MMCSF_HIP(hipMemcpyAsync(h, found.p, sizeof(h), hipMemcpyDeviceToHost, s));
+    MMCSF_HIP(hipStreamSynchronize(s));
+    for (int p = 0; p < 3; ++p) pairs[2 - p] = std::ldexp((double)h[p], shift);
 }
 
 

@@ -312,6 +312,8 @@ void build_csl_walk(Hyb &h, hipStream_t s);
 void build_level_maps(Csf &c, hipStream_t s);
 // hot[m] = the rows of tensor mode m holding `frac` of the nonzeros, most used first
 void hot_footprints(const Tensor &t, double frac, uint64_t *hot, hipStream_t s);
+// pairs[m] = the distinct pairs of coordinates of the other two modes (3-D; estimated when large)
+void pair_counts(const Tensor &t, double *pairs, hipStream_t s);
 // mixed-mode partition: level-1 entry of every nonzero of an unsplit CSF (at
 // its tensor position, resolved like the reference's search over
 // denseSlcPtr; 0xFFFFFFFF where that search reads before the first entry)

@@ -29,6 +29,12 @@ def footprint(ind, rows, frac=0.9):
     ([30_000, 9000, 500], [None, 1.2, None], 60_000),  # more rows than the counting table holds
     ([20_000, 30_000, 400], [1.2, 1.1, None], 150_000),
     ([9000, 8192, 8193], [None, None, None], 100_000),
+    # the concentrated mode above the leaf; pairs counted exactly up to 2^16
+    # nonzeros, by a sample of the pairs past it
+    ([30_000, 3000, 2000], [1.5, None, None], 65_500),
+    ([30_000, 3000, 2000], [1.5, None, None], 66_000),
+    ([30_000, 5000, 4000], [1.4, None, None], 700_001),
+    ([3000, 2000, 1000], [1.4, None, None], 700_001),
 ])
 def test_mode_tree_orders_follow_the_footprints(cuda, dims, skew, nnz):
     import mmcsf
@@ -37,19 +43,22 @@ def test_mode_tree_orders_follow_the_footprints(cuda, dims, skew, nnz):
     f = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), 12, fbr_threshold=128)
     info = f.info()
     hot = [footprint(inds[m], dims[m]) for m in range(3)]
+    n = len(vals)
     for m in (0, 1):
         a, b = sorted((x for x in range(3) if x != m), key=lambda x: dims[x])
         # the default order ends in b; the swapped one in a
-        if 2 * hot[a] < hot[b]:
-            want = [m, b, a]
-        elif 2 * hot[b] < hot[a]:
-            want = [m, a, b]
+        pairs = {x: len(np.unique(inds[m].astype(np.int64) * dims[x] + inds[x])) for x in (a, b)}
+        sampled = n > 1 << 16  # counts within 3 %: either order is right nearer to a line
+        if 2 * hot[a] < hot[b] or 2 * hot[b] < hot[a]:
+            dense, spread = (a, b) if hot[a] < hot[b] else (b, a)
+            x, y = pairs[spread] / n, pairs[dense] / n
+            if sampled and min(abs(x / 0.9 - 1), abs(y / 0.65 - 1)) < 0.03:
+                continue
+            want = [m, dense, spread] if x >= 0.9 and y <= 0.65 else [m, spread, dense]
         else:
-            # the order with fewer level-1 entries, counted with the -f 128 split
-            na, nb = ([-(-c // 128) for c in np.unique(inds[m].astype(np.int64) * dims[x] + inds[x],
-                                                       return_counts=True)[1]] for x in (a, b))
-            na, nb = sum(na), sum(nb)
-            want = [m, b, a] if nb < na else [m, a, b]
+            if sampled and abs(pairs[a] / pairs[b] - 1) < 0.03:
+                continue
+            want = [m, b, a] if pairs[b] < pairs[a] else [m, a, b]
         assert info["modeTreeOrder"][m] == want, (m, hot)
 
 
