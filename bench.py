@@ -254,8 +254,8 @@ def run_c2(args):
                           "kernel_ms_f32": f32_k, "kernel_ms_bf16": b16_k}), flush=True)
         return
 
-    # the reference's layout: one MM-CSF tree, non-root modes scatter (LDS
-    # privatisation of hot rows, atomics for the rest)
+    # the reference's layout: one MM-CSF tree, the non-root modes in the order
+    # of their level
     log("timing the single-tree path")
     fmt1 = mmcsf.Format(X, mmcsf.TYPE_MMCSF, fbr_threshold=128, mode_trees=False)
     info1 = fmt1.info()
@@ -372,7 +372,7 @@ def run_c2(args):
             },
         },
         "single_tree": {
-            "note": "the reference's MM-CSF layout (-a 0): one tree, modes other than its root scatter",
+            "note": "the reference's MM-CSF layout (-a 0): one tree, the other modes in its levels' orders",
             "kernel_ms": [round(k, 4) for k in single_k],
             "all_mode_kernel_ms": round(sum(single_k), 4),
             "gbs": round(sum(bytes_single) / (sum(single_k) * 1e-3) / 1e9, 2),

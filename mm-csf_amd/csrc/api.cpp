@@ -445,9 +445,10 @@ void build_mixed(const Tensor &t, const mmcsf_options *opt, bool nat, Format &f,
 // The fibers are counted by pair_counts before anything is sorted; with both
 // trees built and one kept, a uniform tensor of 20M nonzeros took 18.0 ms to
 // build instead of 13.9, one of 20000 1.35 ms instead of 1.15.
-// One tree and 20M nonzeros (500000 x 200000 x 50000),
-// R = 32, all modes: 2.87 ms through level maps, 0.77 ms through root trees,
-// for 0.95 GB of structure instead of 0.54 and a build of 20 ms instead of 8.
+// The one-tree types at 20M nonzeros (500000 x 200000 x 50000), R = 32, all
+// modes: 2.87 ms through level maps, 0.77 ms through root trees, for 0.95 GB of
+// structure instead of 0.54 and a build of 13 ms instead of 8; at 200000
+// nonzeros (30000 x 2000 x 1000) 50 and 21 us, builds of 1.1 and 1.9 ms.
 void build_mode_trees(const Tensor &t, const mmcsf_options *opt, bool nat, int root, bool positions, Format &f,
                       hipStream_t s) {
     const uint64_t kNoSplit = 999999999ull;
