@@ -103,8 +103,8 @@ __global__ __launch_bounds__(256) void k_gram(const float *__restrict__ U, uint3
 }
 
 __global__ void k_zero_d(double *p, uint64_t n) {
-    uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0;
+    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+        p[i] = 0.0;
 }
 
 // ---------------------------------------------------------------------------
