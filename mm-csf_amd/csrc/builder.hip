@@ -621,20 +621,21 @@ __global__ void k_word_pop(const uint32_t *__restrict__ bits, uint64_t words, ui
     if (w < words) cnt[w] = (uint32_t)(__popc(bits[2 * w]) + __popc(bits[2 * w + 1]));
 }
 
-void build_walk_ranks(Csf &c, hipStream_t s) {
+bool build_walk_ranks(Csf &c, hipStream_t s) {
     const int N = c.ndims;
     const uint64_t n = c.nnz, nL = c.cnt[N - 2];
-    if (n == 0) return;
+    if (n == 0) return true;
     Temp tmp;
     auto ranks = [&](const DevArray<uint32_t> &bits, uint64_t items, DevArray<uint32_t> &rank) {
         const uint64_t words = (items + 63) / 64;
         rank.alloc(words);
         TmpArray<uint32_t> cnt(words);
         hipLaunchKernelGGL(k_word_pop, dim3(nblk(words)), dim3(kBS), 0, s, bits.p, words, cnt.p);
-        exclusive_sum(cnt.p, rank.p, words, s, tmp);
+        return exclusive_sum(cnt.p, rank.p, words, s, tmp);
     };
-    ranks(c.fbit, n, c.frank);
-    if (N == 4) ranks(c.sbit, nL, c.jrank);
+    bool ok = ranks(c.fbit, n, c.frank) == nL;
+    if (N == 4) ok = ranks(c.sbit, nL, c.jrank) == c.cnt[1] && ok;
+    return ok;
 }
 
 // ---------------------------------------------------------------------------

@@ -205,15 +205,24 @@ void csf_fields(W &w, C &c) {
                 w.skip(n * sizeof(uint32_t));
             }
         if (cc.fbit.p && cc.nnz) {
-            // derived again; every array read for that has to be there and as
-            // long as the counts say
+            // The traversals index the arrays of a level by the ranks of the start
+            // bits, which are derived again: every array has to be there and as
+            // long as the counts say, and the bits have to start with a set one
+            // and be as many as the entries, so that no rank is past them.
             const int N = cc.ndims;
-            bool ok = N >= 3 && cc.leaf.n >= cc.nnz && cc.fbit.n >= cc.nnz / 32 + 3 && cc.cnt[N - 1] == cc.nnz;
-            for (int l = 1; ok && l < N - 1; ++l) ok = cc.idx[l].n >= cc.cnt[l] && cc.cnt[l] > 0;
-            if (ok && N == 4) ok = cc.sbit.n >= cc.cnt[2] / 32 + 3;
+            const uint64_t nL = N >= 3 ? cc.cnt[N - 2] : 0;
+            bool ok = N >= 3 && cc.leaf.n >= cc.nnz && cc.vals.n >= cc.nnz && cc.fbit.n >= cc.nnz / 32 + 3 &&
+                      cc.cnt[N - 1] == cc.nnz && cc.fbrSlc.n >= cc.cnt[1] && cc.chunkCost.n >= (cc.nnz + 63) / 64 + 1;
+            for (int l = 0; ok && l < N - 1; ++l)
+                ok = cc.idx[l].n >= cc.cnt[l] && cc.ptr[l].n >= cc.cnt[l] + 1 && cc.cnt[l] > 0;
+            if (ok && N == 4) ok = cc.sbit.n >= nL / 32 + 3;
             MMCSF_REQUIRE(ok, MMCSF_ERR_IO, "format cache: bad tree");
             w.st.drain();
-            build_walk_ranks(cc, w.st.s);
+            uint32_t first[2] = {0, 1};
+            MMCSF_HIP(hipMemcpyAsync(&first[0], cc.fbit.p, 4, hipMemcpyDeviceToHost, w.st.s));
+            if (N == 4) MMCSF_HIP(hipMemcpyAsync(&first[1], cc.sbit.p, 4, hipMemcpyDeviceToHost, w.st.s));
+            ok = build_walk_ranks(cc, w.st.s);  // (waits for the stream)
+            MMCSF_REQUIRE(ok && (first[0] & first[1] & 1u), MMCSF_ERR_IO, "format cache: bad tree");
             if (mapped) build_level_maps(cc, w.st.s);
         }
     }

@@ -57,3 +57,45 @@ def test_cpd_norms_at_wide_ranks(cuda, dims, R):
         lam, st = mmcsf.cpd_als(f, U, iters=2, tol=0.0, no_alloc=no_alloc)
         np.testing.assert_allclose(st["fit_history"], fits, atol=1e-4, rtol=0)
         assert np.isfinite(lam).all() and all(bool(torch.isfinite(u).all()) for u in U)
+
+
+# ---- format caches whose start bits contradict their counts ---------------------------
+
+def start_words(starts, items):
+    """The start bits of a level as the cache stores them: a word count, then the
+    words."""
+    w = np.zeros(items // 32 + 3, dtype=np.uint32)
+    np.bitwise_or.at(w, starts // 32, np.uint32(1) << (starts % 32).astype(np.uint32))
+    return w
+
+
+@pytest.mark.parametrize("dims", [[60, 50, 40], [20, 18, 15, 12]])
+@pytest.mark.parametrize("fmt_type,kw", [(8, {}), (10, {}), (14, {"mode_trees": False}), (12, {})])
+def test_cache_with_wrong_start_bits_is_refused(cuda, tmp_path, dims, fmt_type, kw):
+    """A start bit too many, one too few, or the first one elsewhere: a nonzero's
+    fiber would be looked for past the arrays."""
+    import mmcsf
+    rng = np.random.default_rng(len(dims))
+    inds, vals = random_tensor(rng, dims, 3000, [1.3] + [None] * (len(dims) - 1))
+    f = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), fmt_type, fbr_threshold=8, **kw)
+    path = tmp_path / "a.fmt"
+    f.save(path)
+    data = path.read_bytes()
+    N = len(dims)
+    levels = [N - 2] if N == 3 else [1, 2]  # bits over fibers, bits over nonzeros
+    for l in levels:
+        starts = f.export("fbrPtr", l)[:-1].astype(np.int64)
+        items = int(f.export("fbrPtr", l)[-1])
+        words = start_words(starts, items)
+        blob = np.uint64(len(words)).tobytes() + words.tobytes()
+        at = data.find(blob)
+        assert at > 0, "the start bits are in the file"
+        free = np.setdiff1d(np.arange(items), starts)
+        more, fewer, late = (np.append(starts, free[-1]), starts[:-1], np.append(starts[1:], free[0]))
+        for bad in (more, fewer, late):
+            b = start_words(bad, items)
+            path.write_bytes(data[:at + 8] + b.tobytes() + data[at + len(blob):])
+            with pytest.raises(mmcsf.MMCSFError, match="bad tree"):
+                mmcsf.Format.load(path)
+    path.write_bytes(data)
+    assert mmcsf.Format.load(path).info() == f.info()
