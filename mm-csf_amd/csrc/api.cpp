@@ -1153,6 +1153,30 @@ int mmcsf_mttkrp(const mmcsf_format *fh, int mode, int R, int dtype, const void 
     });
 }
 
+namespace {
+// whether the byte ranges [a, a + an) and [b, b + bn) share memory
+bool overlap(const void *a, uint64_t an, const void *b, uint64_t bn) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return a && b && an && bn && x < y + bn && y < x + an;
+}
+
+// Whether the outputs of several modes may be cleared and written together: no
+// two share memory, and none shares it with a factor (which the modes after it
+// would read).  Otherwise the modes follow one another.
+bool outputs_apart(const Format &f, int R, int dtype, const void *const *factors, float *const *outs) {
+    const uint64_t es = dtype == MMCSF_F32 ? 4 : 2;
+    for (int m = 0; m < f.ndims; ++m) {
+        const uint64_t n = f.dims[m] * (uint64_t)R;
+        for (int q = 0; q < f.ndims; ++q) {
+            const uint64_t k = f.dims[q] * (uint64_t)R;
+            if (q < m && overlap(outs[m], 4 * n, outs[q], 4 * k)) return false;
+            if (overlap(outs[m], 4 * n, factors[q], es * k)) return false;
+        }
+    }
+    return true;
+}
+}  // namespace
+
 int mmcsf_mttkrp_allmode(const mmcsf_format *fh, int R, int dtype, const void *const *factors, float *const *outs,
                          void *stream, float *ms_per_mode) {
     return guarded([&] {
@@ -1178,8 +1202,8 @@ int mmcsf_mttkrp_allmode(const mmcsf_format *fh, int R, int dtype, const void *c
         for (int m = 0; m < f.ndims; ++m) F.U[m] = factors[m];
         F.dtype = dtype;
         F.R = R;
-        // every output cleared by one launch, and (untimed, every mode with a
-        // root tree) every mode walked by one where the walks are short
+        // outputs apart: every output cleared by one launch, and (untimed, every
+        // mode with a root tree) every mode walked by one where the walks are short
         uint64_t count[kMaxDims];
         const Csf *trees[kMaxDims];
         bool roots = !ms_per_mode && !f.mixed;
@@ -1190,11 +1214,12 @@ int mmcsf_mttkrp_allmode(const mmcsf_format *fh, int R, int dtype, const void *c
             roots = roots && trees[m]->order[0] == m;
         }
         MMCSF_REQUIRE(R >= 1 && R <= 256, MMCSF_ERR_UNSUPPORTED, "R must be in 1..256");
-        fill_zero_all(outs, count, f.ndims, s);
-        if (!roots || !mttkrp_roots(trees, f.ndims, F, outs, s))
+        const bool apart = outputs_apart(f, R, dtype, factors, outs);
+        if (apart) fill_zero_all(outs, count, f.ndims, s);
+        if (!apart || !roots || !mttkrp_roots(trees, f.ndims, F, outs, s))
             for (int m = 0; m < f.ndims; ++m)
                 mttkrp_mode(f, m, F, outs[m], s, ms_per_mode ? ev[2 * m] : nullptr,
-                            ms_per_mode ? ev[2 * m + 1] : nullptr, true);
+                            ms_per_mode ? ev[2 * m + 1] : nullptr, apart);
         if (ms_per_mode) {
             MMCSF_HIP(hipEventSynchronize(ev[2 * f.ndims - 1]));
             for (int m = 0; m < f.ndims; ++m)
@@ -1413,7 +1438,8 @@ int mmcsf_cp_loss_grad(const mmcsf_format *fh, int R, int dtype, const void *con
                       "CP completion needs a B-CSF or MM-CSF format");
         MMCSF_REQUIRE(f.csf.pos.p || f.nnz == 0, MMCSF_ERR_ARG, "format holds no nonzero positions");
         hipStream_t s = static_cast<hipStream_t>(stream);
-        // the gradients and the loss (two floats wide) cleared by one launch
+        // the gradients, where they are apart, and the loss (two floats wide)
+        // cleared by one launch
         const Csf *trees[kMaxDims];
         float *out[kMaxDims + 1];
         uint64_t count[kMaxDims + 1];
@@ -1426,9 +1452,12 @@ int mmcsf_cp_loss_grad(const mmcsf_format *fh, int R, int dtype, const void *con
         }
         out[walks] = reinterpret_cast<float *>(loss);
         count[walks] = 2;
-        fill_zero_all(out, count, walks + 1, s);
-        for (int i = 0; i < walks; ++i)
+        const bool apart = outputs_apart(f, R, dtype, factors, grads);
+        fill_zero_all(apart ? out : out + walks, apart ? count : count + walks, apart ? walks + 1 : 1, s);
+        for (int i = 0; i < walks; ++i) {
+            if (!apart) fill_zero(out[i], count[i], s);
             cp_gradient(*trees[i], F, nullptr, alpha, out[i], i == 0 ? loss : nullptr, s);
+        }
         if (walks) cp_half(loss, s);
         else cp_forward(f.csf, F, nullptr, loss, s);
     });

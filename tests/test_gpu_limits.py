@@ -99,3 +99,57 @@ def test_cache_with_wrong_start_bits_is_refused(cuda, tmp_path, dims, fmt_type, 
                 mmcsf.Format.load(path)
     path.write_bytes(data)
     assert mmcsf.Format.load(path).info() == f.info()
+
+
+# ---- outputs that share memory, tensors without nonzeros ---------------------------------
+
+FORMATS = [(12, {}), (12, {"mode_trees": False}), (12, {"mixed": True}), (14, {}), (14, {"mode_trees": False})]
+
+
+@pytest.mark.parametrize("dims,nnz", [([300, 200, 100], 5000), ([40, 30, 25, 20], 5000)])
+@pytest.mark.parametrize("fmt_type,kw", FORMATS)
+def test_allmode_outputs_in_one_buffer(cuda, dims, nnz, fmt_type, kw):
+    """The modes follow one another: one buffer given for every mode holds the
+    last one's rows, and an output in a factor's place is read by the modes
+    after it."""
+    import torch
+    import mmcsf
+    import oracle as O
+    rng = np.random.default_rng(nnz)
+    inds, vals = random_tensor(rng, dims, nnz)
+    f = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), fmt_type, fbr_threshold=64, **kw)
+    N, R = len(dims), 32
+    U = [rng.random((d, R)).astype(np.float32) for d in dims]
+    Ud = [torch.from_numpy(u).to(cuda) for u in U]
+    for timed in (False, True):
+        buf = torch.full((max(dims) * R,), 9.0, device=cuda)
+        outs = [buf[:d * R].view(d, R) for d in dims]
+        mmcsf.mttkrp_allmode(f, Ud, outs=outs, timed=timed)
+        assert rel(outs[-1].cpu().numpy(), O.mttkrp_coo_f64(inds, vals, N - 1, U)) < 1e-5
+        # the output of a mode in place of its factor
+        V = [u.clone() for u in Ud]
+        mmcsf.mttkrp_allmode(f, V, outs=V, timed=timed)
+        W = [u.astype(np.float64) for u in U]
+        for m in range(N):
+            W[m] = O.mttkrp_coo_f64(inds, vals, m, [w.astype(np.float32) for w in W])
+            assert rel(V[m].cpu().numpy(), W[m]) < 1e-5, m
+
+
+def test_loss_grad_gradients_in_one_buffer(cuda):
+    import torch
+    import mmcsf
+    from oracle import dense as D
+    rng = np.random.default_rng(4)
+    dims, R = [300, 200, 100], 16
+    inds, vals = random_tensor(rng, dims, 5000)
+    f = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), 12, fbr_threshold=64)
+    U = [(rng.random((d, R)) - 0.5).astype(np.float32) for d in dims]
+    Ud = [torch.from_numpy(u).to(cuda) for u in U]
+    buf = torch.full((max(dims) * R,), 9.0, device=cuda)
+    loss = torch.full((), 7.0, dtype=torch.float64, device=cuda)
+    ptrs = (C.c_void_p * 3)(*[buf.data_ptr()] * 3)
+    mmcsf._check(mmcsf.lib().mmcsf_cp_loss_grad(f._h, R, mmcsf.F32, mmcsf._factor_ptrs(Ud), 1.0, ptrs,
+                                                C.c_void_p(loss.data_ptr()), mmcsf._stream_ptr()))
+    got = buf[:dims[2] * R].view(dims[2], R).cpu().numpy()
+    assert rel(got, D.cp_grad(inds, vals, [u.astype(np.float64) for u in U])[2]) < 1e-5
+    assert abs(float(loss) / D.cp_loss(inds, vals, [u.astype(np.float64) for u in U])[0] - 1) < 1e-5
