@@ -1213,7 +1213,7 @@ int mmcsf_mttkrp_allmode(const mmcsf_format *fh, int R, int dtype, const void *c
             trees[m] = f.hasTree[m] ? &f.tree[m] : &f.csf;
             roots = roots && trees[m]->order[0] == m;
         }
-        MMCSF_REQUIRE(R >= 1 && R <= 256, MMCSF_ERR_UNSUPPORTED, "R must be in 1..256");
+        MMCSF_REQUIRE(R >= 1 && (R <= 256 || f.nnz == 0), MMCSF_ERR_UNSUPPORTED, "R must be in 1..256");
         const bool apart = outputs_apart(f, R, dtype, factors, outs);
         if (apart) fill_zero_all(outs, count, f.ndims, s);
         if (!apart || !roots || !mttkrp_roots(trees, f.ndims, F, outs, s))

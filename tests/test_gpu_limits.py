@@ -153,3 +153,19 @@ def test_loss_grad_gradients_in_one_buffer(cuda):
     got = buf[:dims[2] * R].view(dims[2], R).cpu().numpy()
     assert rel(got, D.cp_grad(inds, vals, [u.astype(np.float64) for u in U])[2]) < 1e-5
     assert abs(float(loss) / D.cp_loss(inds, vals, [u.astype(np.float64) for u in U])[0] - 1) < 1e-5
+
+
+@pytest.mark.parametrize("R", [1, 64, 256, 300])
+@pytest.mark.parametrize("fmt_type,kw", [(12, {}), (12, {"mode_trees": False}), (14, {})])
+def test_allmode_without_nonzeros(cuda, fmt_type, kw, R):
+    """Zeros at every rank, as from the call for one mode."""
+    import torch
+    import mmcsf
+    dims = [30, 20, 10]
+    t = mmcsf.Tensor.from_numpy(dims, [np.zeros(0, dtype=np.int64)] * 3, np.zeros(0, dtype=np.float32))
+    f = mmcsf.Format(t, fmt_type, **kw)
+    U = [torch.ones((d, R), device=cuda) for d in dims]
+    outs = [torch.full((d, R), 9.0, device=cuda) for d in dims]
+    mmcsf.mttkrp_allmode(f, U, outs=outs)
+    assert all(int(o.count_nonzero()) == 0 for o in outs)
+    assert int(mmcsf.mttkrp(f, 0, U).count_nonzero()) == 0
