@@ -74,10 +74,10 @@ typedef struct mmcsf_options {
     uint64_t fbrThreashold;   /* -f fiber split threshold (99999999) */
     int factorDtype;          /* -d 0|1: FP32 / BF16 factor storage (new flag) */
     uint64_t seed;            /* -x seed of generated inputs (new flag, 1) */
-    int modeTrees;            /* -a 1|0 (new flag, 1): MM-CSF and the one-tree types 9 / 13 /
-                                 14 also keep a root tree per other mode, so every mode's
-                                 MTTKRP is a root traversal; 0 = the reference's single tree,
-                                 the other modes through its level maps */
+    int modeTrees;            /* -a 1|0 (new flag, 1): MM-CSF also keeps a root tree per
+                                 other mode, so every mode's MTTKRP is a root traversal;
+                                 0 = the reference's single tree, the other modes through its
+                                 level maps (as in the one-tree types 9 / 13 / 14 always) */
     int mixedPart;            /* -M 1|0 (new flag, 0): MM-CSF partitions the nonzeros by the
                                  reference's heuristic (mm_partition_reuseBased,
                                  util.h:2386-2512, threshold -h) instead of its override
@@ -278,9 +278,8 @@ int mmcsf_format_to_tensor(const mmcsf_format *f, mmcsf_tensor **out);
  *                                    (mttkrp_gpu.h:75-81, mttkrp_gpu.cu:3380, 3860)
  * COO, B-CSF and HB-CSF serve their root mode (modeOrder[0]) only, like
  * the reference; MM-CSF and the one-tree types 9 / 13 / 14 serve every mode
- * (types 9 / 13 / 14: the root mode walks the tree, the other modes a root tree
- * of their own or, -a 0, the one tree in the order of their level,
- * mttkrp_gpu.cu:2131-2528, 2853-3378, and for type 13 the
+ * (types 9 / 13 / 14: the root mode walks the tree, the other modes the same
+ * tree in the order of their level, mttkrp_gpu.cu:2131-2528, 2853-3378, and for type 13 the
  * host routines MTTKRP_HCSR_CPU[_4D] / _mode1 / _mode2, mttkrp_cpu.cpp:160-348,
  * whose 3-D-only mode1 / mode2 roles this generalises to 4-D: every mode of a
  * 4-D type-13 format is its exact MTTKRP).

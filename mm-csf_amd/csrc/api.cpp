@@ -445,18 +445,13 @@ void build_mixed(const Tensor &t, const mmcsf_options *opt, bool nat, Format &f,
 // The fibers are counted by pair_counts before anything is sorted; with both
 // trees built and one kept, a uniform tensor of 20M nonzeros took 18.0 ms to
 // build instead of 13.9, one of 20000 1.35 ms instead of 1.15.
-// The one-tree types at 20M nonzeros (500000 x 200000 x 50000), R = 32, all
-// modes: 2.87 ms through level maps, 0.77 ms through root trees, for 0.95 GB of
-// structure instead of 0.54 and a build of 13 ms instead of 8; at 200000
-// nonzeros (30000 x 2000 x 1000) 50 and 21 us, builds of 1.1 and 1.9 ms.
-void build_mode_trees(const Tensor &t, const mmcsf_options *opt, bool nat, int root, bool positions, Format &f,
-                      hipStream_t s) {
+void build_mode_trees(const Tensor &t, const mmcsf_options *opt, bool nat, int root, Format &f, hipStream_t s) {
     const uint64_t kNoSplit = 999999999ull;
     auto build_tree = [&](const int *o, Csf &c) {
         DevArray<uint32_t> k[kMaxDims];
         DevArray<float> v;
         DevArray<uint32_t> p;
-        sort_coo(t, o, k, v, s, positions ? &p : nullptr);
+        sort_coo(t, o, k, v, s, &p);
         build_csf(t.ndims, t.dims, t.nnz, o, k, std::move(v), opt->fbrThreashold, kNoSplit, c, s);
         c.pos = std::move(p);
     };
@@ -864,7 +859,7 @@ int mmcsf_format_build(const mmcsf_tensor *th, int type, const mmcsf_options *op
             uint64_t fs = t.ndims == 4 ? 128 : kNoSplit;  // util.h:1325-1326
             build_csf(t.ndims, t.dims, t.nnz, order, keys, std::move(vals), opt->fbrThreashold, fs, f.csf, s);
             f.csf.pos = std::move(pos);
-            if (opt->modeTrees) build_mode_trees(t, opt, nat, order[0], true, f, s);
+            if (opt->modeTrees) build_mode_trees(t, opt, nat, order[0], f, s);
             else build_level_maps(f.csf, s);  // the other modes, from the one tree
         } else {
             order_tensormode(t.ndims, t.dims, (int)opt->mode, nat, order);
@@ -882,14 +877,13 @@ int mmcsf_format_build(const mmcsf_tensor *th, int type, const mmcsf_options *op
                     f.csf.pos = std::move(pos);
                     // type 13 is create_HCSR alone (mttkrp.cu:244-247): no slice bins
                     if (type != MMCSF_TYPE_SINGLECSF) build_bins_tiled(f.csf, s);
-                    // one-tree types: the reference's arrays are the one tree's; the
-                    // other modes walk root trees of their own beside it, as in
-                    // MM-CSF (positions serve the CP passes, which take the root
-                    // mode only here), or, -a 0, level maps of the one tree
-                    if (one_tree_type(type)) {
-                        if (opt->modeTrees) build_mode_trees(t, opt, nat, order[0], false, f, s);
-                        else build_level_maps(f.csf, s);
-                    }
+                    // one-tree types hold their structure once: the other modes through
+                    // level maps of the one tree, whatever modeTrees says.  Root trees
+                    // beside it would take 0.77 ms instead of 2.87 (all modes, R = 32,
+                    // 20M nonzeros, 500000 x 200000 x 50000) for 0.95 GB instead of
+                    // 0.54, and a build of 10.7 ms instead of 5.9 (5M nonzeros): MM-CSF
+                    // is the type that makes that choice.
+                    if (one_tree_type(type)) build_level_maps(f.csf, s);
                 } else {
                     build_hyb(t.ndims, t.dims, std::move(f.csf), f.hyb, s);
                     build_csl_walk(f.hyb, s);

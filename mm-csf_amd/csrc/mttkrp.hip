@@ -567,7 +567,8 @@ void mttkrp_mode(const Format &f, int mode, const Factors &F, float *out, hipStr
     }
     if (f.hasTree[mode]) {
         // MM-CSF refuses bfloat16 rows at 8-byte boundaries where 16 are needed;
-        // the one-tree types take them in every mode but their root
+        // the one-tree types (whose caches may hold root trees, though none is
+        // built) take them in every mode but their root
         mttkrp_csf(f.tree[mode], f.dims, 0, F, out, s, evStart, evEnd, false, zeroed, f.type != MMCSF_TYPE_MMCSF);
         return;
     }

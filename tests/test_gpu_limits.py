@@ -169,3 +169,26 @@ def test_allmode_without_nonzeros(cuda, fmt_type, kw, R):
     mmcsf.mttkrp_allmode(f, U, outs=outs)
     assert all(int(o.count_nonzero()) == 0 for o in outs)
     assert int(mmcsf.mttkrp(f, 0, U).count_nonzero()) == 0
+
+
+# ---- the one-tree types hold one tree ---------------------------------------------------
+
+@pytest.mark.parametrize("dims", [[300, 200, 100], [60, 40, 30, 20]])
+@pytest.mark.parametrize("fmt_type", [9, 13, 14])
+def test_one_tree_types_hold_one_tree(cuda, tmp_path, fmt_type, dims):
+    """Whatever modeTrees says: no tree beside the one, which every mode reads, and
+    no more memory than the tree (at most 16 bytes a nonzero per index level, 12 for
+    its leaf) with 4 bytes a nonzero and level for the orders of the modes."""
+    import mmcsf
+    rng = np.random.default_rng(fmt_type)
+    inds, vals = random_tensor(rng, dims, 8000)
+    t = mmcsf.Tensor.from_numpy(dims, inds, vals)
+    a, b = (mmcsf.Format(t, fmt_type, fbr_threshold=64, mode_trees=mt) for mt in (True, False))
+    info, N, n = a.info(), len(dims), len(vals)
+    assert info == b.info()
+    assert info["modeTrees"] == 0
+    assert all(info["modeTreeOrder"][m] == info["modeOrder"] for m in range(N))
+    assert info["deviceBytes"] <= n * (16 * (N - 1) + 12 + 4 * (N - 1)) + 4096
+    a.save(tmp_path / "a.fmt")
+    b.save(tmp_path / "b.fmt")
+    assert (tmp_path / "a.fmt").read_bytes() == (tmp_path / "b.fmt").read_bytes()
