@@ -648,9 +648,13 @@ void mttkrp_hyb(const Hyb &h, const uint64_t *dims, const Factors &F, float *out
             else run_geo<CooSel<4>::template K, CooArgs, uint16_t>(g, a, groups, s);
         }
     }
-    // The walked parts, which share no slice, in one launch where the walks are
-    // short (3.3M nonzeros, R = 10: 49 -> 47 us the call).
-    if (h.cslWalk.nnz && h.csf.nnz) {
+    // The walked parts, which share no slice, in one launch where both walks are
+    // short.  The launch shares its blocks by nonzeros, and the CSL part's cost
+    // several times the CSF part's (a level-1 row each): once the walks are more
+    // than their latencies, one part's blocks wait for the other's.  In turn /
+    // together, R = 32: 200000 nonzeros (20000 x 10000 x 3000) 31 / 26 us, 1M
+    // (50000 x 30000 x 9973) 51 / 56, 5M 103 / 149, 20M 283 / 439.
+    if (h.cslWalk.nnz && h.csf.nnz && h.cslWalk.nnz + h.csf.nnz <= 1ull << 18) {
         const Csf *trees[2] = {&h.csf, &h.cslWalk};
         float *const outs[2] = {out, out};
         if (mttkrp_roots(trees, 2, F, outs, s)) return;

@@ -192,3 +192,25 @@ def test_one_tree_types_hold_one_tree(cuda, tmp_path, fmt_type, dims):
     a.save(tmp_path / "a.fmt")
     b.save(tmp_path / "b.fmt")
     assert (tmp_path / "a.fmt").read_bytes() == (tmp_path / "b.fmt").read_bytes()
+
+
+# ---- dispatch lines of walks -----------------------------------------------------------
+
+@pytest.mark.parametrize("nnz", [1000, 200_000, 262_144, 330_000])
+@pytest.mark.parametrize("R", [5, 32, 64])
+def test_hbcsf_parts_together_and_in_turn(cuda, nnz, R):
+    """The walked parts of HB-CSF on both sides of 2^18 nonzeros; with and without
+    one of the parts."""
+    import torch
+    import mmcsf
+    import oracle as O
+    rng = np.random.default_rng(nnz + R)
+    for dims, skew in (([30_000, 9000, 400], [1.3, None, None]),    # every part
+                       ([20, 10, 5000], [None] * 3),                # long fibers only
+                       ([nnz // 4 + 1, 90_000, 80_000], [None] * 3)):  # single-nonzero fibers
+        inds, vals = random_tensor(rng, dims, nnz, skew)
+        f = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), 10, mode=0, fbr_threshold=1 << 30)
+        U = [rng.random((d, R)).astype(np.float32) for d in dims]
+        out = torch.full((dims[0], R), 9.0, device=cuda)
+        mmcsf.mttkrp(f, 0, [torch.from_numpy(u).to(cuda) for u in U], out=out)
+        assert rel(out.cpu().numpy(), O.mttkrp_coo_f64(inds, vals, 0, U)) < 1e-5, dims
