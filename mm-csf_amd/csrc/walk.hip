@@ -39,28 +39,41 @@ WalkArgs args_of(const Csf &c, const Factors &F) {
     return a;
 }
 
-// Columns that one MTTKRP pass takes.  A pass holds a group's rows, partial sums
-// and loads in flight in registers.  Past two column blocks (64 float32
+// Columns that one float32 MTTKRP pass takes.  A pass holds a group's rows,
+// partial sums and loads in flight in registers.  Past two column blocks (64
 // columns) it runs at two waves per SIMD, and past four (128) it spills: passes
-// over 64 columns, which read the tree again, take over.  All modes, one pass /
-// passes of 64, float32: 30M nonzeros, 3-D (500000 x 200000 x 50000) R = 96
-// 4.06 / 3.22 ms, 128 4.62 / 4.26, 160 9.4 / 5.4, 256 11.7 / 8.6; 2M nonzeros
-// (3000 x 2000 x 1000) R = 96 246 / 243 us, 128 251 / 294, 160 499 / 378, 256
-// 595 / 567.  So from 97 to 128 columns it is one pass, but for 3-D tables past
-// the L2s (4 MB per XCD), which passes bring closer to fitting.  A 4-D walk
-// does not factor at two column blocks and waits on such tables' lines most:
-// there passes of 32 columns win from R = 64 on (30M nonzeros, tables of 43 MB:
-// 4.70 / 4.57 ms, R = 128 9.9 / 9.0).  Bfloat16 rows are half as wide and stay
-// in one pass (R = 128: 2.38 / 2.45 ms, 2M nonzeros R = 256 284 / 410 us).
+// over 64 columns, which read the tree again, take over where nothing speaks
+// against them:
+//   - Rows that are no multiple of 128 bytes are read line by line in one pass,
+//     but a line that two passes share is read by both.  That shows where the
+//     lines come from past the L2s: uniform 3-D tables, 4M nonzeros, R = 72,
+//     passes / one pass 0.75-0.84 at 1 MB of tables, 0.88-0.96 at 4 MB, 0.9-1.05
+//     at 9, 1.06-1.15 at 18, 1.15-1.22 at 35 (R = 144: 0.72-0.84 at 18 MB,
+//     1.13-1.17 at 30M nonzeros and 230 MB).  Tables past 8 MB therefore need
+//     whole lines, R % 32 == 0 (30M nonzeros, 410 MB: R = 96 0.94-0.98, 160 0.90-0.96).
+//   - Each pass is a launch and its latencies.  At R = 72 and 96 the passes gain
+//     from about 1.5M nonzeros on (3-D, one mode: 200000 nonzeros 1.16 times the
+//     time, 800000 1.07-1.13, 1.6M 0.99-1.03, 2M 0.93-1.02); up to R = 160, where
+//     one pass spills, they cost nothing at 200000 (0.92-1.01), at 192 1.09-1.13.
+//   - From 97 to 128 columns one pass has no half-used block to lose: two take
+//     0.84-1.17 of its time near, 0.95-1.24 far.
+//   - Past 192 columns, over near tables, four passes take 0.75 to 1.23 of one's
+//     time from mode to mode; far ones of whole lines 0.70-1.01.
+// 32-column passes of 4-D walks at R = 64 gain where modes are uniform (0.72-1.02)
+// and lose where all but one are skewed (1.04-1.16): one pass.  Bfloat16 rows
+// are half as wide and stay in one pass (R = 128: 2.38 / 2.45 ms, 2M nonzeros
+// R = 256 284 / 410 us).
 int pass_columns(int N, const WalkArgs &a, const Factors &F) {
     const int R = F.R;
-    if (F.dtype != MMCSF_F32) return R;
+    if (F.dtype != MMCSF_F32 || R <= 64) return R;
     uint64_t bytes = 0;
     for (int l = 1; l < N; ++l) bytes += a.tabBytes[l];
-    const bool far = bytes >= (24ull << 20);
-    if (N == 4 && far && R > 32 && R % 32 == 0) return 32;
-    if (R > 128 || (R > 64 && R <= 96) || (R > 96 && far && N == 3)) return 64;
-    return R;
+    const bool near = bytes < (8ull << 20), lines = R % 32 == 0;
+    const bool many = a.nnz >= 3u << 19;
+    if (R <= 96) return many && (near || lines) ? 64 : R;
+    if (R <= 128) return R;
+    if (R <= 192) return (near || lines) && (many || R <= 160) ? 64 : R;
+    return many && !near && lines ? 64 : R;
 }
 
 // the pass that starts at column `at`: `width` columns, fewer at the end, but

@@ -1037,9 +1037,7 @@ void dispatch(const Cfg &c, int R, F f) {
         MMCSF_WALK(8, 1, 8)
         MMCSF_WALK(8, 2, 4)
         MMCSF_WALK(8, 4, 2)
-        if constexpr (!(OP == kMttkrp && std::is_same_v<T, float>)) {  // (its passes end at 128 columns)
-            MMCSF_WALK(8, 8, 1)
-        }
+        MMCSF_WALK(8, 8, 1)
     } else {
         MMCSF_WALK(8, 1, 4)
         MMCSF_WALK(8, 2, 2)

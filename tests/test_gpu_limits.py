@@ -214,3 +214,28 @@ def test_hbcsf_parts_together_and_in_turn(cuda, nnz, R):
         out = torch.full((dims[0], R), 9.0, device=cuda)
         mmcsf.mttkrp(f, 0, [torch.from_numpy(u).to(cuda) for u in U], out=out)
         assert rel(out.cpu().numpy(), O.mttkrp_coo_f64(inds, vals, 0, U)) < 1e-5, dims
+
+
+@pytest.mark.parametrize("nnz", [1_000_000, 1_650_000])
+@pytest.mark.parametrize("dims", [[3000, 2000, 1000], [40_000, 30_000, 9000], [400, 300, 200, 100]])
+def test_column_passes_on_both_sides_of_their_lines(cuda, dims, nnz):
+    """Walks shorter and longer than the 1.5M nonzeros, tables smaller and larger than
+    the 8 MB, from which on a wide rank goes in passes: every column as at R = 32,
+    within 1e-6 (two float32 orders of the same sums)."""
+    import torch
+    import mmcsf
+    rng = np.random.default_rng(nnz + len(dims))
+    inds, vals = random_tensor(rng, dims, nnz)
+    t = mmcsf.Tensor.from_numpy(dims, inds, vals)
+    forms = [mmcsf.Format(t, 12, fbr_threshold=128), mmcsf.Format(t, 14, fbr_threshold=128), mmcsf.Format(t, 3)]
+    full = [torch.rand((d, 256), generator=torch.Generator(device=cuda).manual_seed(d), device=cuda) for d in dims]
+    want = []
+    for m in range(len(dims)):
+        parts = [mmcsf.mttkrp(forms[0], m, [u[:, c:c + 32].contiguous() for u in full]) for c in range(0, 256, 32)]
+        want.append(torch.cat(parts, 1).double())
+    for R in (65, 72, 96, 100, 128, 130, 160, 161, 192, 200, 224, 255, 256):
+        U = [u[:, :R].contiguous() for u in full]
+        for f in forms:
+            for m in range(len(dims) if f.type != 3 else 1):
+                d = mmcsf.mttkrp(f, m, U).double() - want[m][:, :R]
+                assert float(d.norm() / want[m][:, :R].norm()) < 1e-6, (f.type, R, m)
