@@ -14,6 +14,7 @@ WalkArgs args_of(const Csf &c, const Factors &F) {
     const int N = c.ndims;
     WalkArgs a{};
     for (int l = 0; l < N - 1; ++l) {
+        a.ptr[l] = c.ptr[l].p;
         a.idx[l] = c.idx[l].p;
         a.cnt[l] = (uint32_t)c.cnt[l];
     }

@@ -44,6 +44,7 @@ namespace mmcsf {
 
 struct WalkArgs {
     const uint32_t *idx[3];
+    const uint32_t *ptr[3];
     const uint32_t *slc;   // slice coordinate of each level-1 entry
     const uint32_t *leaf;
     const float *val;

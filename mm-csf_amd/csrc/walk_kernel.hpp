@@ -36,12 +36,29 @@ __device__ __forceinline__ uint32_t wave_lower(const uint32_t *__restrict__ a, u
     return lo;
 }
 
+// Largest i < n with a[i] <= key (a non-decreasing, a[0] <= key), the same way.
+__device__ __forceinline__ uint32_t wave_upper(const uint32_t *__restrict__ a, uint32_t n, uint32_t key) {
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t lo = 0, hi = n;
+    while (hi - lo > 1) {
+        const uint32_t step = (hi - lo + 63) / 64;
+        const uint32_t probe = lo + lane * step;
+        const bool le = lane == 0 || (probe < hi && a[probe] <= key);
+        const uint64_t m = __ballot(le);
+        const uint32_t last = 63u - (uint32_t)__builtin_clzll(m);
+        lo += last * step;
+        hi = std::min(hi, lo + step);
+    }
+    return lo;
+}
+
 // Chunks [cb, ce) of wave wv of `waves`: an equal share of the total traversal
-// cost, or one chunk where there is a wave for each (the search is two
+// cost, or one chunk where there is a wave for each (SHORT; the search is two
 // dependent reads or more, of the ~8 that such a short run waits for).
+template <bool SHORT = true>
 __device__ __forceinline__ void wave_run(const uint32_t *__restrict__ cost, uint32_t chunks, uint64_t wv,
                                          uint64_t waves, uint32_t &cb, uint32_t &ce) {
-    if (chunks <= waves) {
+    if (SHORT && chunks <= waves) {
         cb = (uint32_t)std::min<uint64_t>(wv, chunks);
         ce = std::min(cb + 1, chunks);
     } else {
@@ -214,10 +231,39 @@ constexpr bool kFactorOf = OP == kMttkrp && NB <= 2 && G >= 2 && !(N == 4 && G =
 // cost 5 % on 4-D trees and 6 % on the CP passes.
 constexpr int kWalkWaves = 4;
 
+template <int N, int G, int NB, int VEC, int OP>
+constexpr int kMinWaves = (OP == kMttkrp && N == 3 && NB == 1 && G * VEC <= 32) ? 3 : 2;
+
+// Operations whose runs start from a search over the tree's pointers, by a wave
+// index in a vector register, instead of from the ranks of the start bits in
+// scalar registers.  The ranks are fewer reads, and MTTKRP gains up to 29
+// registers by the scalars, but the loops of these passes come out slower with
+// them (same registers and waves per SIMD): residuals at R = 12 to 32, 4M
+// nonzeros in short rows (300 x 200 x 1000), 92-95 us by vector, 99-102 by
+// scalar; loss and gradient at R = 64 float32, 20M nonzeros (1000000 x 500000 x
+// 100000, Zipf(1.1) x Zipf(1.1) x uniform), mode 0 1180 us by search, 1225 by
+// rank.  Passes of more registers lose a wave per SIMD the other way (R = 128
+// bfloat16 3.25 -> 3.98 ms), narrower gradients 2 %.
+template <int NB, int VEC, int OP>
+constexpr bool kSearchOf = (OP == kLossResid && NB * VEC <= 8) || (OP == kLossGrad && NB == 2 && VEC == 4);
+
+// the walk of this block: the launch's only one, or that of its row of the grid
+__device__ __forceinline__ const WalkArgs &walk_of(const WalkArgs &p) { return p; }
+__device__ __forceinline__ const WalkArgs &walk_of(const WalkSet &p) { return p.walk[blockIdx.y]; }
+__device__ __forceinline__ uint32_t blocks_of(const WalkArgs &) { return gridDim.x; }
+__device__ __forceinline__ uint32_t blocks_of(const WalkSet &p) { return p.blocks[blockIdx.y]; }
+
 // RAG: ranks that VEC does not divide (float32 MTTKRP; its own instances, since
-// the column arithmetic costs the widest cases a wave per SIMD)
-template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG, int SRC>
-__device__ __forceinline__ void walk(const WalkArgs &a, const uint32_t gridBlocks) {
+// the column arithmetic costs the widest cases a wave per SIMD).
+// P: WalkArgs for one walk, WalkSet for several in one launch.
+// (The body stays in the kernel: inlined from a function of its own, mode 0 of
+// the R = 64 gradient above takes 1226 us instead of 1180.)
+template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG, int SRC, typename P>
+__global__ __launch_bounds__(64 * kWalkWaves, (kMinWaves<N, G, NB, VEC, OP>)) void k_walk(P p) {
+    const uint32_t gridBlocks = blocks_of(p);
+    if constexpr (std::is_same_v<P, WalkSet>)
+        if (blockIdx.x >= gridBlocks) return;
+    const WalkArgs &a = walk_of(p);
     static_assert(G == 1 || G == 2 || G == 4 || G == 8, "row groups of 1..8 lanes");
     static_assert(G % TB == 0, "steps per batch divide the steps of a chunk");
     static_assert(VEC % 4 == 0, "rows are written as float4");
@@ -231,6 +277,7 @@ __device__ __forceinline__ void walk(const WalkArgs &a, const uint32_t gridBlock
     constexpr bool kByFiber = OP == kTtm || OP == kTtmStream;
     constexpr bool kUpper = !kByFiber;
     constexpr bool kFactor = kFactorOf<N, G, NB, OP>;
+    constexpr bool kSearch = kSearchOf<NB, VEC, OP>;
     static_assert(!(kFactor && (OP == kLossGrad || OP == kLossResid)), "the CP passes multiply per nonzero");
     // residuals / weights are addressed by tensor-order position
     constexpr bool kPos = OP == kLossResid || OP == kWeightGrad;
@@ -255,12 +302,12 @@ __device__ __forceinline__ void walk(const WalkArgs &a, const uint32_t gridBlock
                                   (blockIdx.x >> 3) % spanBlocks;
     // (the wave's index in a scalar register: so are its run and the tree
     // positions at its start)
-    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t w = kSearch ? threadIdx.x >> 6 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint64_t wv = (uint64_t)lb * wavesPerBlock + w;
     const uint32_t chunks = (uint32_t)(((uint64_t)a.nnz + 63) / 64);
     uint32_t cb, ce;
-    wave_run(a.cost, chunks, wv, waves, cb, ce);
-    const int R = a.cols;  // columns of this pass; rows are a.R wide
+    wave_run<!kSearch>(a.cost, chunks, wv, waves, cb, ce);
+    const int R = kCp ? a.R : a.cols;  // columns of this pass; rows are a.R wide
     const uint32_t rowBytes = (uint32_t)a.R * (uint32_t)sizeof(T);
     // First of this lane's columns in block b.  RAG: the row's last lane has
     // fewer than VEC columns of its own; it takes the last VEC columns of the
@@ -338,8 +385,10 @@ __device__ __forceinline__ void walk(const WalkArgs &a, const uint32_t gridBlock
     [[maybe_unused]] __shared__ uint32_t tailRow[kWalkWaves];
     if (cb >= ce) {
         // no run: nothing to join (each wave passes one barrier, here or at the
-        // end; a condition around the whole run costs 6 registers more, and
-        // the widest case then a wave per SIMD)
+        // end: s_barrier counts the waves that arrive, wherever they stand, and
+        // every wave of the block arrives exactly once; a condition around the
+        // whole run costs 6 registers more, and the widest case then a wave per
+        // SIMD)
         if constexpr (kGrad) {
             if (lane == 0) tailRow[w] = kNone;
             __syncthreads();
@@ -348,7 +397,18 @@ __device__ __forceinline__ void walk(const WalkArgs &a, const uint32_t gridBlock
     }
     const uint32_t x0 = (uint32_t)(cb * 64);
     [[maybe_unused]] uint32_t fcur = kNone, jcur = kNone;
-    if constexpr (SRC == kTree) {
+    if constexpr (kSearch) {
+        // leaf fiber (and 4-D level-1 entry) of the nonzero before the run; the
+        // unsigned wrap at x0 = 0 stands for -1
+        const uint32_t f0 = wave_upper(a.ptr[LF], a.cnt[LF], x0);  // leaf fiber of x0
+        fcur = x0 == 0 ? kNone : (a.ptr[LF][f0] == x0 ? f0 - 1 : f0);
+        uint32_t j0 = f0;
+        if constexpr (N == 4) {
+            j0 = wave_upper(a.ptr[1], a.cnt[1], f0);
+            jcur = fcur == kNone ? kNone : (a.ptr[1][j0] == f0 && fcur != f0 ? j0 - 1 : j0);
+        }
+        scur = a.slc[j0];
+    } else if constexpr (SRC == kTree) {
         // leaf fiber (and 4-D level-1 entry) of the nonzero before the run, by
         // the ranks of the start bits; the unsigned wrap at x0 = 0 stands for -1
         fcur = a.frank[cb] - 1u;
@@ -928,21 +988,6 @@ __device__ __forceinline__ void walk(const WalkArgs &a, const uint32_t gridBlock
     }
 }
 
-template <int N, int G, int NB, int VEC, int OP>
-constexpr int kMinWaves = (OP == kMttkrp && N == 3 && NB == 1 && G * VEC <= 32) ? 3 : 2;
-
-template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG, int SRC>
-__global__ __launch_bounds__(64 * kWalkWaves, (kMinWaves<N, G, NB, VEC, OP>)) void k_walk(WalkArgs a) {
-    walk<N, G, NB, TB, T, VEC, OP, RAG, SRC>(a, gridDim.x);
-}
-
-// The walks of several trees in one launch, a row of the grid each.
-template <int N, int G, int NB, int TB, typename T, int VEC, int OP, bool RAG, int SRC>
-__global__ __launch_bounds__(64 * kWalkWaves, (kMinWaves<N, G, NB, VEC, OP>)) void k_walk_set(WalkSet set) {
-    if (blockIdx.x < set.blocks[blockIdx.y])
-        walk<N, G, NB, TB, T, VEC, OP, RAG, SRC>(set.walk[blockIdx.y], set.blocks[blockIdx.y]);
-}
-
 struct Cfg {
     int G, NB, TB, VEC;
 };
@@ -977,7 +1022,7 @@ struct Walk {
     // waves than chunks would give empty waves only.  The waves of a small
     // tensor are spread over the CUs.
     static void launch(const WalkArgs &a, hipStream_t s) {
-        auto fn = k_walk<N, G, NB, TB, T, VEC, OP, RAG, SRC>;
+        auto fn = k_walk<N, G, NB, TB, T, VEC, OP, RAG, SRC, WalkArgs>;
         const uint64_t cus = (uint64_t)device_cu_count();
         const uint64_t chunks = ((uint64_t)a.nnz + 63) / 64;
         const uint64_t block = std::min<uint64_t>(kWalkWaves, (chunks + cus - 1) / cus);
@@ -997,7 +1042,7 @@ struct Walk {
     // The line is drawn at the chunks per resident wave of ~8M nonzeros.
     static constexpr uint64_t kSetChunks = 96;
     static bool launch_set(WalkSet &set, int walks, bool always, hipStream_t s) {
-        auto fn = k_walk_set<N, G, NB, TB, T, VEC, OP, RAG, SRC>;
+        auto fn = k_walk<N, G, NB, TB, T, VEC, OP, RAG, SRC, WalkSet>;
         const uint64_t cus = (uint64_t)device_cu_count();
         uint64_t chunks = 0, most = 0;
         for (int i = 0; i < walks; ++i) chunks += ((uint64_t)set.walk[i].nnz + 63) / 64;
@@ -1068,7 +1113,7 @@ void dispatch_all(int ndims, const Factors &fac, int cols, F f) {
 template <int OP, int SRC>
 void walk_preload() {
     hipFuncAttributes attr;
-    MMCSF_HIP(hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(k_walk<3, 8, 1, 8, float, 4, OP, false, SRC>)));
+    MMCSF_HIP(hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(k_walk<3, 8, 1, 8, float, 4, OP, false, SRC, WalkArgs>)));
 }
 
 template <int OP, int SRC>

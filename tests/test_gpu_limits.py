@@ -239,3 +239,30 @@ def test_column_passes_on_both_sides_of_their_lines(cuda, dims, nnz):
             for m in range(len(dims) if f.type != 3 else 1):
                 d = mmcsf.mttkrp(f, m, U).double() - want[m][:, :R]
                 assert float(d.norm() / want[m][:, :R].norm()) < 1e-6, (f.type, R, m)
+
+
+@pytest.mark.parametrize("dims,skew,nnz", [([5, 4, 3], None, 1), ([300, 200, 100], None, 64), ([300, 200, 100], None, 65),
+                                           ([40, 9, 5000], None, 30_000), ([6000, 500, 400], [1.3, None, None], 300_000),
+                                           ([30, 25, 20, 15], None, 4097), ([600, 90, 80, 70], [1.2, None, None, 1.2], 250_000)])
+def test_completion_run_starts(cuda, dims, skew, nnz):
+    """Loss, residuals and gradients at ranks on both sides of the forms of a run's
+    start, over one run, a chunk per wave and more, long and short fibers."""
+    import torch
+    import mmcsf
+    from oracle import dense as D
+    rng = np.random.default_rng(nnz)
+    inds, vals = random_tensor(rng, dims, nnz, skew)
+    f = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), 12, fbr_threshold=128)
+    for R, dt in ((4, "f32"), (12, "f32"), (32, "f32"), (48, "f32"), (64, "f32"), (96, "f32"), (32, "bf16"), (64, "bf16")):
+        Ud = [torch.from_numpy(((rng.random((d, R)) - 0.4) * 0.5).astype(np.float32)).to(cuda) for d in dims]
+        if dt == "bf16":
+            Ud = [u.to(torch.bfloat16) for u in Ud]
+        U = [u.float().cpu().numpy().astype(np.float64) for u in Ud]
+        loss64, e64 = D.cp_loss(inds, vals, U)
+        loss, res = mmcsf.cp_forward(f, Ud, residual=True)
+        assert abs(float(loss) / loss64 - 1) < 1e-5, (R, dt)
+        assert rel(-res.cpu().numpy(), e64) < 1e-5, (R, dt)  # (the oracle's residual is value - model)
+        loss, grads = mmcsf.cp_loss_grad(f, Ud)
+        assert abs(float(loss) / loss64 - 1) < 1e-5, (R, dt)
+        for m, want in enumerate(D.cp_grad(inds, vals, U)):
+            assert rel(grads[m].cpu().numpy(), want) < 1e-5, (R, dt, m)
