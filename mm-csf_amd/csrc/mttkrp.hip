@@ -84,17 +84,24 @@ __global__ __launch_bounds__(kBlock) void k_csf(CsfArgs a) {
         slc = ns;
     };
     for (uint32_t xb = x0; xb < x1; xb += B) {
+        // every index of the batch before the first row: a row's load waits for its
+        // index, and one wait then serves the batch
+        uint32_t li[B];
         float vv[B];
         RowT rows[B];
 #pragma unroll
         for (int k = 0; k < B; ++k) {
             const uint32_t x = xb + k;
+            li[k] = 0;
             vv[k] = 0.f;
             if (x < x1) {
+                li[k] = a.leaf[x];
                 vv[k] = a.val[x];
-                rows[k].load(UL, a.leaf[x], R, lane);
             }
         }
+#pragma unroll
+        for (int k = 0; k < B; ++k)
+            if (xb + k < x1) rows[k].load(UL, li[k], R, lane);
 #pragma unroll
         for (int k = 0; k < B; ++k) {
             const uint32_t x = xb + k;
