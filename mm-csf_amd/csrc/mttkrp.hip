@@ -130,8 +130,8 @@ __global__ __launch_bounds__(kBlock) void k_csf(CsfArgs a) {
 }
 
 // --------------------------------------------------------------------------
-// Level-map MTTKRP for what the mapped walk does not serve (R < 4, tables of
-// 4 GiB and more, bfloat16 rows at 8-byte boundaries): every group sums a
+// Level-map MTTKRP for what the mapped walk does not serve (R > 3: tables of 4 GiB
+// and more, bfloat16 rows at 8-byte boundaries): every group sums a
 // contiguous run of the nonzeros in the order of the output level.
 // --------------------------------------------------------------------------
 struct MapArgs {
@@ -182,6 +182,141 @@ __global__ __launch_bounds__(kBlock) void k_map(MapArgs a) {
         acc.fma(a.val[x], p);
     }
     acc.atomic_add(a.out, cur, a.R, lane);
+}
+
+// --------------------------------------------------------------------------
+// Modes below the root at R <= 3, which no walk serves, in stored order: every
+// nonzero's row is added to its output row, a lane per nonzero.  Neighbours with
+// one output row (the nonzeros of a fiber) are summed by shuffles first; rows that
+// come early in a block (the hot ones do) are held in LDS, in float64, in sets of
+// four by their low bits, and added to memory once; the others pass through a
+// stage of the wave, from which consecutive lanes add to consecutive columns of a
+// row.  (With one place by the low bits, a hot row that finds it taken collects
+// every nonzero of the block as a float32 addition: relative error 8e-6 instead
+// of 1.6e-7.)  Bound by the structure's reads and the latency of the rows.  R = 1,
+// group kernel over level maps / here: the two modes below the root of
+// 300 x 200 x 1000, 4M nonzeros, 772 and 624 / 28 and 31 us; every mode of
+// 20000 x 5000 x 800 x 300, 4M, 3.52 / 0.58 ms.
+// (At R = 4 to 16 it would take 0.25 to 0.9 of the mapped walk's time where modes
+// are skewed, but a hot row's total then collects a float32 addition from every
+// block: relative error 3.4e-7 where the walk's is 1.2e-7.)
+// --------------------------------------------------------------------------
+struct ScatterArgs {
+    const uint32_t *fbit, *frank, *sbit, *jrank;
+    const uint32_t *slc, *idx1, *idx2, *leaf;
+    const float *val;
+    const float *U[4];  // per level; U[outLevel] is not read
+    float *out;
+    uint32_t nnz;
+    int outLevel;
+};
+
+constexpr int kScatterBlock = 1024;
+
+template <int N, int R>
+__global__ __launch_bounds__(kScatterBlock) void k_scatter(ScatterArgs a) {
+    constexpr int kStage = 16, kStride = R | 1;
+    constexpr uint32_t kSlots = R == 1 ? 4096 : 2048, kNone = 0xffffffffu;  // coordinates are below 2^31
+    __shared__ __align__(16) uint32_t held[kSlots];
+    __shared__ double acc[R][kSlots];
+    __shared__ volatile float stage[kScatterBlock / 64][kStage * kStride];
+    __shared__ volatile uint32_t stageRow[kScatterBlock / 64][kStage];
+    for (uint32_t i = threadIdx.x; i < kSlots; i += blockDim.x) {
+        held[i] = kNone;
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[r][i] = 0.0;
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint64_t chunks = ((uint64_t)a.nnz + 63) / 64, waves = (uint64_t)gridDim.x * (blockDim.x >> 6);
+    const uint64_t wv = blockIdx.x * (uint64_t)(blockDim.x >> 6) + w;
+    const uint32_t cb = (uint32_t)(wv * chunks / waves), ce = (uint32_t)((wv + 1) * chunks / waves);
+    for (uint32_t c = cb; c < ce; ++c) {
+        const bool in = (uint64_t)c * 64 + lane < a.nnz;
+        const uint32_t x = in ? c * 64u + (uint32_t)lane : a.nnz - 1u;
+        const uint32_t f = dev::rank_of(a.fbit, a.frank, x);
+        const uint32_t j = N == 4 ? dev::rank_of(a.sbit, a.jrank, f) : f;
+        const uint32_t at[4] = {a.slc[j], a.idx1[j], N == 4 ? a.idx2[f] : a.leaf[x], N == 4 ? a.leaf[x] : 0u};
+        uint32_t row = 0;
+#pragma unroll
+        for (int l = 0; l < N; ++l)
+            if (l == a.outLevel) row = at[l];
+        float p[R];
+        const float v = a.val[x];
+#pragma unroll
+        for (int r = 0; r < R; ++r) p[r] = v;
+#pragma unroll
+        for (int l = 0; l < N; ++l)
+            if (l != a.outLevel) {
+                const float *u = a.U[l] + (size_t)at[l] * R;
+#pragma unroll
+                for (int r = 0; r < R; ++r) p[r] *= u[r];
+            }
+        // (lanes past the tensor hold its last row: nothing, also where a factor
+        // is not finite)
+#pragma unroll
+        for (int r = 0; r < R; ++r) p[r] = in ? p[r] : 0.f;
+        // neighbours with one output row: their sum to the first of them
+        const uint32_t before = __shfl_up(row, 1, 64);
+        const bool first = lane == 0 || row != before;
+        const uint64_t heads = __ballot(first);
+        if (heads != ~0ull) {
+            const int run = __popcll(heads & (~0ull >> (63 - lane)));
+            for (int off = 1; off < 64; off <<= 1) {
+                const bool same = __shfl_down(run, off, 64) == run && lane + off < 64;
+                if (__ballot(same) == 0) break;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float o = __shfl_down(p[r], off, 64);
+                    if (same) p[r] += o;
+                }
+            }
+        }
+        // the row's place among the four of its set, or a free one
+        uint32_t slot = row % (kSlots / 4) * 4;
+        bool mineHeld = false;
+        if (first && in) {
+            const uint4 q = *reinterpret_cast<const uint4 *>(held + slot);
+            const uint32_t owner[4] = {q.x, q.y, q.z, q.w};
+            int way = owner[0] == row ? 0 : owner[1] == row ? 1 : owner[2] == row ? 2 : owner[3] == row ? 3 : 4;
+            for (int t = 0; way == 4 && t < 4; ++t) {
+                if (owner[t] != kNone) continue;
+                const uint32_t was = atomicCAS(&held[slot + t], kNone, row);
+                if (was == kNone || was == row) way = t;
+            }
+            mineHeld = way < 4;
+            slot += (uint32_t)way & 3u;
+        }
+        if (mineHeld) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) unsafeAtomicAdd(&acc[r][slot], (double)p[r]);
+        }
+        // the other rows through the wave's stage, so that one request adds to all
+        // columns of a row
+        uint64_t cold = __ballot(first && in && !mineHeld);
+        while (cold) {
+            const int mine = __popcll(cold & ((1ull << lane) - 1)), n = min(__popcll(cold), kStage);
+            const bool put = ((cold >> lane) & 1) && mine < kStage;
+            __builtin_amdgcn_wave_barrier();
+            if (put) {
+                stageRow[w][mine] = row;
+#pragma unroll
+                for (int r = 0; r < R; ++r) stage[w][mine * kStride + r] = p[r];
+            }
+            __builtin_amdgcn_wave_barrier();
+            for (int i = lane; i < n * R; i += 64)
+                unsafeAtomicAdd(a.out + (size_t)stageRow[w][i / R] * R + i % R, (float)stage[w][i / R * kStride + i % R]);
+            __builtin_amdgcn_wave_barrier();
+            cold &= ~__ballot(put);
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < kSlots; i += blockDim.x) {
+        const uint32_t row = held[i];
+        if (row == kNone) continue;
+#pragma unroll
+        for (int r = 0; r < R; ++r) unsafeAtomicAdd(a.out + (size_t)row * R + r, (float)acc[r][i]);
+    }
 }
 
 // --------------------------------------------------------------------------
@@ -435,6 +570,26 @@ void launch_map_t(const Geo &g, MapArgs &a, int dtype, hipStream_t s) {
         run_geo<MapLaunch<N>::template K, MapArgs, uint16_t>(g, a, groups, s);
 }
 
+template <int N, int R>
+void launch_scatter(const ScatterArgs &a, hipStream_t s) {
+    auto fn = k_scatter<N, R>;
+    int perCU = 0;
+    MMCSF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, fn, kScatterBlock, 0));
+    // every wave a chunk at least
+    const uint64_t chunks = ((uint64_t)a.nnz + 63) / 64;
+    const uint64_t blocks = std::min<uint64_t>((uint64_t)device_cu_count() * std::max(perCU, 1),
+                                               (chunks + kScatterBlock / 64 - 1) / (kScatterBlock / 64));
+    fn<<<dim3((unsigned)blocks), dim3(kScatterBlock), 0, s>>>(a);
+    MMCSF_HIP(hipGetLastError());
+}
+
+template <int N>
+void run_scatter(const ScatterArgs &a, int R, hipStream_t s) {
+    if (R == 1) launch_scatter<N, 1>(a, s);
+    else if (R == 2) launch_scatter<N, 2>(a, s);
+    else launch_scatter<N, 3>(a, s);
+}
+
 void check_align(const void *p, int dtype, const Geo &g) {
     size_t need = g.VEC == 4 ? (dtype == MMCSF_F32 ? 16 : 8) : (dtype == MMCSF_F32 ? 4 : 2);
     if (reinterpret_cast<uintptr_t>(p) % need)
@@ -523,6 +678,26 @@ void mttkrp_csf(const Csf &c, const uint64_t *dims, int outLevel, const Factors 
     if (outLevel > 0) {
         const LevelMap &map = c.map[outLevel];
         MMCSF_REQUIRE(map.ord.p != nullptr, MMCSF_ERR_ARG, "this format serves its root mode only");
+        // (every size measured, 150000 to 20M nonzeros, 1.4 to 20 times the group kernel)
+        if (F.R <= 3) {
+            ScatterArgs a{};
+            a.fbit = c.fbit.p;
+            a.frank = c.frank.p;
+            a.sbit = c.sbit.p;
+            a.jrank = c.jrank.p;
+            a.slc = c.fbrSlc.p;
+            a.idx1 = c.idx[1].p;
+            a.idx2 = c.idx[2].p;
+            a.leaf = c.leaf.p;
+            a.val = c.vals.p;
+            for (int l = 0; l < N; ++l) a.U[l] = static_cast<const float *>(F.U[c.order[l]]);
+            a.out = out;
+            a.nnz = (uint32_t)c.nnz;
+            a.outLevel = outLevel;
+            if (N == 3) run_scatter<3>(a, F.R, s);
+            else run_scatter<4>(a, F.R, s);
+            return;
+        }
         if (map_walk_supports(c, F, outLevel, out)) {
             mttkrp_map_walk(c, outLevel, F, out, s, accumulate);
             return;

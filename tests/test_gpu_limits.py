@@ -266,3 +266,29 @@ def test_completion_run_starts(cuda, dims, skew, nnz):
         assert abs(float(loss) / loss64 - 1) < 1e-5, (R, dt)
         for m, want in enumerate(D.cp_grad(inds, vals, U)):
             assert rel(grads[m].cpu().numpy(), want) < 1e-5, (R, dt, m)
+
+
+@pytest.mark.parametrize("dims,skew,nnz", [
+    ([40, 30, 20], None, 1),
+    ([300, 200, 100], None, 1023),
+    ([9000, 5000, 300], [1.3, 1.2, None], 150_001),  # rows held, rows staged, a whole level held
+    ([30, 20, 2000], None, 200_000),                 # long fibers, every row held
+    ([70_000, 60_000, 50_000], None, 90_000),        # nearly every row staged
+    ([5000, 900, 800, 60], [1.2, None, None, None], 120_000),
+])
+@pytest.mark.parametrize("kw", [{"fmt_type": 14}, {"fmt_type": 12, "mode_trees": False}, {"fmt_type": 12, "mixed": True}])
+def test_modes_below_the_root_at_ranks_1_to_3(cuda, dims, skew, nnz, kw):
+    import torch
+    import mmcsf
+    import oracle as O
+    if kw.get("mixed") and nnz < 2000:
+        pytest.skip("the mixed-mode partition refuses tensors of one slice")
+    rng = np.random.default_rng(nnz)
+    inds, vals = random_tensor(rng, dims, nnz, skew)
+    f = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, inds, vals), fbr_threshold=128, **kw)
+    for R in (1, 2, 3):
+        U = [(rng.random((d, R)) + 0.1).astype(np.float32) for d in dims]
+        outs = [torch.full((d, R), 9.0, device=cuda) for d in dims]
+        mmcsf.mttkrp_allmode(f, [torch.from_numpy(u).to(cuda) for u in U], outs=outs)
+        for m in range(len(dims)):
+            assert rel(outs[m].cpu().numpy(), O.mttkrp_coo_f64(inds, vals, m, U)) < 1e-5, (R, m)
