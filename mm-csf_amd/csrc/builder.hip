@@ -621,20 +621,26 @@ __global__ void k_word_pop(const uint32_t *__restrict__ bits, uint64_t words, ui
     if (w < words) cnt[w] = (uint32_t)(__popc(bits[2 * w]) + __popc(bits[2 * w + 1]));
 }
 
-bool build_walk_ranks(Csf &c, hipStream_t s) {
+bool build_walk_ranks(Csf &c, hipStream_t s, bool check) {
     const int N = c.ndims;
     const uint64_t n = c.nnz, nL = c.cnt[N - 2];
     if (n == 0) return true;
     Temp tmp;
-    auto ranks = [&](const DevArray<uint32_t> &bits, uint64_t items, DevArray<uint32_t> &rank) {
+    auto ranks = [&](const DevArray<uint32_t> &bits, uint64_t items, uint64_t starts, DevArray<uint32_t> &rank) {
         const uint64_t words = (items + 63) / 64;
         rank.alloc(words);
         TmpArray<uint32_t> cnt(words);
         hipLaunchKernelGGL(k_word_pop, dim3(nblk(words)), dim3(kBS), 0, s, bits.p, words, cnt.p);
-        return exclusive_sum(cnt.p, rank.p, words, s, tmp);
+        if (check) return exclusive_sum(cnt.p, rank.p, words, s, tmp) == starts;
+        size_t bytes = 0;
+        MMCSF_HIP(rocprim::exclusive_scan(nullptr, bytes, cnt.p, rank.p, 0u, (size_t)words,
+                                          rocprim::plus<uint32_t>(), s));
+        MMCSF_HIP(rocprim::exclusive_scan(tmp.get(bytes), bytes, cnt.p, rank.p, 0u, (size_t)words,
+                                          rocprim::plus<uint32_t>(), s));
+        return true;
     };
-    bool ok = ranks(c.fbit, n, c.frank) == nL;
-    if (N == 4) ok = ranks(c.sbit, nL, c.jrank) == c.cnt[1] && ok;
+    bool ok = ranks(c.fbit, n, nL, c.frank);
+    if (N == 4) ok = ranks(c.sbit, nL, c.cnt[1], c.jrank) && ok;
     return ok;
 }
 
@@ -657,7 +663,7 @@ void build_walk_bits(Csf &c, hipStream_t s) {
     };
     mark(c.fbit, n, c.ptr[N - 2].p, nL);
     if (N == 4) mark(c.sbit, nL, c.ptr[1].p, c.cnt[1]);
-    build_walk_ranks(c, s);
+    (void)build_walk_ranks(c, s);
     // cost prefix over chunks: waves split the traversal by cost, not by
     // nonzeros (chunks where many slices start take longer)
     const uint64_t chunks = (n + 63) / 64;
@@ -698,16 +704,19 @@ __global__ void k_row_cost(const uint32_t *__restrict__ key, uint64_t n, bool pl
 void build_row_cost(const uint32_t *key, uint64_t n, uint64_t rows, DevArray<uint32_t> &prefix, hipStream_t s) {
     const uint64_t chunks = (n + 63) / 64;
     prefix.alloc(chunks + 1);
-    uint64_t total = 0;
-    if (chunks) {
-        Temp tmp;
-        TmpArray<uint32_t> cost(chunks);
-        const uint32_t ws = 24;  // as for the trees
-        const bool plain = chunks * 64 + ws * std::min(n, rows) >= 0xF0000000ull;
-        hipLaunchKernelGGL(k_row_cost, dim3(nblk(n)), dim3(kBS), 0, s, key, n, plain, ws, cost.p);
-        total = exclusive_sum(cost.p, prefix.p, chunks, s, tmp);
-    }
-    hipLaunchKernelGGL(k_set, dim3(1), dim3(1), 0, s, prefix.p, chunks, (uint32_t)total);
+    Temp tmp;
+    TmpArray<uint32_t> cost(chunks + 1);
+    const uint32_t ws = 24;  // as for the trees
+    const bool plain = chunks * 64 + ws * std::min(n, rows) >= 0xF0000000ull;
+    // the entry past the chunks costs nothing: the scan over it leaves the total
+    // there, and the host need not read it
+    hipLaunchKernelGGL(k_set, dim3(1), dim3(1), 0, s, cost.p, chunks, 0u);
+    if (n) hipLaunchKernelGGL(k_row_cost, dim3(nblk(n)), dim3(kBS), 0, s, key, n, plain, ws, cost.p);
+    size_t bytes = 0;
+    MMCSF_HIP(rocprim::exclusive_scan(nullptr, bytes, cost.p, prefix.p, 0u, (size_t)(chunks + 1),
+                                      rocprim::plus<uint32_t>(), s));
+    MMCSF_HIP(rocprim::exclusive_scan(tmp.get(bytes), bytes, cost.p, prefix.p, 0u, (size_t)(chunks + 1),
+                                      rocprim::plus<uint32_t>(), s));
     MMCSF_HIP(hipGetLastError());
     MMCSF_HIP(hipStreamSynchronize(s));
 }

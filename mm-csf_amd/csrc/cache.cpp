@@ -221,7 +221,7 @@ void csf_fields(W &w, C &c) {
             uint32_t first[2] = {0, 1};
             MMCSF_HIP(hipMemcpyAsync(&first[0], cc.fbit.p, 4, hipMemcpyDeviceToHost, w.st.s));
             if (N == 4) MMCSF_HIP(hipMemcpyAsync(&first[1], cc.sbit.p, 4, hipMemcpyDeviceToHost, w.st.s));
-            ok = build_walk_ranks(cc, w.st.s);  // (waits for the stream)
+            ok = build_walk_ranks(cc, w.st.s, true);  // (waits for the stream)
             MMCSF_REQUIRE(ok && (first[0] & first[1] & 1u), MMCSF_ERR_IO, "format cache: bad tree");
             if (mapped) build_level_maps(cc, w.st.s);
         }

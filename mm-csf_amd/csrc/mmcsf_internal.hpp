@@ -288,9 +288,9 @@ void order_tensormode(int ndims, const uint64_t *dims, int mode, bool nat, int *
 // keys[l] = coordinate of order[l], and permuted values.
 // start bitmasks of a built tree (called by build_csf and build_hyb)
 void build_walk_bits(Csf &c, hipStream_t s);
-// c.frank and c.jrank from the start bitmasks; false when there are not as many
-// start bits as entries (a file's; a build's are)
-bool build_walk_ranks(Csf &c, hipStream_t s);
+// c.frank and c.jrank from the start bitmasks; check (which waits for the stream):
+// false when there are not as many start bits as entries
+bool build_walk_ranks(Csf &c, hipStream_t s, bool check = false);
 // pos (optional) receives the tensor-order position of every sorted nonzero.
 // keepKeys: the caller keeps every key array (else only the last level's, which
 // becomes a tree's leaf array; the others are temporaries).
