@@ -292,3 +292,24 @@ def test_modes_below_the_root_at_ranks_1_to_3(cuda, dims, skew, nnz, kw):
         mmcsf.mttkrp_allmode(f, [torch.from_numpy(u).to(cuda) for u in U], outs=outs)
         for m in range(len(dims)):
             assert rel(outs[m].cpu().numpy(), O.mttkrp_coo_f64(inds, vals, m, U)) < 1e-5, (R, m)
+
+
+@pytest.mark.parametrize("fibers,per_fiber", [(60_000, 20), (3, 400_000), (90_000, 15)])
+def test_ttm_few_rows_of_many_nonzeros(cuda, fibers, per_fiber):
+    """More chunks than waves and outputs on both sides of 10 MB: all rows cleared, or
+    the run ends; the output holds other numbers before the call."""
+    import torch
+    import mmcsf
+    rng = np.random.default_rng(fibers)
+    f = np.repeat(np.arange(fibers, dtype=np.int64), per_fiber)
+    leaf = np.tile(np.arange(per_fiber, dtype=np.int64), fibers)
+    dims = [(fibers - 1) // 50 + 1, 50, max(4000, per_fiber)]
+    vals = (rng.random(len(f)) + 0.25).astype(np.float32)
+    fm = mmcsf.Format(mmcsf.Tensor.from_numpy(dims, [f // 50, f % 50, leaf], vals), 8, mode=0)
+    assert fm.info()["modeOrder"] == [0, 1, 2]
+    for R in (4, 28, 40):
+        U = rng.random((dims[2], R)).astype(np.float32)
+        Y = torch.full((fibers, R), 3.0, device=cuda)
+        mmcsf.ttm(fm, torch.from_numpy(U).to(cuda), out=Y)
+        want = vals.astype(np.float64).reshape(fibers, per_fiber) @ U[:per_fiber].astype(np.float64)
+        assert rel(Y.cpu().numpy(), want) < 1e-5, R
