@@ -891,7 +891,15 @@ int mmcsf_format_build(const mmcsf_tensor *th, int type, const mmcsf_options *op
             }
         }
         // the first MTTKRP on this format runs without loading code objects
-        if (type != MMCSF_TYPE_COO_CPU) preload_kernels(type == MMCSF_TYPE_MMCSF || type == MMCSF_TYPE_BCSF);
+        if (type != MMCSF_TYPE_COO_CPU) {
+            unsigned what = type == MMCSF_TYPE_COO ? kPreCoo : kPreTree;
+            bool trees = false;
+            for (int m = 0; m < t.ndims; ++m) trees = trees || f.hasTree[m];
+            if (trees || (f.hyb.csf.nnz && f.hyb.cslWalk.nnz)) what |= kPreSet;
+            if (f.mixed || one_tree_type(type) || (type == MMCSF_TYPE_MMCSF && !trees)) what |= kPreMap;
+            if (type == MMCSF_TYPE_MMCSF || type == MMCSF_TYPE_BCSF) what |= kPreCp;
+            preload_kernels(what);
+        }
         *out = fh.release();
     });
 }

@@ -365,9 +365,16 @@ void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, h
 void check_walk_align(const Csf &c, const Factors &F, int skipLevel, const float *out);
 bool walk_aligned(const Csf &c, const Factors &F, int skipLevel, const float *out);
 void mttkrp_hyb(const Hyb &h, const uint64_t *dims, const Factors &F, float *out, hipStream_t s);
-// loads the code objects of the MTTKRP kernels (and, cp, of the CP
-// completion passes) on the current device, once per process
-void preload_kernels(bool cp);
+// The code objects of the calls that a format serves, loaded on the current
+// device (each once per process), so that the first call does not wait for them
+enum Preload : unsigned {
+    kPreTree = 1,  // the root walk
+    kPreSet = 2,   // several root walks in one launch
+    kPreCoo = 4,   // the COO walk
+    kPreMap = 8,   // the walk over a level map
+    kPreCp = 16,   // the CP completion passes
+};
+void preload_kernels(unsigned what);
 void preload_group_kernels();
 void fill_zero(float *p, uint64_t n, hipStream_t s);
 // up to kMaxDims + 1 arrays in one launch

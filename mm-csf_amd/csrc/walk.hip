@@ -319,27 +319,25 @@ void ttm_fibers(const Csf &c, const Factors &F, float *Y, hipStream_t s) {
     else walk_launch<kTtm>(c.ndims, F, a, s);
 }
 
-void preload_kernels(bool cp) {
-    // once per device: the code objects of the traversals a format runs
+void preload_kernels(unsigned what) {
     static std::mutex lock;
-    static bool done[64][2];
+    static unsigned done[64];
     int dev = 0;
     MMCSF_HIP(hipGetDevice(&dev));
     if (dev < 0 || dev >= 64) return;
     std::lock_guard<std::mutex> g(lock);
-    if (!done[dev][0]) {
-        walk_preload<kMttkrp>();
-        walk_preload<kMttkrp, kCoo>();
-        walk_preload<kMttkrp, kMap>();
-        preload_group_kernels();
-        done[dev][0] = true;
-    }
-    if (cp && !done[dev][1]) {
+    const unsigned load = what & ~done[dev];
+    if (!done[dev]) preload_group_kernels();
+    if (load & kPreTree) walk_preload<kMttkrp>();
+    if (load & kPreSet) walk_preload_set<kMttkrp>();
+    if (load & kPreCoo) walk_preload<kMttkrp, kCoo>();
+    if (load & kPreMap) walk_preload<kMttkrp, kMap>();
+    if (load & kPreCp) {
         walk_preload<kLossResid>();
         walk_preload<kLossGrad>();
         walk_preload<kWeightGrad>();
-        done[dev][1] = true;
     }
+    done[dev] |= load;
 }
 
 void cp_half(double *loss, hipStream_t s) {

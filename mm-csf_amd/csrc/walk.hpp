@@ -106,5 +106,7 @@ template <int OP, int SRC = kTree>
 bool walk_launch_set(int ndims, const Factors &F, WalkSet &set, int walks, bool always, hipStream_t s);
 template <int OP, int SRC = kTree>
 void walk_preload();
+template <int OP, int SRC = kTree>
+void walk_preload_set();
 
 }  // namespace mmcsf

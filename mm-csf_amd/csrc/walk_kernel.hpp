@@ -1125,6 +1125,12 @@ void walk_preload() {
 }
 
 template <int OP, int SRC>
+void walk_preload_set() {
+    hipFuncAttributes attr;
+    MMCSF_HIP(hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(k_walk<3, 8, 1, 8, float, 4, OP, false, SRC, WalkSet>)));
+}
+
+template <int OP, int SRC>
 void walk_launch(int ndims, const Factors &F, const WalkArgs &a, hipStream_t s) {
     dispatch_all<OP, SRC>(ndims, F, a.cols, [&](auto w) { w.launch(a, s); });
 }

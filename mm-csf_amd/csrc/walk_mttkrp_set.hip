@@ -3,4 +3,5 @@
 
 namespace mmcsf {
 template bool walk_launch_set<kMttkrp>(int, const Factors &, WalkSet &, int, bool, hipStream_t);
+template void walk_preload_set<kMttkrp>();
 }  // namespace mmcsf

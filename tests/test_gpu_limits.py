@@ -313,3 +313,37 @@ def test_ttm_few_rows_of_many_nonzeros(cuda, fibers, per_fiber):
         mmcsf.ttm(fm, torch.from_numpy(U).to(cuda), out=Y)
         want = vals.astype(np.float64).reshape(fibers, per_fiber) @ U[:per_fiber].astype(np.float64)
         assert rel(Y.cpu().numpy(), want) < 1e-5, R
+
+
+# ---- the first call on a format -----------------------------------------------------------
+
+@pytest.mark.parametrize("fmt_type,kw", [(12, {}), (12, {"mode_trees": False}), (14, {}), (10, {}), (3, {})])
+def test_first_call_loads_no_code(cuda, fmt_type, kw):
+    """In a process of its own: the build has loaded the code objects of the calls that
+    the format serves, so the first one takes its launches (0.2 ms on a first use),
+    not a load (2 to 4 ms each)."""
+    import os
+    import subprocess
+    import sys
+    import mmcsf
+    code = f"""
+import sys, time
+sys.path.insert(0, {os.path.dirname(os.path.dirname(mmcsf.__file__))!r})
+import torch, mmcsf
+dims = [20000, 10000, 3000]
+X = mmcsf.Tensor.generate(dims, 100_000, [1, 0, 1], [1.1, 1.0, 1.1], 7)
+U = [torch.rand((d, 32), device="cuda") for d in dims]
+outs = [torch.empty((d, 32), device="cuda") for d in dims]
+f = mmcsf.Format(X, {fmt_type}, fbr_threshold=128, **{kw!r})
+torch.cuda.synchronize()
+t = time.perf_counter()
+if f.type in (12, 14):
+    mmcsf.mttkrp_allmode(f, U, outs=outs)
+else:
+    mmcsf.mttkrp(f, 0, U, out=outs[0])
+torch.cuda.synchronize()
+print("first call ms", (time.perf_counter() - t) * 1e3)
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr
+    assert float(r.stdout.split()[-1]) < 1.5
