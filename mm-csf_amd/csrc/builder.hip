@@ -1156,9 +1156,13 @@ __global__ void k_reach(const uint64_t *__restrict__ prefix, uint64_t rows, doub
 // The distinct pairs of two modes' coordinates among the nonzeros, for the mode
 // pairs (0,1), (0,2), (1,2), estimated from the pairs whose hash starts with
 // `shift` zero bits: a pair is in the sample or not with all its nonzeros, so
-// the sample's distinct pairs times 2^shift is the estimate, and with about
-// 2^kPairBits of them it is good to a fraction of a percent.  One pass over the
-// index arrays, four nonzeros per lane and load.  Sampled pairs wait in an LDS
+// the sample's distinct pairs times 2^shift is the estimate.  `shift` leaves
+// 2^(kPairBits - 1) to 2^kPairBits nonzeros in the sample, so its pairs are that
+// times the pairs per nonzero, and the estimate's standard deviation is one over
+// their square root: 0.5 % where nearly every nonzero is a pair of its own, 1 % at
+// 0.19 pairs per nonzero.  (The multipliers that mix the two coordinates are odd
+// and arbitrary: the fraction bits of the square roots of 2, 3, 5 and 7.)  One
+// pass over the index arrays, four nonzeros per lane and load.  Sampled pairs wait in an LDS
 // queue per wave (coordinates are below 2^31: the mode pair fits above the key)
 // and go 64 at a time into an open-addressing table of mask + 1 slots (key + 1;
 // 0 is free), at least twice the sample; a pair that finds no slot within
@@ -1205,11 +1209,11 @@ __global__ __launch_bounds__(kBS) void k_pair_count(const uint32_t *__restrict__
         held = 0;
     };
     auto offer = [&](bool in, uint32_t a, uint32_t b, uint64_t width, uint64_t pair) {
-        uint32_t h = a * 0x9e3779b1u + b * 0x85ebca77u;
+        uint32_t h = a * 0x6a09e667u + b * 0xbb67ae85u;
         h ^= h >> 15;
-        h *= 0x2c1b3c6du;
+        h *= 0x3c6ef373u;
         h ^= h >> 13;
-        h *= 0x297a2d39u;
+        h *= 0xa54ff53bu;
         h ^= h >> 16;
         in = in && (shift == 0 || h >> (32 - shift) == 0);
         const uint64_t who = __ballot(in);
@@ -1290,8 +1294,9 @@ void hot_footprints(const Tensor &t, double frac, uint64_t *hot, hipStream_t s) 
 }
 
 // pairs[m] = the distinct coordinate pairs of the two modes other than m of a
-// 3-D tensor, which is the level-1 entries of the trees that have the one at
-// the root and the other below (an estimate past 2^kPairBits nonzeros)
+// 3-D tensor (an estimate past 2^kPairBits nonzeros): the level-1 entries of the
+// trees that have the one at the root and the other below, before the -f split
+// cuts long fibers
 void pair_counts(const Tensor &t, double *pairs, hipStream_t s) {
     const uint64_t n = t.nnz;
     pairs[0] = pairs[1] = pairs[2] = 0.0;
