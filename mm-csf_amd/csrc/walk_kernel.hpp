@@ -1047,8 +1047,12 @@ struct Walk {
     // Side by side / in turn, all modes from the call on: 1M nonzeros 41 / 56 us
     // (3-D, R = 32), 67 / 104 (4-D, R = 32), 6M 176 / 192 and 377 / 398, 10M
     // 350 / 361 and 274 / 276 (3-D, R = 16); at 20M 541 / 516 (3-D, R = 16).
-    // The line is drawn at the chunks per resident wave of ~8M nonzeros.
-    static constexpr uint64_t kSetChunks = 96;
+    // The line is drawn at the chunks per resident wave of ~8M nonzeros.  Past two
+    // column blocks a wave holds its rows for longer and two of them share a SIMD,
+    // and modes of unequal cost wait for one another early: in turn / side by side
+    // at R = 100 (100000 x 50000 x 5000, skewed) 1.26 at 200000 nonzeros, 1.01 at
+    // 500000, 0.98 at 1M, 0.90 at 4M.
+    static constexpr uint64_t kSetChunks = NB <= 2 ? 96 : 8;
     static bool launch_set(WalkSet &set, int walks, bool always, hipStream_t s) {
         auto fn = k_walk<N, G, NB, TB, T, VEC, OP, RAG, SRC, WalkSet>;
         const uint64_t cus = (uint64_t)device_cu_count();
