@@ -153,13 +153,26 @@ bool walk_aligned(const Csf &c, const Factors &F, int skipLevel, const float *ou
     return reinterpret_cast<uintptr_t>(out) % (F.R % 4 != 0 ? 4 : 16) == 0;
 }
 
-// Ranks: every multiple of four, and any float32 rank from 4 on.  Below 4 the
-// row is narrower than one lane's load and the per-group kernel serves it.  At
-// R = 10 (HB-CSF, 3.3M nonzeros, 123457 x 70001 x 9973) the per-group kernel,
-// one column a lane in groups of 64, takes 324 us; the whole call 334 -> 53 us.
-bool walk_supports(const Csf &c, int R, int dtype) {
+// What a walk can run: every multiple of four, and any float32 rank from 4 on.
+static bool walk_fits(const Csf &c, int R, int dtype) {
     return R >= 4 && R <= 256 && (R % 4 == 0 || dtype == MMCSF_F32) && tables_fit(c, R) &&
            (c.nnz == 0 || (c.fbit.p && c.frank.p && c.chunkCost.p && (c.ndims == 3 || (c.sbit.p && c.jrank.p))));
+}
+
+// Short tensors at wide ranks that four does not divide: the walk takes them in
+// one spilling pass or a launch per pass, the per-group kernels, one column a
+// lane, in one launch.  Group kernel / walk, root mode: 50000 nonzeros R = 129 18 /
+// 24 us, COO 15 / 23; 200000 R = 255 41 / 50, COO 35 / 54; 700000 R = 161 90 / 70
+// (3-D, tables of 4 MB), 85 / 98 (4-D), 193 / 219 (COO, 200 MB); 1.4M 163 / 116,
+// 164 / 162, 328 / 357; up to R = 127 the walk from 50000 nonzeros on (17 / 17).
+static bool group_kernel_shorter(uint64_t nnz, int R) { return R > 128 && R % 4 != 0 && nnz < 1u << 20; }
+
+// Below a rank of 4 the row is narrower than one lane's load and the per-group
+// kernel serves it.  At R = 10 (HB-CSF, 3.3M nonzeros, 123457 x 70001 x 9973) the
+// per-group kernel, one column a lane in groups of 64, takes 324 us; the whole
+// call 334 -> 53 us.
+bool walk_supports(const Csf &c, int R, int dtype) {
+    return walk_fits(c, R, dtype) && !group_kernel_shorter(c.nnz, R);
 }
 
 void mttkrp_root(const Csf &c, const Factors &F, float *out, hipStream_t s, bool accumulate) {
@@ -180,7 +193,7 @@ void mttkrp_root(const Csf &c, const Factors &F, float *out, hipStream_t s, bool
 // rest.  2000 x 2000 x 2000, 1M nonzeros, R = 32: 54 -> 19 us the call.
 bool coo_walk_supports(const Format &f, const Factors &F) {
     if (F.R < 4 || F.R > 256 || (F.R % 4 != 0 && F.dtype != MMCSF_F32)) return false;
-    if (!f.cooCost.p) return false;
+    if (!f.cooCost.p || group_kernel_shorter(f.nnz, F.R)) return false;
     const uintptr_t need = F.R % 4 != 0 ? 4 : (F.dtype == MMCSF_BF16 && F.R % 8 != 0) ? 8 : 16;
     for (int l = 1; l < f.ndims; ++l) {
         if (f.dims[f.cooOrder[l]] * (uint64_t)F.R * 4u > 0xFFFFF000ull) return false;
@@ -222,7 +235,7 @@ void mttkrp_coo_walk(const Format &f, const Factors &F, float *out, hipStream_t 
 // two modes below the root: 7.19 -> 2.59 ms.  Those reads bound it: each lane's
 // is a line of its own past the L2, ~8.6 CU clocks apiece.
 bool map_walk_supports(const Csf &c, const Factors &F, int outLevel, const float *out) {
-    return walk_supports(c, F.R, F.dtype) && walk_aligned(c, F, outLevel, out);
+    return walk_fits(c, F.R, F.dtype) && walk_aligned(c, F, outLevel, out);
 }
 
 void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, hipStream_t s, bool accumulate) {
