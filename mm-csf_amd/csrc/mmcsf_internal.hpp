@@ -355,8 +355,10 @@ bool walk_supports(const Csf &c, int R, int dtype);
 void mttkrp_root(const Csf &c, const Factors &F, float *out, hipStream_t s, bool accumulate = false);
 // the root walks of several trees in one launch, into zeroed outputs (which may
 // be one output for trees without a root row in common); false (nothing
-// launched) when they are better launched one by one
-bool mttkrp_roots(const Csf *const *trees, int walks, const Factors &F, float *const *outs, hipStream_t s);
+// launched) when they are better launched one by one; unlike: their nonzeros cost
+// differently
+bool mttkrp_roots(const Csf *const *trees, int walks, const Factors &F, float *const *outs, hipStream_t s,
+                  bool unlike = false);
 // the MTTKRP of the mode at level outLevel > 0 of a tree with level maps
 bool map_walk_supports(const Csf &c, const Factors &F, int outLevel, const float *out);
 void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, hipStream_t s, bool accumulate);

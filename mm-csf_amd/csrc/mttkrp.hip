@@ -830,16 +830,20 @@ void mttkrp_hyb(const Hyb &h, const uint64_t *dims, const Factors &F, float *out
             else run_geo<CooSel<4>::template K, CooArgs, uint16_t>(g, a, groups, s);
         }
     }
-    // The walked parts, which share no slice, in one launch where both walks are
-    // short.  The launch shares its blocks by nonzeros, and the CSL part's cost
-    // several times the CSF part's (a level-1 row each): once the walks are more
-    // than their latencies, one part's blocks wait for the other's.  In turn /
-    // together, R = 32: 200000 nonzeros (20000 x 10000 x 3000) 31 / 26 us, 1M
-    // (50000 x 30000 x 9973) 51 / 56, 5M 103 / 149, 20M 283 / 439.
-    if (h.cslWalk.nnz && h.csf.nnz && h.cslWalk.nnz + h.csf.nnz <= 1ull << 18) {
+    // The walked parts, which share no slice, in one launch where the walks are
+    // short: up to 2^19 nonzeros, and up to 2^22 where the CSF part is at least half
+    // the CSL part (a sweep of random sizes and laws, R = 10 to 64, in turn / together:
+    // 1.1-1.2 below 2^21, 1.09-1.15 from there to 2^22, 1.05 past it with 0.83 at worst;
+    // larger CSL parts 1.11 below 2^19, 1.06 past it with 0.82 at worst).  A part of at
+    // most 256 nonzeros is a latency, whatever the other's size (1.03-1.2).  The parts'
+    // nonzeros cost differently; with the blocks shared by nonzeros one part's waited
+    // for the other's (5M nonzeros, R = 40: 170 us in turn, 257 together).
+    const uint64_t csf = h.csf.nnz, csl = h.cslWalk.nnz;
+    if (csf && csl &&
+        (csf + csl <= 1u << 19 || (csl <= 2 * csf && csf + csl <= 1u << 22) || std::min(csf, csl) <= 256)) {
         const Csf *trees[2] = {&h.csf, &h.cslWalk};
         float *const outs[2] = {out, out};
-        if (mttkrp_roots(trees, 2, F, outs, s)) return;
+        if (mttkrp_roots(trees, 2, F, outs, s, true)) return;
     }
     // CSL part (3-D): walked as a tree of one-nonzero fibers; the CSL kernel
     // where the walk cannot run (R < 4, tables above 4 GiB)

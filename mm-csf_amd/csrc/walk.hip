@@ -260,8 +260,14 @@ void mttkrp_map_walk(const Csf &c, int outLevel, const Factors &F, float *out, h
 // few chunks per wave is a chain of ~8 memory latencies and a launch; the modes'
 // chains then run side by side (300 x 200 x 100, 20000 nonzeros, R = 32: six
 // launches for the outputs and the walks, 34 us a call, are two, 20 us).
-bool mttkrp_roots(const Csf *const *trees, int walks, const Factors &F, float *const *outs, hipStream_t s) {
+// unlike: trees whose nonzeros cost differently (HB-CSF's parts).  The blocks are
+// then shared by the rows above the leaf that a walk reads and the slices that it
+// writes, each as 8 nonzeros, instead of by chunks (as 2 nonzeros: 2 to 5 % slower
+// over the sizes and laws that go together; as none: up to 1.7 times the time).
+bool mttkrp_roots(const Csf *const *trees, int walks, const Factors &F, float *const *outs, hipStream_t s,
+                  bool unlike) {
     WalkSet set{};
+    uint64_t weight[kMaxDims];
     for (int m = 0; m < walks; ++m) {
         const Csf &c = *trees[m];
         for (int l = 1; l < c.ndims; ++l)
@@ -269,6 +275,7 @@ bool mttkrp_roots(const Csf *const *trees, int walks, const Factors &F, float *c
         if (c.nnz == 0 || !walk_supports(c, F.R, F.dtype) || !walk_aligned(c, F, 0, outs[m])) return false;
         set.walk[m] = args_of(c, F);
         set.walk[m].out = outs[m];
+        weight[m] = unlike ? c.nnz + 8 * (c.cnt[c.ndims - 2] + c.cnt[0]) : (c.nnz + 63) / 64;
     }
     const int N = trees[0]->ndims, R = F.R;
     // passes over columns as for one walk; the first decides for all of them
@@ -277,7 +284,7 @@ bool mttkrp_roots(const Csf *const *trees, int walks, const Factors &F, float *c
         WalkSet p = set;
         const int cols = pass_width(R, at, width);
         for (int m = 0; m < walks; ++m) take_columns(N, p.walk[m], F, at, cols);
-        if (!walk_launch_set<kMttkrp>(N, F, p, walks, at > 0, s)) return false;
+        if (!walk_launch_set<kMttkrp>(N, F, p, walks, weight, at > 0, s)) return false;
         at += cols;
     }
     return true;

@@ -101,9 +101,11 @@ enum WalkOp : int {
 template <int OP, int SRC = kTree>
 void walk_launch(int ndims, const Factors &F, const WalkArgs &a, hipStream_t s);
 // several traversals alike but for their trees, in one launch; false (nothing
-// launched) when they are better launched one by one, unless `always`
+// launched) when they are better launched one by one, unless `always`; weight:
+// what the blocks are shared by
 template <int OP, int SRC = kTree>
-bool walk_launch_set(int ndims, const Factors &F, WalkSet &set, int walks, bool always, hipStream_t s);
+bool walk_launch_set(int ndims, const Factors &F, WalkSet &set, int walks, const uint64_t *weight, bool always,
+                     hipStream_t s);
 template <int OP, int SRC = kTree>
 void walk_preload();
 template <int OP, int SRC = kTree>

@@ -1053,21 +1053,33 @@ struct Walk {
     // at R = 100 (100000 x 50000 x 5000, skewed) 1.26 at 200000 nonzeros, 1.01 at
     // 500000, 0.98 at 1M, 0.90 at 4M.
     static constexpr uint64_t kSetChunks = NB <= 2 ? 96 : 8;
-    static bool launch_set(WalkSet &set, int walks, bool always, hipStream_t s) {
+    static bool launch_set(WalkSet &set, int walks, const uint64_t *weight, bool always, hipStream_t s) {
         auto fn = k_walk<N, G, NB, TB, T, VEC, OP, RAG, SRC, WalkSet>;
         const uint64_t cus = (uint64_t)device_cu_count();
-        uint64_t chunks = 0, most = 0;
-        for (int i = 0; i < walks; ++i) chunks += ((uint64_t)set.walk[i].nnz + 63) / 64;
+        uint64_t chunks = 0, most = 0, total = 0;
+        bool alike = true;
+        for (int i = 0; i < walks; ++i) {
+            chunks += ((uint64_t)set.walk[i].nnz + 63) / 64;
+            total += weight[i];
+            alike = alike && weight[i] == weight[0];
+        }
         const uint64_t resident = resident_blocks(fn);
         if (!always && chunks > kSetChunks * resident * kWalkWaves) return false;
         const uint64_t block = std::min<uint64_t>(kWalkWaves, (chunks + cus - 1) / cus);
         for (int i = 0; i < walks; ++i) {
             const uint64_t c = ((uint64_t)set.walk[i].nnz + 63) / 64;
-            // the resident blocks, shared by chunks
-            const uint64_t b = std::min<uint64_t>(std::max<uint64_t>(resident * c / chunks, 1), (c + block - 1) / block);
+            // The resident blocks, shared by weight.  Shares that differ are multiples
+            // of the XCDs (as is the width of the grid, the shorter rows' idle blocks
+            // in it): one block more than an XCD holds would start when another ends
+            // (361000 and 1085000 nonzeros, R = 32: 189 and 578 blocks of 768 resident
+            // 38.7 us, 192 and 576 29.4).
+            uint64_t share = std::max<uint64_t>(resident * weight[i] / total, 1);
+            if (!alike && share >= 8) share -= share % 8;
+            const uint64_t b = std::min<uint64_t>(share, (c + block - 1) / block);
             set.blocks[i] = (uint32_t)b;
             most = std::max(most, b);
         }
+        if (!alike) most = (most + 7) / 8 * 8;
         fn<<<dim3((unsigned)most, (unsigned)walks), dim3((unsigned)(64 * block)), 0, s>>>(set);
         MMCSF_HIP(hipGetLastError());
         return true;
@@ -1140,9 +1152,10 @@ void walk_launch(int ndims, const Factors &F, const WalkArgs &a, hipStream_t s) 
 }
 
 template <int OP, int SRC>
-bool walk_launch_set(int ndims, const Factors &F, WalkSet &set, int walks, bool always, hipStream_t s) {
+bool walk_launch_set(int ndims, const Factors &F, WalkSet &set, int walks, const uint64_t *weight, bool always,
+                     hipStream_t s) {
     bool done = false;
-    dispatch_all<OP, SRC>(ndims, F, set.walk[0].cols, [&](auto w) { done = w.launch_set(set, walks, always, s); });
+    dispatch_all<OP, SRC>(ndims, F, set.walk[0].cols, [&](auto w) { done = w.launch_set(set, walks, weight, always, s); });
     return done;
 }
 

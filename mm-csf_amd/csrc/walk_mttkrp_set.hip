@@ -2,6 +2,6 @@
 #include "walk_kernel.hpp"
 
 namespace mmcsf {
-template bool walk_launch_set<kMttkrp>(int, const Factors &, WalkSet &, int, bool, hipStream_t);
+template bool walk_launch_set<kMttkrp>(int, const Factors &, WalkSet &, int, const uint64_t *, bool, hipStream_t);
 template void walk_preload_set<kMttkrp>();
 }  // namespace mmcsf
